@@ -260,12 +260,16 @@ int reels_hip_i8lora_bwd_gelu_f16(const void* dy, const void* x, const void* h, 
  * fp32 compute, the reference's Float32 path with int8 frozen weights (_dequantize_for_compute
  * with T = Float32, src/layers/quantization.jl:61-64, and lora_forward / lora_backward in
  * Float32, src/layers/lora.jl:56-118). Every operand, intermediate and result is f32:
- *   W = fl32(q[n][k] * s[n])                   materialised in the workspace once per call
+ *   W = q[n][k] * s[n]
  *   h = x * A                                  [M][r]
  *   y = (x W^T + bias) + lora_scale * (h B)    (the reference's order: mixed_add, then adapter)
  *   u = dy B^T;  dx = dy W + lora_scale * u A^T;  dA = lora_scale x^T u;  dB = lora_scale h^T dy
  * with the layouts of the bf16 entry points (x [M][K], A [K][r], B [r][N], y [M][N], dA [K][r],
- * dB [r][N]). The sums run in f32 on fp32 MFMA. workspace: reels_hip_i8lora_workspace_bytes_f32.
+ * dB [r][N]). The weight products take the f32 activations apart into three bf16 values that sum
+ * to them exactly and multiply the exact codes on bf16 MFMA with f32 sums; s multiplies as a power
+ * of two inside and its mantissa on the f32 sum (forward) or on dy (dX). Their error against 64
+ * bits is below that of a chain of f32 multiply-adds. The rank-r products run on fp32 MFMA.
+ * workspace: reels_hip_i8lora_workspace_bytes_f32.
  */
 size_t reels_hip_i8lora_workspace_bytes_f32(int64_t M, int64_t K, int64_t N, int64_t r,
                                             int which);

@@ -29,6 +29,14 @@ struct GemmArgs {
   // bfgemm only, without a split reduction: gout [M][Ncols] = gelu_tanh(out) from the rounded
   // 16-bit outputs (the same bits as gelu_kernel on out), written beside out when != nullptr
   uint16_t* gout;
+  // launch_planegemm only: f32 operands (act is [M][3 Kred] bf16 planes, colscale as above)
+  const float* fL;     // [M][fr] or nullptr
+  const float* fR;     // [Ncols][fr]
+  const float* fbias;  // [Ncols] or nullptr
+  float* fout;         // [M][Ncols]
+  int fr;              // rank (any)
+  bool fvout;          // Ncols is a multiple of 4
+  int64_t ldp;         // row stride of part (ksplit > 1)
 };
 
 // mode 0 = FWD (out = s * act q^T + c L R^T + bias), 1 = DX (out = act q + c L R^T, or
@@ -50,6 +58,13 @@ int launch_bfgemm(int mode, int elt, const GemmArgs& a, const uint16_t* wd, hipS
 bool bfgemm_fuses_gelu(const GemmArgs& a);
 // a.gout (the forward GELU epilogue) needs the same: a.ksplit <= 1 and 16-byte aligned buffers
 bool bfgemm_fuses_gelu_fwd(const GemmArgs& a);
+
+// f32 GEMM on bf16 MFMA: fout = (act wd^T colscale + fbias) + c fL fR^T, where act holds three bf16
+// planes per row that sum to the f32 activations exactly ([M][low | middle | high], Kred columns
+// each) and wd [Ncols][Kred] values exact in bf16. Kred % 64 == 0, planes and weight below 2^31
+// bytes. ksplit (planegemm_splits) workgroups per tile through part [ksplit][M][ldp]
+int planegemm_splits(int64_t M, int64_t Ncols, int64_t Kred);
+int launch_planegemm(int mode, const GemmArgs& a, const uint16_t* wd, hipStream_t st);
 
 // wd[n][k] = deq(q[n][k], s[n]) in element type elt (bf16: bf16(fl32(q s)); f16: f16(q f16(s))),
 // q [N][K] row stride ldq (K % 16 == 0)
@@ -99,6 +114,11 @@ int launch_skinny(int mode, int elt, const SkinnyPlan& p, const uint16_t* act, c
 // out = c * sum over splits of part[sp][o][j] (split order): out[o][j], or out[j][o] with trans
 int launch_reduce_partials(const float* part, int splits, int64_t Od, int rp, int r, float c,
                            float* out, bool trans, hipStream_t st);
+// the same for dA (outA[o][j]) and dB (outB[j][o]) in one launch, and (bpart set) the bias
+// gradient bout[o] = sum over dB's splits of bpart[sp][o]
+int launch_reduce_partials2(const float* partA, int splitsA, int64_t OdA, float* outA,
+                            const float* partB, int splitsB, int64_t OdB, float* outB, int rp,
+                            int r, float c, const float* bpart, float* bout, hipStream_t st);
 
 // out[o] = sum_m src[m][o] in f32 (src [M][Od] of element type elt: REELS_HIP_F32, _BF16 or
 // _F16): the bias gradient. Split-M partials in part (colsum_partial_bytes(M, Od) bytes), summed

@@ -592,10 +592,20 @@ constexpr int GM = 4;
 // projection followed by its GELU), and 2 writes out = rnd(rnd(sum) * gelu_tanh'(gx)), the GELU's
 // pullback of the product; both from the rounded 16-bit values the plain kernel stores, so the
 // bits equal the separate GELU passes.
+// EPI 3 (bf16 planes, SPLIT or not): the f32 product on bf16 MFMA. An activation row holds three
+// bf16 planes of an f32 row, [low | middle | high] of a.Kred columns each, whose sum is the f32
+// value exactly; wd holds the codes times a power of two, exact in bf16. The reduction walks the
+// low planes over the whole range first, then the middle, then the high ones (the weight again
+// from its start each time), so small terms are added up before large ones: against 64 bits the
+// sum is 3 to 6 times closer than a chain of fp32 MFMAs (5120 terms, signed data: 2.2e-7 against
+// 1.2e-6; all-positive: 3.9e-7 against 1.1e-6), whereas taking the three planes of each step
+// together loses to it on one-signed data (3.9e-6: the alignment inside the instruction truncates
+// small products next to a large accumulator). Three bf16 products at 16 times the fp32 MFMA rate;
+// 4680 x 1536 -> 8960 forward 1099 us with v_mfma_f32_16x16x4_f32, 383 us with this.
 template <int ELT, bool SPLIT, int EPI = 0>
 __global__ __launch_bounds__(512)
 void bfgemm_kernel(GemmArgs a, const uint16_t* __restrict__ wd, int tiles_n, int tiles_m) {
-  static_assert(EPI == 0 || !SPLIT, "the GELU epilogues run on the unsplit kernel");
+  static_assert(EPI == 0 || EPI == 3 || !SPLIT, "the GELU epilogues run on the unsplit kernel");
   using E = Elt<ELT>;
   typedef typename E::v8 V8;
   using namespace bfg;
@@ -624,8 +634,11 @@ void bfgemm_kernel(GemmArgs a, const uint16_t* __restrict__ wd, int tiles_n, int
   // this workgroup's reduction steps [kb, kb + nk) of 64
   const int nkt = (int)(Kred / BK);
   const int kb = (int)((int64_t)split * nkt / ks);
-  const int nk = (int)((int64_t)(split + 1) * nkt / ks) - kb;
-  const i32x4 ract = buffer_rsrc(a.act, (uint32_t)(M * Kred * 2));
+  int nkr = (int)((int64_t)(split + 1) * nkt / ks) - kb;
+  if constexpr (EPI == 3) nkr = __builtin_amdgcn_readfirstlane(nkr);  // scalar copy offsets below
+  const int nk = EPI == 3 ? 3 * nkr : nkr;  // EPI 3: the range once per plane
+  const int64_t lda = EPI == 3 ? 3 * Kred : Kred;
+  const i32x4 ract = buffer_rsrc(a.act, (uint32_t)(M * lda * 2));
   const i32x4 rw = buffer_rsrc(wd, (uint32_t)(Ncols * Kred * 2));
   uint32_t voa[4], vow[4];  // copies i: rows (w*4+i)*8 + lane/8 of each tile, 16 bytes per lane
 #pragma unroll
@@ -634,7 +647,7 @@ void bfgemm_kernel(GemmArgs a, const uint16_t* __restrict__ wd, int tiles_n, int
     const int c = (lane & 7) ^ bf_swz(row);
     const int64_t m = (m0 + row < M) ? m0 + row : M - 1;
     const int64_t n = (n0 + row < Ncols) ? n0 + row : Ncols - 1;
-    voa[i] = (uint32_t)((m * Kred + (int64_t)kb * BK + c * 8) * 2);
+    voa[i] = (uint32_t)((m * lda + (int64_t)kb * BK + c * 8) * 2);
     vow[i] = (uint32_t)((n * Kred + (int64_t)kb * BK + c * 8) * 2);
   }
   const i32x4 rnone = buffer_rsrc(a.act, 0u);  // zero records: a copy through it reads nothing
@@ -642,11 +655,16 @@ void bfgemm_kernel(GemmArgs a, const uint16_t* __restrict__ wd, int tiles_n, int
   // uses activation stage kt % 3 and weight stage kt % 2
   auto abase = [&](int kt) { return smem + (kt % 3) * ACT; };
   auto wbase = [&](int kt) { return smem + 3 * ACT + (kt & 1) * WB; };
+  // byte offsets of step kt from the range's start (EPI 3: plane pl of the row, step kt - pl nkr)
+  // (sign bits: comparisons would go through vector registers, and the offsets must be scalar)
+  auto plane = [&](int kt) { return (int)((uint32_t)(nkr - 1 - kt) >> 31) + (int)((uint32_t)(2 * nkr - 1 - kt) >> 31); };
+  auto woff = [&](int kt) { return (uint32_t)(EPI == 3 ? kt - plane(kt) * nkr : kt) * (BK * 2); };
+  auto aoff = [&](int kt) { return woff(kt) + (EPI == 3 ? (uint32_t)(plane(kt) * (int)Kred * 2) : 0u); };
   auto issue_act = [&](int kt, int i) {
-    dma16(ract, voa[i], (uint32_t)kt * (BK * 2), abase(kt) + (w * 4 + i) * 1024);
+    dma16(ract, voa[i], aoff(kt), abase(kt) + (w * 4 + i) * 1024);
   };
   auto issue_w = [&](int kt, int i) {
-    dma16(rw, vow[i], (uint32_t)kt * (BK * 2), wbase(kt) + (w * 4 + i) * 1024);
+    dma16(rw, vow[i], woff(kt), wbase(kt) + (w * 4 + i) * 1024);
   };
   // LoRA operands (rank up to 32): the L tile [256 tokens][32] and the R tile [256 columns][32],
   // rows of 64 bytes, zeros past the rank, copied before the first steps' copies into activation
@@ -666,6 +684,21 @@ void bfgemm_kernel(GemmArgs a, const uint16_t* __restrict__ wd, int tiles_n, int
     const uint32_t vo = (c * 8 < rp) ? (uint32_t)((origin + row) * rp * 2 + c * 16) : 0xFFFFFFF0u;
     const i32x4 rs = lr_lds ? buffer_rsrc(isr ? a.R : a.L, (uint32_t)(rows * rp * 2)) : rnone;
     dma16(rs, vo, 0u, abase(kt) + (isr ? 16384 : 0) + ci * 1024);
+  };
+
+  // EPI 3, ranks up to 32 (multiples of 4): the f32 L tile [256 tokens][32] and R tile [256
+  // columns][32] (128-byte rows, swizzled like the operand tiles, zeros past the rank) are copied
+  // in place of step nk - 2's copies of a step past the end: L into the activation stage, R into
+  // the weight stage that are free by then. Copy i of wave w as in the operand copies.
+  const bool flr_lds = EPI == 3 && a.fr > 0 && a.fr <= 32 && (a.fr & 3) == 0 && split == 0;
+  i32x4 rfl = rnone, rfr = rnone;
+  if (flr_lds) {
+    rfl = buffer_rsrc(a.fL, (uint32_t)(M * a.fr * 4));
+    rfr = buffer_rsrc(a.fR, (uint32_t)(Ncols * a.fr * 4));
+  }
+  auto flr_off = [&](int64_t origin, int i) {
+    const int row = (w * 4 + i) * 8 + (lane >> 3), c = (lane & 7) ^ bf_swz(row);
+    return c * 4 < a.fr ? (uint32_t)(((origin + row) * a.fr + c * 4) * 4) : 0xFFFFFFF0u;
   };
 
   f32x4 acc[4][8];  // [output-column tile][token tile]
@@ -777,7 +810,8 @@ void bfgemm_kernel(GemmArgs a, const uint16_t* __restrict__ wd, int tiles_n, int
       x[tj] = read_x(sa, 1, tj);
       if (tj == 0) read_w(sw, 1, w1);
       if (tj & 1) {
-        if constexpr (LR) dma16(rnone, 0u, 0u, abase(kt + 2) + (w * 4 + (tj >> 1)) * 1024);
+        if constexpr (LR && EPI == 3) dma16(rfl, flr_off(m0, tj >> 1), 0u, abase(kt + 2) + (w * 4 + (tj >> 1)) * 1024);
+        else if constexpr (LR) dma16(rnone, 0u, 0u, abase(kt + 2) + (w * 4 + (tj >> 1)) * 1024);
         else issue_act(kt + 2, tj >> 1);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -801,7 +835,8 @@ void bfgemm_kernel(GemmArgs a, const uint16_t* __restrict__ wd, int tiles_n, int
       __builtin_amdgcn_sched_barrier(0);
       x[tj] = read_x(san, 0, tj);
       if (tj & 1) {
-        if constexpr (LR) dma16(rnone, 0u, 0u, wbase(kt + 2) + (w * 4 + (tj >> 1)) * 1024);
+        if constexpr (LR && EPI == 3) dma16(rfr, flr_off(n0, tj >> 1), 0u, wbase(kt + 2) + (w * 4 + (tj >> 1)) * 1024);
+        else if constexpr (LR) dma16(rnone, 0u, 0u, wbase(kt + 2) + (w * 4 + (tj >> 1)) * 1024);
         else issue_w(kt + 2, tj >> 1);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -822,6 +857,114 @@ void bfgemm_kernel(GemmArgs a, const uint16_t* __restrict__ wd, int tiles_n, int
     for (int tj = 0; tj < 8; ++tj) mfma4(w1, x[tj], tj);
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);  // the last zero-record copies have landed
+
+  if constexpr (EPI == 3) {
+    // f32 epilogue: (acc colscale + bias) + c L R^T, the rank-r product on fp32 MFMA (a lane
+    // supplies 4 consecutive j, zeros past r) from the L and R tiles in LDS, or from global memory
+    // at ranks above 32 or no multiple of 4. Buffer accesses relative to the tile: 32-bit
+    // offsets, rows past the end read zeros and store nothing.
+    const int r = a.fr;
+    const bool lor_here = r > 0 && split == 0;
+    const int mrows = (int)(M - m0 < BM ? M - m0 : BM), ncols = (int)(Ncols - n0 < BN ? Ncols - n0 : BN);
+    auto rsrc = [](const float* p, int bytes) {
+      return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), (short)0, bytes, 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rL = rsrc(lor_here ? a.fL + m0 * r : a.fbias, lor_here ? mrows * r * 4 : 0);
+    const __amdgpu_buffer_rsrc_t rR = rsrc(lor_here ? a.fR + n0 * r : a.fbias, lor_here ? ncols * r * 4 : 0);
+    const __amdgpu_buffer_rsrc_t rS = rsrc(a.colscale + n0, a.colscale != nullptr ? ncols * 4 : 0);
+    const __amdgpu_buffer_rsrc_t rB = rsrc(a.fbias + n0, !SPLIT && a.fbias != nullptr ? ncols * 4 : 0);
+    auto ld4 = [](const __amdgpu_buffer_rsrc_t& rs, int off) {
+      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+    };
+    const bool scaled = a.colscale != nullptr;
+    if (flr_lds) {
+      __builtin_amdgcn_s_barrier();  // every wave's copies of L and R have landed
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const uint8_t* sL = abase(nk) + (wm * 128 + l16) * 128;
+    const uint8_t* sR = wbase(nk) + (wn * 64 + l16) * 128;
+    const int ldo = (int)(SPLIT ? a.ldp : Ncols);
+    float* dst = (SPLIT ? a.part + ((int64_t)split * M + m0) * ldo : a.fout + m0 * ldo) + n0;
+    const __amdgpu_buffer_rsrc_t rO = rsrc(dst, ((mrows - 1) * ldo + (SPLIT ? ldo - (int)n0 : ncols)) * 4);
+    // the column scales and the bias before the first store: a load after it would wait for the
+    // stores too (vmcnt counts both)
+    f32x4 sc[4], bs[4];
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) {
+      const int cb = (wn * 64 + ti * 16 + lq * 4) * 4;
+      sc[ti] = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
+      if (scaled) sc[ti] = ld4(rS, cb);
+      bs[ti] = ld4(rB, cb);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) {
+      const int cl = wn * 64 + ti * 16;
+#pragma unroll
+      for (int th = 0; th < 8; th += 4) {  // four token tiles at a time: registers
+        f32x4 lor[4];
+#pragma unroll
+        for (int tj = 0; tj < 4; ++tj) lor[tj] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (flr_lds) {
+#pragma unroll
+          for (int jc = 0; jc < 2; ++jc) {
+            const int off = ((4 * jc + lq) ^ swz) << 4;
+            const f32x4 rv = *reinterpret_cast<const f32x4*>(sR + ti * 2048 + off);
+            f32x4 lv[4];
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj) lv[tj] = *reinterpret_cast<const f32x4*>(sL + (th + tj) * 2048 + off);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int tj = 0; tj < 4; ++tj)
+                lor[tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[e], lv[tj][e], lor[tj], 0, 0, 0);
+          }
+        } else if (lor_here) {
+          for (int j0 = 0; j0 < r; j0 += 16) {
+            const int jl = j0 + lq * 4;
+            f32x4 rv = ld4(rR, jl < r ? ((cl + l16) * r + jl) * 4 : 0x7fffffff), lv[4];
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj)
+              lv[tj] = ld4(rL, jl < r ? ((wm * 128 + (th + tj) * 16 + l16) * r + jl) * 4 : 0x7fffffff);
+            if (r & 3) {  // a load may reach into the next row
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if (jl + e >= r) {
+                  rv[e] = 0.0f;
+#pragma unroll
+                  for (int tj = 0; tj < 4; ++tj) lv[tj][e] = 0.0f;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int tj = 0; tj < 4; ++tj)
+                lor[tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[e], lv[tj][e], lor[tj], 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int tj = 0; tj < 4; ++tj) {
+          const int row = wm * 128 + (th + tj) * 16 + l16, col = cl + lq * 4, off = (row * ldo + col) * 4;
+          f32x4 o;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) o[v] = (acc[ti][th + tj][v] * sc[ti][v] + bs[ti][v]) + a.c * lor[tj][v];
+          if (SPLIT || a.fvout) {
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rO,
+                                                   row < mrows && col < ncols ? off : 0x7fffffff, 0, 0);
+          } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[v]), rO,
+                                                    row < mrows && col + v < ncols ? off + 4 * v : 0x7fffffff, 0, 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    return;
+  }
 
   // epilogue: bias and one rounding per output (acc + bias, the LoRA term already in acc; ranks
   // above 32 add c lor here, their up-projection on MFMA with k = 32 per instruction and lanes
@@ -995,6 +1138,61 @@ int bfgemm_splits(int64_t M, int64_t Ncols, int64_t Kred) {
   if (s > nk / 4) s = nk / 4;
   if (s > 16) s = 16;
   return s < 2 ? 1 : (int)s;
+}
+
+// out[m][n] = sum over splits of part[sp][m][n] (split order) + bias[n], f32 (rows of part of ldp
+// floats, a multiple of 4): the reduction pass of the split GEMM on bf16 planes
+__global__ __launch_bounds__(256) void splitk_reduce_f32_kernel(const float* __restrict__ part, int ks,
+                                                                int64_t M, int64_t Ncols, int64_t ldp,
+                                                                const float* __restrict__ bias,
+                                                                float* __restrict__ out) {
+  const int64_t n4 = ldp / 4, total = M * n4, plane = M * ldp;
+  const int64_t step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += step) {
+    const int64_t m = i / n4, n = (i - m * n4) * 4;
+    f32x4 sum = *reinterpret_cast<const f32x4*>(part + i * 4);
+#pragma unroll 4
+    for (int sp = 1; sp < ks; ++sp) sum += *reinterpret_cast<const f32x4*>(part + sp * plane + i * 4);
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (n + v < Ncols) out[m * Ncols + n + v] = sum[v] + (bias != nullptr ? bias[n + v] : 0.0f);
+  }
+}
+
+int planegemm_splits(int64_t M, int64_t Ncols, int64_t Kp) {
+  const int64_t tiles = ceil_div(M, bfg::BM) * ceil_div(Ncols, bfg::BN);
+  if (tiles <= 0 || tiles >= 128) return 1;
+  int64_t s = (256 + tiles / 2) / tiles;
+  const int64_t nk = Kp / bfg::BK;
+  if (s > nk / 2) s = nk / 2;
+  if (s > 16) s = 16;
+  return s < 2 ? 1 : (int)s;
+}
+
+int launch_planegemm(int mode, const GemmArgs& a, const uint16_t* wd, hipStream_t st) {
+  if (a.Kred % bfg::BK != 0 || a.M * a.Kred * 6 >= ((int64_t)1 << 31) || a.Ncols * a.Kred * 2 >= ((int64_t)1 << 31) ||
+      (a.ksplit > 1 && (a.part == nullptr || a.ldp % 4 != 0 || a.ldp < a.Ncols || a.ksplit > a.Kred / bfg::BK)))
+    return fail(REELS_HIP_EINVAL, "planegemm: shape not supported");
+  static std::once_flag once;
+  static hipError_t attr_err = hipSuccess;
+  std::call_once(once, [&] {
+    const void* ks[] = {(const void*)bfgemm_kernel<REELS_HIP_BF16, false, 3>, (const void*)bfgemm_kernel<REELS_HIP_BF16, true, 3>};
+    for (const void* k : ks)
+      if (attr_err == hipSuccess) attr_err = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bfg::LDS);
+  });
+  if (attr_err != hipSuccess)
+    return fail(REELS_HIP_EHIP, std::string("planegemm: hipFuncSetAttribute: ") + hipGetErrorString(attr_err));
+  if (a.M == 0 || a.Ncols == 0) return REELS_HIP_OK;
+  const int tn = (int)ceil_div(a.Ncols, bfg::BN), tm = (int)ceil_div(a.M, bfg::BM);
+  { TraceScope _ts(st, mode == 0 ? "planegemm_kernel<0>" : "planegemm_kernel<1>");
+    if (a.ksplit > 1) bfgemm_kernel<REELS_HIP_BF16, true, 3><<<tn * tm * a.ksplit, bfg::NT, bfg::LDS, st>>>(a, wd, tn, tm);
+    else bfgemm_kernel<REELS_HIP_BF16, false, 3><<<tn * tm, bfg::NT, bfg::LDS, st>>>(a, wd, tn, tm); }
+  if (int rc = check_launch("planegemm_kernel")) return rc;
+  if (a.ksplit <= 1) return REELS_HIP_OK;
+  const int64_t n4 = ceil_div(a.M * (a.ldp / 4), 256);
+  { TraceScope _ts(st, "splitk_reduce_f32_kernel");
+    splitk_reduce_f32_kernel<<<(unsigned)(n4 < 4096 ? n4 : 4096), 256, 0, st>>>(a.part, a.ksplit, a.M, a.Ncols, a.ldp, a.fbias, a.fout); }
+  return check_launch("splitk_reduce_f32_kernel");
 }
 
 bool bfgemm_fuses_gelu(const GemmArgs& a) {

@@ -1196,6 +1196,18 @@ int launch_reduce_partials(const float* part, int splits, int64_t Od, int rp, in
   return check_launch("reduce_partials_kernel");
 }
 
+int launch_reduce_partials2(const float* partA, int splitsA, int64_t OdA, float* outA,
+                            const float* partB, int splitsB, int64_t OdB, float* outB, int rp,
+                            int r, float c, const float* bpart, float* bout, hipStream_t st) {
+  const int nb0 = (int)ceil_div(OdA * r, 256), nb1 = (int)(ceil_div(OdB, 8) * ceil_div(r, 32));
+  const int nb2 = bpart ? (int)ceil_div(OdB, 256) : 0;
+  { TraceScope _ts(st, "reduce_partials2_kernel");
+    reduce_partials2_kernel<<<(unsigned)(nb0 + nb1 + nb2), 256, 0, st>>>(
+        RpJob{partA, outA, OdA, splitsA}, RpJob{partB, outB, OdB, splitsB}, nb0, rp, r, c,
+        RpJob{bpart, bout, OdB, splitsB}, nb0 + nb1); }
+  return check_launch("reduce_partials2_kernel");
+}
+
 }  // namespace reels
 
 using namespace reels;

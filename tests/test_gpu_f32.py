@@ -190,3 +190,84 @@ def test_f32_gelu_tanh(dev, n):
         bad = np.flatnonzero(~ok)
         assert bad.size == 0, (what, [(int(i), float(got[i]), float(want[i]), float(xs[i]))
                                       for i in bad[:6]])
+
+
+@pytest.mark.parametrize("M,K,N,r,bias", [
+    (1, 130, 66, 2, True),       # one token; K, N not multiples of 4; split reductions
+    (257, 63, 65, 5, True),      # lengths around one GEMM step of 64, rank not a multiple of 4
+    (129, 65, 257, 40, False),   # a second output tile of one column, rank above one LDS tile
+    (33, 191, 1, 1, True),       # one output column
+    (300, 320, 260, 160, True),  # rank above one chunk of 128
+    (2100, 72, 1000, 24, True),  # many token splits, ragged output columns
+])
+def test_f32_plane_gemm_edges(dev, M, K, N, r, bias):
+    """The products on bf16 planes at the edges of their tiles and steps: every output against the
+    oracle within the file's 1e-5 (the planes are exact, the sums f32), and the result of unaligned
+    (4-byte aligned) operands equal to that of aligned copies bit for bit."""
+    import torch
+    from reels_amd import QuantizedMatrix, i8lora_forward
+    cs = make_case(M, K, N, r, float(r), seed=900 + M + K + N + r, bias=bias)
+    g = check(dev, cs, f"planes {M}x{K}x{N}r{r}")
+    flat = torch.zeros((M * K + 1,), device=dev)
+    flat[1:] = todev(cs["x"], dev).reshape(-1)
+    x = flat[1:].view(M, K)
+    assert x.data_ptr() % 16 != 0
+    W = QuantizedMatrix(todev(cs["q"], dev), todev(cs["s"], dev), torch.float32)
+    y, _ = i8lora_forward(x, W, todev(cs["A"], dev), todev(cs["B"], dev),
+                          todev(cs["bias"], dev) if bias else None, cs["c"])
+    torch.cuda.synchronize(dev)
+    assert np.array_equal(y.cpu().numpy(), g["y"])
+
+
+def test_f32_token_chunks(dev):
+    # 40200 tokens x 8960: the planes of x would exceed 2 GiB, so the forward runs as two chunks;
+    # rows on both sides of the boundary against f64 products, h in full
+    import torch
+    from reels_amd import QuantizedMatrix, i8lora_forward
+    M, K, N, r = 40200, 8960, 96, 8
+    print(f"[f32] token chunks {M}x{K}x{N}r{r}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn((M, K), generator=g, device=dev)
+    q = torch.randint(-127, 128, (N, K), generator=g, device=dev).to(torch.int8)
+    s = torch.rand((N,), generator=g, device=dev) * 1e-3
+    A = torch.randn((K, r), generator=g, device=dev) * 0.01
+    B = torch.randn((r, N), generator=g, device=dev) * 0.01
+    y, h = i8lora_forward(x, QuantizedMatrix(q, s, torch.float32), A, B, None, 0.5, save_h=True)
+    rows = torch.tensor([0, 255, 20223, 20224, 20479, 20480, 40199], device=dev)
+    xd = x[rows].double()
+    hd = xd @ A.double()
+    yd = xd @ (q.double() * s.double()[:, None]).t() + 0.5 * hd @ B.double()
+    assert_parity(y[rows].cpu().numpy(), yd.cpu().numpy(), "chunked y", tol=TOL)
+    assert_parity(h[rows].cpu().numpy(), hd.cpu().numpy(), "chunked h", tol=TOL)
+
+
+def test_f32_special_values(dev):
+    """Infinities and NaNs reach exactly the rows they are in, values near the ends of the f32 range
+    keep f32's relative precision, scales of zero and of subnormal size multiply as fl32(q s)."""
+    import torch
+    from reels_amd import QuantizedMatrix, i8lora_backward, i8lora_forward
+    M, K, N = 9, 70, 12
+    x = f32v(950, (M, K), 1.0)
+    q = np.random.default_rng(951).integers(1, 128, (N, K)).astype(np.int8)
+    s = np.full(N, 1e-3, np.float32)
+    s[3], s[4], s[5] = 0.0, 1e-39, -2e-3
+    x[1, 7], x[2, 7], x[3, 7], x[3, 9] = np.inf, np.nan, np.inf, -np.inf
+    x[4] *= np.float32(1e34)
+    x[5] *= np.float32(1e-30)
+    x[6, 0] = np.uint32(0x7f800001).view(np.float32)  # a NaN whose upper half alone is Inf
+    W = QuantizedMatrix(todev(q, dev), todev(s, dev), torch.float32)
+    y = i8lora_forward(todev(x, dev), W)[0].cpu().numpy()
+    with np.errstate(all="ignore"):
+        ref = x.astype(np.float64) @ (q.astype(np.float64) * s.astype(np.float64)[:, None]).T
+    ok = s != 0  # Inf times a zero weight is NaN
+    assert np.isinf(y[1, ok]).all() and (np.sign(y[1, ok]) == np.sign(s[ok])).all()
+    assert np.isnan(y[2]).all() and np.isnan(y[3]).all() and np.isnan(y[6]).all()
+    for m in (0, 4, 5, 7, 8):
+        big = np.abs(ref[m]) > 1e-36  # results above f32's subnormal range
+        scale = np.abs(x[m].astype(np.float64)) @ (np.abs(q.astype(np.float64)) * np.abs(s)[:, None]).T
+        assert (np.abs(y[m] - ref[m])[big] <= 1e-6 * scale[big]).all(), m
+    assert (y[0, 3] == 0) and (y[4, 3] == 0)
+    dy = f32v(952, (M, N), 1.0)
+    dy[1, 2], dy[2, 3] = np.inf, np.nan
+    dx = i8lora_backward(todev(dy, dev), None, W, want_dA=False, want_dB=False)[0].cpu().numpy()
+    assert np.isinf(dx[1]).all() and np.isnan(dx[2]).all() and np.isfinite(dx[[0, 3, 4]]).all()
