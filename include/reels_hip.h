@@ -97,7 +97,8 @@ size_t reels_hip_i8lora_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t
  *   y = bf16(sum_k x[m][k] W[n][k] + lora_scale * sum_j h[m][j] B[j][n] + bias[n])
  * with W = bf16(fl32(q * s)) written into the workspace once per call when K and N are multiples
  * of 64 and there are many tokens (the reference's _materialize_weight, quantization.jl:54-64);
- * otherwise W = q * s exact with s[n] applied to the f32 sum: K or N not a multiple of 64, and the
+ * otherwise W = q * s exact with s[n] applied to the f32 sum: K or N not a multiple of 64 (on
+ * zero-padded copies in the workspace), and the
  * few-token path (M <= 240, or M <= 1024 with N * K <= 2^22; K and N multiples of 64), which
  * reads the int8 codes without a weight copy. With few 256 x 256 output tiles (a few hundred
  * tokens) the GEMM splits its reduction over several workgroups and sums their f32 partials in a
@@ -140,7 +141,8 @@ int reels_hip_i8lora_fwd_f16(const void* x, const int8_t* q, const float* scales
  *     return REELS_HIP_EINVAL before any work;
  *   - it always multiplies the int8 codes (s applied to the f32 sum), never a dequantized bf16
  *     copy, so its y can differ from reels_hip_i8lora_fwd's in the last bf16 bit where that entry
- *     point takes the dequantized-weight path (K and N multiples of 64);
+ *     point takes the dequantized-weight path (K and N multiples of 64), and where K or N is not a
+ *     multiple of 64 and that entry point's zero-padded copies do not fit the scratch;
  *   - calls that overlap on one GPU (other streams or threads) race on the shared scratch.
  */
 int reels_hip_i8lora_fwd_noalloc(const void* x, const int8_t* q, const float* scales,
@@ -154,9 +156,11 @@ int reels_hip_i8lora_fwd_noalloc(const void* x, const int8_t* q, const float* sc
  *   u  = bf16(dy * B^T)                                                      [M][r]
  *   dx = bf16(sum_n dy[m][n] W[n][k] + lora_scale * sum_j u[m][j] A[k][j])
  *   dA = lora_scale * x^T u   (f32 [K][r]);   dB = lora_scale * h^T dy   (f32 [r][N])
- * W = bf16(fl32(q * s)) when K and N are multiples of 64 (a transposed copy in the workspace, or,
- * on the few-token path of reels_hip_i8lora_fwd, built in registers from the codes); when K or N
- * is not a multiple of 64 the product is taken as sum_n bf16(dy[m][n] s[n]) q[n][k]. h: the
+ * W = bf16(fl32(q * s)) (a transposed copy in the workspace, or, on the few-token path of
+ * reels_hip_i8lora_fwd, built in registers from the codes); K or N that are no multiples of 64 are
+ * zero-padded in the workspace. On the smallest such layers (up to 64 tokens, K and N up to 128),
+ * at sizes those copies do not support and with unaligned operands at multiples of 64, the product
+ * is taken as sum_n bf16(dy[m][n] s[n]) q[n][k]. h: the
  * forward's h_save ([M][r]) or NULL to recompute it.
  * dx, dA, dB may each be NULL to skip that output. r = 0 gives dx = deq(W)^T dy alone
  * (_weight_transpose_mul). dA and dB are overwritten (not accumulated) and are bitwise

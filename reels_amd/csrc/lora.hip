@@ -11,11 +11,13 @@
 //      (no float atomics: bitwise reproducible)                          (HBM-bound)
 // Every rank takes the fast kernels: the LoRA panels h, u and the adapter operands live in the
 // workspace with rp = round_up(r, 16) columns (zeros past r), and the projection and gradient
-// kernels run in rank chunks of up to 128. Shapes the fast kernels do not take (K or N not
-// multiples of 16, unaligned pointers) run through the generic kernels at the bottom, which
-// compute the same formulas with the same bf16 rounding points, one output element per thread.
+// kernels run in rank chunks of up to 128. Widths that are no multiples of 64 run on operands
+// zero-padded to the next multiples in the workspace (pad_shape). What neither takes (unaligned
+// pointers, widths of 2^22 and more) runs through the generic kernels at the bottom, which compute
+// the same formulas with the same bf16 rounding points, one output element per thread.
 #include "i8gemm.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace reels {
@@ -682,6 +684,53 @@ __global__ void fill_f32_kernel(float* p, int64_t n, float v) {
 // dst[i][j] = j < cols ? src[i][j] : 0 for j < cols_dst (16-bit elements; rows of ld_src and
 // ld_dst): widens a [rows][r] LoRA operand to the padded [rows][rp] layout of the fast kernels,
 // or (cols = cols_dst = r) compacts a padded one back to [rows][r]
+// Up to kMaxCopies 2-d copies in one launch: rows of bsrc valid bytes at stride lds go to rows of
+// bdst bytes at stride ldd, zeros past the valid bytes and past rows_src. Any alignment (a 16-byte
+// access at any address is one instruction; only the piece across the end of a row goes byte by
+// byte). Four 16-byte pieces per thread, their loads issued together.
+struct CopyJob {
+  const uint8_t* src;
+  uint8_t* dst;
+  int64_t lds, ldd, bsrc, bdst, rows_src;
+  uint32_t cpr, total;  // 16-byte pieces per output row, in all
+};
+constexpr int kMaxCopies = 8, kCopyPieces = 4;
+struct CopyJobs {
+  CopyJob j[kMaxCopies];
+  uint32_t end[kMaxCopies];  // first block past each job's
+  int n;
+};
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+__global__ __launch_bounds__(256) void copy2d_kernel(CopyJobs js) {
+  int k = 0;
+  while (k + 1 < js.n && blockIdx.x >= js.end[k]) ++k;
+  const CopyJob& a = js.j[k];
+  const uint32_t b = blockIdx.x - (k > 0 ? js.end[k - 1] : 0u);
+  u32x4 v[kCopyPieces];
+#pragma unroll
+  for (int i = 0; i < kCopyPieces; ++i) {
+    const uint32_t id = (b * kCopyPieces + i) * 256u + threadIdx.x;
+    v[i] = u32x4{0u, 0u, 0u, 0u};
+    if (id >= a.total) continue;
+    const uint32_t row = id / a.cpr, off = (id - row * a.cpr) * 16u;
+    if (row >= a.rows_src) continue;
+    const uint8_t* p = a.src + row * a.lds + off;
+    if (off + 16 <= a.bsrc) v[i] = *reinterpret_cast<const u32x4_any*>(p);
+    else
+      for (int e = 0; off + e < a.bsrc; ++e) v[i][e >> 2] |= (uint32_t)p[e] << (8 * (e & 3));
+  }
+#pragma unroll
+  for (int i = 0; i < kCopyPieces; ++i) {
+    const uint32_t id = (b * kCopyPieces + i) * 256u + threadIdx.x;
+    if (id >= a.total) continue;
+    const uint32_t row = id / a.cpr, off = (id - row * a.cpr) * 16u;
+    uint8_t* p = a.dst + row * a.ldd + off;
+    if (off + 16 <= a.bdst) *reinterpret_cast<u32x4_any*>(p) = v[i];
+    else
+      for (int e = 0; off + e < a.bdst; ++e) p[e] = (uint8_t)(v[i][e >> 2] >> (8 * (e & 3)));
+  }
+}
+
 __global__ void pad_cols_kernel(const uint16_t* __restrict__ src, int64_t rows, int cols,
                                 int64_t ld_src, uint16_t* __restrict__ dst, int cols_dst,
                                 int64_t ld_dst) {
@@ -957,7 +1006,87 @@ static WsLayout ws_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which,
   return w;
 }
 
+// Widths that are no multiples of 64: the call runs on copies zero-padded to the next multiples
+// (Kp, Np) in the workspace, so it meets the same kernels as any other shape, and the outputs'
+// valid parts are copied out. The forward then multiplies the int8 codes (s on the f32 sum), as
+// the direct kernels do for these widths; dX multiplies the dequantized weight. The copies cost a
+// read and a write of each operand, four launches of 5-9 us in 88 us forward and backward for 777
+// tokens, 1000 -> 3000; the one-output-per-thread kernels took 11.0 ms there, and widths that are
+// multiples of 16 ran unsplit 256 x 256 tiles (1000 tokens, 528 -> 2064: 236 against 89 us). dX's
+// error against 64 bits stays: 2.341e-3 to 2.349e-3 with rnd(dy s) times the codes, 2.343e-3 to
+// 2.347e-3 with rnd(q s), over seven shapes.
+static bool pad_shape(int64_t M, int64_t K, int64_t N) {
+  if (K % 64 == 0 && N % 64 == 0) return false;
+  // tiny layers: the direct kernels' single launch is shorter than the copies' launches (one token,
+  // 100 -> 100 forward 14 against 21 us; 64 tokens forward and backward 60 us either way; 256 tokens
+  // 91 against 63, 16 tokens 200 -> 200 78 against 65, 300 -> 100 forward 26 against 21)
+  if (M <= 64 && K <= 128 && N <= 128) return false;
+  const int64_t Kp = (K + 63) / 64 * 64, Np = (N + 63) / 64 * 64, most = (int64_t)1 << 31;
+  return Kp < ((int64_t)1 << 22) && Np < ((int64_t)1 << 22) && Kp * Np * 2 < most &&
+         M * std::max(Kp, Np) / 8 < most;  // the copies count their 16-byte pieces in 32 bits
+}
+
+struct PadLayout {
+  int64_t Kp, Np, rp;  // padded widths, and the rank padded to a multiple of 16
+  size_t q, s, x, A, B, bias, y, h, dy, dx, dA, dB, db, inner, total;
+  Plan p;  // the plan of the padded call
+};
+
+static PadLayout pad_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which) {
+  PadLayout w{};
+  w.Kp = (K + 63) / 64 * 64;
+  w.Np = (N + 63) / 64 * 64;
+  w.rp = (r + 15) / 16 * 16;
+  r = w.rp;
+  size_t off = 0;
+  auto take = [&](size_t bytes) { size_t o = off; off = align_up(off + bytes, 256); return o; };
+  w.q = take((size_t)w.Np * w.Kp);
+  w.s = take((size_t)w.Np * 4);
+  w.x = take((size_t)M * w.Kp * 2);
+  w.A = take((size_t)w.Kp * r * 2);
+  w.B = take((size_t)w.Np * r * 2);
+  w.h = take((size_t)M * r * 2);
+  if (which == REELS_HIP_WS_FWD) {
+    w.bias = take((size_t)w.Np * 2);
+    w.y = take((size_t)M * w.Np * 2);
+  } else {
+    w.dy = take((size_t)M * w.Np * 2);
+    w.dx = take((size_t)M * w.Kp * 2);
+    w.dA = take((size_t)w.Kp * r * 4);
+    w.dB = take((size_t)w.Np * r * 4);
+    w.db = take((size_t)w.Np * 4);
+  }
+  w.p = make_plan(M, w.Kp, w.Np, r, true);
+  if (which == REELS_HIP_WS_FWD && !w.p.skinny) w.p.i8f = w.p.deq;
+  w.inner = off;
+  w.total = off + ws_layout(M, w.Kp, w.Np, r, which, w.p).total;
+  return w;
+}
+
 static int grid1(int64_t n, int bs = 256) { return (int)ceil_div(n, bs); }
+
+// collects 2-d copies (rows x cols elements of esz bytes, zero-padded to rows_d x cols_d) and runs
+// them as one launch
+struct Copies {
+  CopyJobs js{};
+  uint32_t blocks = 0;
+  void add(const void* src, int64_t rows, int64_t cols, int64_t lds, void* dst, int64_t rows_d,
+           int64_t cols_d, int64_t ldd, int esz) {
+    if (rows_d <= 0 || cols_d <= 0) return;
+    CopyJob& j = js.j[js.n];
+    j.src = static_cast<const uint8_t*>(src); j.dst = static_cast<uint8_t*>(dst);
+    j.lds = lds * esz; j.ldd = ldd * esz; j.bsrc = cols * esz; j.bdst = cols_d * esz; j.rows_src = rows;
+    j.cpr = (uint32_t)ceil_div(j.bdst, 16);
+    j.total = (uint32_t)(rows_d * j.cpr);
+    blocks += (uint32_t)ceil_div(j.total, 256 * kCopyPieces);
+    js.end[js.n++] = blocks;
+  }
+  int launch(hipStream_t st) const {
+    if (js.n == 0) return REELS_HIP_OK;
+    { TraceScope _ts(st, "copy2d_kernel"); copy2d_kernel<<<blocks, 256, 0, st>>>(js); }
+    return check_launch("copy2d_kernel");
+  }
+};
 
 // out[c][r] = in[r][c] (rows_pad >= rows output rows, zeros past rows) for one or two matrices
 // in one launch (in1 NULL: one)
@@ -1212,6 +1341,9 @@ int launch_reduce_partials2(const float* partA, int splitsA, int64_t OdA, float*
 
 using namespace reels;
 
+// scratch of the allocation-free forward (below)
+constexpr size_t kScratchBytes = (size_t)32 << 20;
+
 extern "C" size_t reels_hip_i8lora_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t r,
                                                    int which) {
   if (M < 0 || K < 0 || N < 0 || r < 0) return 0;
@@ -1219,6 +1351,10 @@ extern "C" size_t reels_hip_i8lora_workspace_bytes(int64_t M, int64_t K, int64_t
     return 0;
   // sized for the fast layout when the shape allows it (pointer alignment cannot be known here;
   // the fast layout is never smaller than the generic one)
+  if (K > 0 && N > 0 && pad_shape(M, K, N)) {
+    const size_t t = pad_layout(M, K, N, r, which == REELS_HIP_WS_BWD ? which : REELS_HIP_WS_FWD).total;
+    if (which != REELS_HIP_WS_FWD_NOALLOC || t <= kScratchBytes) return t;
+  }
   Plan p = make_plan(M, K, N, r, true);
   if (which == REELS_HIP_WS_FWD_NOALLOC) {
     noalloc_plan(p);
@@ -1237,7 +1373,6 @@ static bool all_aligned(std::initializer_list<const void*> ps) {
 // Scratch of reels_hip_i8lora_fwd_noalloc: one array per GPU, held until the process ends. Host
 // code never uses the array's name as an address (on the host it is a stand-in symbol); the
 // device address comes from hipGetSymbolAddress, once per device, on that device's first call.
-constexpr size_t kScratchBytes = (size_t)32 << 20;
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
@@ -1263,13 +1398,24 @@ static int scratch_for_current_device(const char* fn, void** out) {
   return REELS_HIP_OK;
 }
 
+static int padded_fwd(int elt, const char* fn, const PadLayout& w, const void* x, const int8_t* q,
+                      const float* scales, const void* A, const void* B, const void* bias, int64_t M,
+                      int64_t K, int64_t N, int64_t r, float lora_scale, void* y, void* h_save,
+                      uint8_t* ws, size_t ws_bytes, void* stream);
+static int padded_bwd(int elt, const char* fn, const PadLayout& w, const void* dy, const void* x,
+                      const void* h, const int8_t* q, const float* scales, const void* A,
+                      const void* B, int64_t M, int64_t K, int64_t N, int64_t r, float lora_scale,
+                      void* dx, float* dA, float* dB, float* dbias, uint8_t* ws, size_t ws_bytes,
+                      void* stream);
+
 // noalloc: never the dequantized-weight plan (its N*K*2-byte copy is what would not fit a modest
 // scratch), the workspace is the device's scratch array
 static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t* q,
                            const float* scales, const void* A, const void* B, const void* bias,
                            int64_t M, int64_t K, int64_t N, int64_t r, float lora_scale, void* y,
                            void* h_save, void* workspace, size_t ws_bytes, void* stream,
-                           bool noalloc = false, void* gout = nullptr, bool* gelu_fused = nullptr) {
+                           bool noalloc = false, void* gout = nullptr, bool* gelu_fused = nullptr,
+                           bool codes = false) {
   clear_error();
   if (M < 0 || K <= 0 || N <= 0 || r < 0 || r > 4096)
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": " "need M >= 0, K > 0, N > 0, 0 <= r <= 4096");
@@ -1278,10 +1424,27 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
   if (M == 0) return REELS_HIP_OK;
   if (!x || !q || !scales || !y || (r > 0 && (!A || !B)))
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": " "NULL x, q, scales, y, or A/B with r > 0");
+  if (pad_shape(M, K, N)) {
+    const PadLayout w = pad_layout(M, K, N, r, REELS_HIP_WS_FWD);
+    // without a workspace the padded copies have to fit the scratch; beyond it the direct kernels run
+    if (!noalloc || w.total <= kScratchBytes) {
+      if (noalloc) {
+        if (int rc = scratch_for_current_device(fn, &workspace)) return rc;
+        ws_bytes = kScratchBytes;
+      }
+      if (workspace == nullptr || ws_bytes < w.total)
+        return fail(REELS_HIP_EWORKSPACE, std::string(fn) + ": " "workspace NULL or smaller than "
+                                          "reels_hip_i8lora_workspace_bytes(..., REELS_HIP_WS_FWD)");
+      if (aligned16(workspace))
+        return padded_fwd(elt, fn, w, x, q, scales, A, B, bias, M, K, N, r, lora_scale, y, h_save,
+                          static_cast<uint8_t*>(workspace), ws_bytes, stream);
+    }
+  }
   const bool al = all_aligned({x, q, scales, A, B, y, h_save}) &&
                   (bias == nullptr || (reinterpret_cast<uintptr_t>(bias) & 7u) == 0);
   Plan p = make_plan(M, K, N, r, al);
   if (noalloc) noalloc_plan(p);
+  if (codes && !p.skinny) p.i8f = p.deq;  // the forward of a padded call multiplies the codes
   WsLayout w = ws_layout(M, K, N, r, REELS_HIP_WS_FWD, p);
   if (noalloc) {
     if (w.total > kScratchBytes)
@@ -1392,6 +1555,15 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": " "NULL dy, q, scales, A/B with r > 0, or x "
                                   "needed for dA / recomputing h");
   if (!dx && !dA && !dB && !dbias) return REELS_HIP_OK;
+  if (pad_shape(M, K, N)) {
+    const PadLayout w = pad_layout(M, K, N, r, REELS_HIP_WS_BWD);
+    if (workspace == nullptr || ws_bytes < w.total)
+      return fail(REELS_HIP_EWORKSPACE, std::string(fn) + ": " "workspace NULL or smaller than "
+                                        "reels_hip_i8lora_workspace_bytes(..., REELS_HIP_WS_BWD)");
+    if (aligned16(workspace))
+      return padded_bwd(elt, fn, w, dy, x, h, q, scales, A, B, M, K, N, r, lora_scale, dx, dA, dB,
+                        dbias, static_cast<uint8_t*>(workspace), ws_bytes, stream);
+  }
   const bool al = all_aligned({dy, x, h, q, scales, A, B, dx, dA, dB, dbias});
   Plan p = make_plan(M, K, N, r, al);
   WsLayout w = ws_layout(M, K, N, r, REELS_HIP_WS_BWD, p);
@@ -1543,6 +1715,86 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
   if (dbias && !dB)
     return launch_colsum(elt, dyb, M, N, reinterpret_cast<float*>(ws + w.pbias), dbias, st);
   return REELS_HIP_OK;
+}
+
+// The padded forms (pad_shape): operands copied zero-padded into the workspace, the call on the
+// padded sizes (the rank padded to a multiple of 16 too: the inner call then copies no panels of its
+// own), the valid outputs copied out. An operand whose width needs no padding and that is
+// 16-byte aligned is used in place, as is such an output.
+static int padded_fwd(int elt, const char* fn, const PadLayout& w, const void* x, const int8_t* q,
+                      const float* scales, const void* A, const void* B, const void* bias, int64_t M,
+                      int64_t K, int64_t N, int64_t r, float lora_scale, void* y, void* h_save,
+                      uint8_t* ws, size_t ws_bytes, void* stream) {
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const int64_t Kp = w.Kp, Np = w.Np, rp = w.rp;
+  Copies in, out;
+  in.add(q, N, K, K, ws + w.q, Np, Kp, Kp, 1);
+  in.add(scales, 1, N, N, ws + w.s, 1, Np, Np, 4);
+  const void *xp = x, *Ap = A, *Bp = B, *bp = bias;
+  void *yp = y, *hp = h_save;
+  if (Kp != K || !aligned16(x)) { in.add(x, M, K, K, ws + w.x, M, Kp, Kp, 2); xp = ws + w.x; }
+  if (r > 0) {
+    in.add(A, K, r, r, ws + w.A, Kp, rp, rp, 2);
+    in.add(B, r, N, N, ws + w.B, rp, Np, Np, 2);
+    Ap = ws + w.A;
+    Bp = ws + w.B;
+  }
+  if (bias) { in.add(bias, 1, N, N, ws + w.bias, 1, Np, Np, 2); bp = ws + w.bias; }
+  if (Np != N || !aligned16(y)) { yp = ws + w.y; out.add(yp, M, N, Np, y, M, N, N, 2); }
+  if (h_save && r > 0 && (rp != r || !aligned16(h_save))) { hp = ws + w.h; out.add(hp, M, r, rp, h_save, M, r, r, 2); }
+  if (int rc = in.launch(st)) return rc;
+  if (int rc = i8lora_fwd_impl(elt, fn, xp, reinterpret_cast<const int8_t*>(ws + w.q),
+                               reinterpret_cast<const float*>(ws + w.s), Ap, Bp, bp, M, Kp, Np, rp,
+                               lora_scale, yp, hp, ws + w.inner, ws_bytes - w.inner, stream, false,
+                               nullptr, nullptr, true))
+    return rc;
+  return out.launch(st);
+}
+
+static int padded_bwd(int elt, const char* fn, const PadLayout& w, const void* dy, const void* x,
+                      const void* h, const int8_t* q, const float* scales, const void* A,
+                      const void* B, int64_t M, int64_t K, int64_t N, int64_t r, float lora_scale,
+                      void* dx, float* dA, float* dB, float* dbias, uint8_t* ws, size_t ws_bytes,
+                      void* stream) {
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const int64_t Kp = w.Kp, Np = w.Np, rp = w.rp;
+  Copies in, out;
+  in.add(q, N, K, K, ws + w.q, Np, Kp, Kp, 1);
+  in.add(scales, 1, N, N, ws + w.s, 1, Np, Np, 4);
+  const void *dyp = dy, *xp = x, *hp = h, *Ap = A, *Bp = B;
+  void* dxp = dx;
+  float *dAp = dA, *dBp = dB, *dbp = dbias;
+  if (Np != N || !aligned16(dy)) { in.add(dy, M, N, N, ws + w.dy, M, Np, Np, 2); dyp = ws + w.dy; }
+  // x is read for dA and to recompute h only
+  const bool need_x = x && r > 0 && (dA || (dB && !h));
+  if (need_x && (Kp != K || !aligned16(x))) { in.add(x, M, K, K, ws + w.x, M, Kp, Kp, 2); xp = ws + w.x; }
+  if (!need_x) xp = nullptr;
+  if (h && r > 0 && (rp != r || !aligned16(h))) { in.add(h, M, r, r, ws + w.h, M, rp, rp, 2); hp = ws + w.h; }
+  if (r > 0) {
+    in.add(A, K, r, r, ws + w.A, Kp, rp, rp, 2);
+    in.add(B, r, N, N, ws + w.B, rp, Np, Np, 2);
+    Ap = ws + w.A;
+    Bp = ws + w.B;
+  }
+  if (dx && (Kp != K || !aligned16(dx))) { dxp = ws + w.dx; out.add(dxp, M, K, Kp, dx, M, K, K, 2); }
+  if (dA && (Kp != K || rp != r || !aligned16(dA))) {
+    dAp = reinterpret_cast<float*>(ws + w.dA);
+    out.add(dAp, K, r, rp, dA, K, r, r, 4);
+  }
+  if (dB && (rp != r || Np != N || !aligned16(dB))) {
+    dBp = reinterpret_cast<float*>(ws + w.dB);
+    out.add(dBp, r, N, Np, dB, r, N, N, 4);
+  }
+  if (dbias && (Np != N || !aligned16(dbias))) {
+    dbp = reinterpret_cast<float*>(ws + w.db);
+    out.add(dbp, 1, N, Np, dbias, 1, N, N, 4);
+  }
+  if (int rc = in.launch(st)) return rc;
+  if (int rc = i8lora_bwd_impl(elt, fn, dyp, xp, hp, reinterpret_cast<const int8_t*>(ws + w.q),
+                               reinterpret_cast<const float*>(ws + w.s), Ap, Bp, M, Kp, Np, rp,
+                               lora_scale, dxp, dAp, dBp, dbp, ws + w.inner, ws_bytes - w.inner, stream))
+    return rc;
+  return out.launch(st);
 }
 
 static int gelu_impl(int elt, const char* fn, const void* x, void* y, int64_t n, void* stream) {
