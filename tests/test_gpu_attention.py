@@ -333,3 +333,53 @@ def test_attention_generic_no_visible_key_and_no_keys(dev):
     res = memory_efficient_attention(q, kk, kk)
     torch.cuda.synchronize()
     assert torch.isnan(res.output).all() and torch.isneginf(res.cache.logsumexp).all()
+
+
+@pytest.mark.parametrize("B,Sq,Sk,H,D,causal,masked,dt", [
+    (1, 63, 65, 1, 33, False, False, "f32"),     # past one 32-wide block of the head dim
+    (1, 64, 64, 2, 96, True, False, "f32"),      # whole tiles
+    (1, 65, 31, 2, 97, False, True, "f32"),      # past the 96-wide kernels, keys below one tile
+    (2, 500, 129, 40, 36, False, False, "f32"),  # more than one workgroup per CU: eight waves
+    (2, 129, 500, 40, 65, True, True, "f16"),    # the same over keys, rows off 16-byte alignment
+    (2, 500, 257, 40, 72, False, False, "bf16"),
+    (1, 127, 128, 3, 127, False, True, "bf16"),  # odd head dim and mask rows
+    (1, 17, 1, 2, 16, False, False, "f16"),      # one key
+])
+def test_attention_generic_tile_edges(dev, B, Sq, Sk, H, D, causal, masked, dt):
+    test_attention_generic_parity(dev, B, Sq, Sk, H, D, causal, masked, dt)
+
+
+def test_attention_generic_large_scores_and_values(dev):
+    """f32 scores of about +-40 (the running maximum moves within a row, most probabilities vanish)
+    and values near the end of the f32 range. A score s carries a relative error of a few 2^-24, so
+    a probability one of |s| 2^-22, 1e-5 at 40: the bar is 5e-5. An infinite value gives outputs
+    of its sign in its element, whatever the low bits of the probabilities, and no others."""
+    import torch
+    from reels_amd import memory_efficient_attention
+    d = torch.device("cuda:0")
+    print("[case] generic attention, large scores", flush=True)
+    q, k, v, _ = _inputs(1, 70, 150, 2, 48, 77, "f32")
+    q = q * np.float32(8)
+    v2 = v * np.float32(1e37)
+    for vals, scale in ((v, 1.0), (v2, 1e37)):
+        res = memory_efficient_attention(*(torch.from_numpy(a).to(d) for a in (q, k, vals)))
+        ro, rl = oracle.attention_forward(q, k, v, elt="f32")
+        assert_parity(res.output.cpu().numpy().astype(np.float64) / scale, ro, "large scores out", tol=5e-5)
+        assert np.max(np.abs(res.cache.logsumexp.cpu().numpy() - rl)) <= 5e-5
+    for dt in ("f32", "bf16", "f16"):
+        q, k, v, _ = _inputs(1, 70, 150, 2, 48, 78, dt)
+        tq, tk, tv = (_dev(a, d, dt) for a in (q, k, v))
+        tv[0, 100, 1, 7] = -float("inf")
+        out = memory_efficient_attention(tq, tk, tv).output.float().cpu().numpy()
+        assert np.isneginf(out[0, :, 1, 7]).all(), dt
+        out[0, :, 1, 7] = 0
+        assert np.isfinite(out).all(), dt
+    # a key of -Inf (f32): its scores are -+Inf by the sign of q, probability zero or no number
+    q, k, v, _ = _inputs(1, 70, 150, 2, 48, 79, "f32")
+    k[0, 9, 0, 3] = -np.inf
+    out = memory_efficient_attention(*(torch.from_numpy(a).to(d) for a in (q, k, v))).output.cpu().numpy()
+    low = q[0, :, 0, 3] > 0
+    keep = np.arange(150) != 9
+    ro, _ = oracle.attention_forward(q[:, :, :1], k[:, keep, :1], v[:, keep, :1], elt="f32")
+    assert np.isnan(out[0, ~low, 0]).all()
+    assert_parity(out[0, low, 0], ro[0, low, 0], "the others of a key at -Inf", tol=1e-5)
