@@ -100,6 +100,10 @@ struct AttArgs {
   int64_t Sq, Sk, H;
   int causal;
   float scale;           // 1 / sqrt(Float32(D)) (attention.jl:129)
+  // dK / dV with the queries split over qsplits workgroups per key block (qper 64-query steps each):
+  // the f32 sums of split sp go to part[sp][dV, then dK][B][Sk][H][D] (dK unscaled)
+  float* part;
+  int qsplits, qper;
 };
 
 // Visibility modes, fixed at compile time so that the common case carries no branch in the
@@ -383,7 +387,7 @@ __global__ __launch_bounds__(256) void attn_corr_kernel(AttArgs a, int64_t B) {
 // Per step: S = Q K^T and dP = dY V^T (lane l: queries 16 qt + 4 g + v, key l16), P from lse,
 // dS = P (dP - correction), dV^T += dY^T P and dK^T += Q^T dS (A operands read transposed, the
 // query order {4g..4g+3, 16+4g..16+4g+3} of each 32-query block of the accumulators).
-template <int ELT, int D, int VM>
+template <int ELT, int D, int VM, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void attn_dkdv_kernel(AttArgs a) {
   using E = Elt<ELT>;
   using namespace att;
@@ -392,7 +396,8 @@ __global__ __launch_bounds__(256, 2) void attn_dkdv_kernel(AttArgs a) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int l16 = lane & 15, g = lane >> 4;
-  const int64_t b = blockIdx.z, h = blockIdx.y;
+  const int sp = SPLIT ? (int)blockIdx.z % a.qsplits : 0;
+  const int64_t b = SPLIT ? blockIdx.z / a.qsplits : blockIdx.z, h = blockIdx.y;
   const int64_t k0 = (int64_t)blockIdx.x * KB + w * KW;
   const int64_t Sq = a.Sq, Sk = a.Sk, H = a.H;
   const float sl2 = a.scale * LOG2E;
@@ -444,7 +449,11 @@ __global__ __launch_bounds__(256, 2) void attn_dkdv_kernel(AttArgs a) {
   // causal: queries before the first key of this workgroup see none of its keys
   int jbeg = 0;
   if (a.causal) jbeg = (int)(((int64_t)blockIdx.x * KB) / QT);
-  const int nsteps = (int)((Sq + QT - 1) / QT);
+  int nsteps = (int)((Sq + QT - 1) / QT);
+  if constexpr (SPLIT) {  // this workgroup's range of steps
+    jbeg = jbeg > sp * a.qper ? jbeg : sp * a.qper;
+    nsteps = nsteps < (sp + 1) * a.qper ? nsteps : (sp + 1) * a.qper;
+  }
   if (jbeg < nsteps) { stats_load(jbeg); issue(jbeg); }
   for (int j = jbeg; j < nsteps; ++j) {
     __builtin_amdgcn_s_waitcnt(0x0F70);  // this wave's copies and statistics of step j
@@ -517,6 +526,18 @@ __global__ __launch_bounds__(256, 2) void attn_dkdv_kernel(AttArgs a) {
   }
   __builtin_amdgcn_s_setprio(0);
   // dV[kj][d], dK[kj][d] = scale dK^T: lane holds d = 16 dt + 4 g + v of key kj
+  if constexpr (SPLIT) {
+    if (kj < Sk) {
+      const int64_t row = ((b * Sk + kj) * H + h) * D, plane = (int64_t)(gridDim.z / a.qsplits) * Sk * H * D;
+      float* pv = a.part + sp * 2 * plane + row;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) {
+        *reinterpret_cast<f32x4*>(pv + 16 * dt + 4 * g) = dvacc[dt];
+        *reinterpret_cast<f32x4*>(pv + plane + 16 * dt + 4 * g) = dkacc[dt];
+      }
+    }
+    return;
+  }
   if (kj < Sk) {
     uint16_t* dvrow = a.dv + ((b * Sk + kj) * H + h) * D;
     uint16_t* dkrow = a.dk + ((b * Sk + kj) * H + h) * D;
@@ -584,7 +605,7 @@ __device__ __forceinline__ u32x4 read_tr32(const uint8_t* tile, int r0, int r1, 
 // LDS: [V rows of the workgroup, 64 KB][2 stages x (Q 16 KB, dY 16 KB)][2 stages x (lse 64, corr 64) f32]
 constexpr int kDkdv32Lds = att::KB2 * 256 + 2 * 2 * att::QT2 * 256 + 2 * 2 * att::QT2 * 4;
 
-template <int ELT, int VM>
+template <int ELT, int VM, bool SPLIT>
 __global__ __launch_bounds__(512, 1) void attn_dkdv32_kernel(AttArgs a) {
   using E = Elt<ELT>;
   using namespace att;
@@ -594,7 +615,8 @@ __global__ __launch_bounds__(512, 1) void attn_dkdv32_kernel(AttArgs a) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int l32 = lane & 31, hf = lane >> 5, l16 = lane & 15, g = lane >> 4;
-  const int64_t b = blockIdx.z, h = blockIdx.y;
+  const int sp = SPLIT ? (int)blockIdx.z % a.qsplits : 0;
+  const int64_t b = SPLIT ? blockIdx.z / a.qsplits : blockIdx.z, h = blockIdx.y;
   const int64_t kb0 = (int64_t)blockIdx.x * KB2;
   const int64_t Sq = a.Sq, Sk = a.Sk, H = a.H;
   const float sl2 = a.scale * LOG2E;
@@ -667,7 +689,11 @@ __global__ __launch_bounds__(512, 1) void attn_dkdv32_kernel(AttArgs a) {
   // causal: queries before the first key of this workgroup see none of its keys
   int jbeg = 0;
   if (a.causal) jbeg = (int)(kb0 / QT2);
-  const int nsteps = (int)((Sq + QT2 - 1) / QT2);
+  int nsteps = (int)((Sq + QT2 - 1) / QT2);
+  if constexpr (SPLIT) {
+    jbeg = jbeg > sp * a.qper ? jbeg : sp * a.qper;
+    nsteps = nsteps < (sp + 1) * a.qper ? nsteps : (sp + 1) * a.qper;
+  }
   if (jbeg < nsteps) { issue_v(); stats_load(jbeg); issue(jbeg); }
   const uint8_t* sv = smem + w * KW2 * 256;
   for (int j = jbeg; j < nsteps; ++j) {
@@ -738,6 +764,21 @@ __global__ __launch_bounds__(512, 1) void attn_dkdv32_kernel(AttArgs a) {
   }
   __builtin_amdgcn_s_setprio(0);
   // dV[kj][d], dK[kj][d] = scale dK^T: element v of tile dt is d = 32 dt + 8 (v / 4) + 4 hf + v % 4
+  if constexpr (SPLIT) {
+    if (kj < Sk) {
+      const int64_t row = ((b * Sk + kj) * H + h) * D, plane = (int64_t)(gridDim.z / a.qsplits) * Sk * H * D;
+      float* pv = a.part + sp * 2 * plane + row;
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int d = 32 * dt + 8 * c + 4 * hf;
+          *reinterpret_cast<f32x4*>(pv + d) = f32x4{dvacc[dt][4 * c], dvacc[dt][4 * c + 1], dvacc[dt][4 * c + 2], dvacc[dt][4 * c + 3]};
+          *reinterpret_cast<f32x4*>(pv + plane + d) = f32x4{dkacc[dt][4 * c], dkacc[dt][4 * c + 1], dkacc[dt][4 * c + 2], dkacc[dt][4 * c + 3]};
+        }
+    }
+    return;
+  }
   if (kj < Sk) {
     uint16_t* dvrow = a.dv + ((b * Sk + kj) * H + h) * D;
     uint16_t* dkrow = a.dk + ((b * Sk + kj) * H + h) * D;
@@ -755,6 +796,24 @@ __global__ __launch_bounds__(512, 1) void attn_dkdv32_kernel(AttArgs a) {
         *reinterpret_cast<u32x2*>(dkrow + d) = pk;
       }
   }
+}
+
+// dv = rnd(sum over splits of dV's partials), dk = rnd(scale times the sum of dK's), in split order;
+// 4 elements of each per thread, n of them per tensor (a multiple of 4)
+template <int ELT>
+__global__ __launch_bounds__(256) void attn_dkdv_sum_kernel(AttArgs a, int64_t n) {
+  using E = Elt<ELT>;
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f}, k = v;
+#pragma unroll 4
+  for (int sp = 0; sp < a.qsplits; ++sp) {
+    v += *reinterpret_cast<const f32x4*>(a.part + (2 * sp) * n + i);
+    k += *reinterpret_cast<const f32x4*>(a.part + (2 * sp + 1) * n + i);
+  }
+  const float sc = a.scale;
+  *reinterpret_cast<u32x2*>(a.dv + i) = u32x2{E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
+  *reinterpret_cast<u32x2*>(a.dk + i) = u32x2{E::pack2(k[0] * sc, k[1] * sc), E::pack2(k[2] * sc, k[3] * sc)};
 }
 
 // dQ: the forward's structure. Per key tile: S^T = K Q^T and dP^T = V dY^T (A operands K and V
@@ -958,48 +1017,93 @@ static int launch_attn_fwd(const AttArgs& a, int64_t B, hipStream_t st) {
   });
 }
 
-// dK / dV at head dim 128: the 256-key workgroups of attn_dkdv32_kernel (one per CU, 256 CUs)
-// or the 64-key ones of attn_dkdv_kernel (two per CU), whichever grid needs less time counted in
-// rounds of workgroups over the CUs. A 256-key round takes 1.74 times as long as a 64-key one
-// (36.0 ms for 20 rounds against 41.4 ms for 40 at 32760 x 32760 x 40 heads), so few keys, as in
-// cross-attention on text tokens, go to the 64-key kernel. Backward at 32760 queries x 40 heads,
-// 64- / 256-key kernel: 77 keys 1.24 / 1.84 ms, 512 keys 1.78 / 2.13, 1024 keys 2.96 / 2.61,
-// 2048 keys 4.90 / 5.35, 3072 keys 6.91 / 6.20, 4096 keys 8.56 / 8.86, 8192 keys 16.7 / 15.2:
-// the rule picks the faster one at each. REELS_HIP_ATTN_DKDV_KEYS=256 or =64 fixes the choice
-// (the tests run both kernels on the same shapes).
-static bool dkdv_wide(int64_t Sk, int64_t H, int64_t B) {
+// Plan of the dK / dV pass: the 256-key workgroups of attn_dkdv32_kernel (head dim 128, one per CU,
+// 256 CUs) or the 64-key ones of attn_dkdv_kernel (two per CU), and over how many workgroups each
+// key block's queries are split. Time is counted in rounds of workgroups over the CUs: a 64-key round
+// over Sq queries takes Sq * 0.0316 us at head dim 128, a 256-key one 1.74 times that (36.0 ms for 20
+// rounds against 41.4 ms for 40 at 32760 x 32760 x 40 heads). A split costs writing and reading f32
+// partials (16 bytes per element of dK and dV and split, at 5 TB/s) and a launch, and has to pay for
+// them by a tenth. With few keys, as in cross-attention on text tokens, the unsplit grids leave CUs
+// idle: 9360 queries x 40 heads on 512 keys, dK / dV 293 us unsplit,
+// 224 us with the sum on three splits of the 256-key kernel; 32760 x 12 heads on 257 keys, forward and
+// backward, 1014 -> 414 us. Unsplit, 32760 queries x 40 heads, 64- / 256-key
+// kernel, whole backward: 77 keys 1.24 / 1.84 ms, 512 keys 1.78 / 2.13, 1024 keys 2.96 / 2.61, 2048
+// keys 4.90 / 5.35, 3072 keys 6.91 / 6.20, 4096 keys 8.56 / 8.86, 8192 keys 16.7 / 15.2.
+// The partials use dQ's buffer, which the dQ kernel fills afterwards, so they have to fit it and it
+// may overlap no other operand. REELS_HIP_ATTN_DKDV_KEYS=256 or =64 fixes the kernel (the tests run
+// both on the same shapes).
+struct DkdvPlan {
+  bool wide;
+  int splits;
+};
+static DkdvPlan dkdv_plan(int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t D, int64_t part_bytes) {
+  int only = 0;
   if (const char* e = std::getenv("REELS_HIP_ATTN_DKDV_KEYS")) {
-    if (std::strcmp(e, "256") == 0) return true;
-    if (std::strcmp(e, "64") == 0) return false;
+    if (std::strcmp(e, "256") == 0) only = 256;
+    if (std::strcmp(e, "64") == 0) only = 64;
   }
-  const int64_t nw = ceil_div(Sk, att::KB2) * H * B, n64 = ceil_div(Sk, att::KB) * H * B;
-  return ceil_div(nw, 256) * 174 < ceil_div(n64, 512) * 100;
+  const double round = Sq * 0.0316 * D / 128;
+  const int64_t one = 2 * B * Sk * H * D * 4;  // bytes of one split's partials
+  const int64_t nsteps = ceil_div(Sq, att::QT);
+  DkdvPlan best{false, 1};
+  double tbest = 1e300;
+  for (int wide = 0; wide < 2; ++wide) {
+    if (wide ? (D != 128 || only == 64) : (D == 128 && only == 256)) continue;
+    const int64_t n = ceil_div(Sk, wide ? att::KB2 : att::KB) * H * B, slots = wide ? 256 : 512;
+    double t1 = 0.0;
+    for (int s = 1; s <= 16; ++s) {
+      if (s > 1 && (s * one > part_bytes || nsteps < 8 * s)) break;
+      double t = (double)ceil_div(n * s, slots) / s * round * (wide ? 1.74 : 1.0);
+      if (s == 1) t1 = t;
+      else t += s * one * 2 / 5e6 + 5.0;
+      if (s > 1 && t > 0.9 * t1) continue;
+      if (t < tbest) { tbest = t; best = DkdvPlan{wide != 0, s}; }
+    }
+  }
+  return best;
 }
 
 template <int ELT, int D>
-static int launch_attn_bwd(const AttArgs& a, int64_t B, hipStream_t st) {
+static int launch_attn_bwd(const AttArgs& args, int64_t B, hipStream_t st) {
+  AttArgs a = args;
   {
     TraceScope _ts(st, "attn_corr_kernel");
     attn_corr_kernel<ELT, D><<<(unsigned)ceil_div(B * a.Sq * a.H, 256 / (D / 8)), 256, 0, st>>>(a, B);
   }
   if (int rc = check_launch("attn_corr_kernel")) return rc;
+  const DkdvPlan plan = dkdv_plan(B, a.Sq, a.Sk, a.H, D, dq_scratch_bytes(a, B, D, 2));
+  a.qsplits = plan.splits;
+  a.qper = (int)ceil_div(ceil_div(a.Sq, att::QT), plan.splits);
+  a.part = reinterpret_cast<float*>(a.o);
   return with_vm(a, [&](auto vm) {
     constexpr int VM = decltype(vm)::value;
-    bool wide = false;
-    if constexpr (D == 128) wide = dkdv_wide(a.Sk, a.H, B);
-    if (a.Sk > 0 && wide) {
-      if (hipError_t e = set_lds(attn_dkdv32_kernel<ELT, VM>, kDkdv32Lds))
-        return fail(REELS_HIP_EHIP, std::string("attention bwd: hipFuncSetAttribute: ") + hipGetErrorString(e));
-      const dim3 grid((unsigned)ceil_div(a.Sk, att::KB2), (unsigned)a.H, (unsigned)B);
-      { TraceScope _ts(st, "attn_dkdv32_kernel"); attn_dkdv32_kernel<ELT, VM><<<grid, 64 * att::NW2, kDkdv32Lds, st>>>(a); }
-      if (int rc = check_launch("attn_dkdv32_kernel")) return rc;
-    } else if (a.Sk > 0) {
+    auto dkdv = [&](auto split) -> int {
+      constexpr bool SPLIT = decltype(split)::value;
+      const unsigned gz = (unsigned)(B * plan.splits);
+      if constexpr (D == 128) {
+        if (plan.wide) {
+          if (hipError_t e = set_lds(attn_dkdv32_kernel<ELT, VM, SPLIT>, kDkdv32Lds))
+            return fail(REELS_HIP_EHIP, std::string("attention bwd: hipFuncSetAttribute: ") + hipGetErrorString(e));
+          const dim3 grid((unsigned)ceil_div(a.Sk, att::KB2), (unsigned)a.H, gz);
+          { TraceScope _ts(st, "attn_dkdv32_kernel"); attn_dkdv32_kernel<ELT, VM, SPLIT><<<grid, 64 * att::NW2, kDkdv32Lds, st>>>(a); }
+          return check_launch("attn_dkdv32_kernel");
+        }
+      }
       const int lds = 4 * att::QT * D * 2 + 2 * 2 * att::QT * 4;  // Q, dY rings + lse / corr
-      if (hipError_t e = set_lds(attn_dkdv_kernel<ELT, D, VM>, lds))
+      if (hipError_t e = set_lds(attn_dkdv_kernel<ELT, D, VM, SPLIT>, lds))
         return fail(REELS_HIP_EHIP, std::string("attention bwd: hipFuncSetAttribute: ") + hipGetErrorString(e));
-      const dim3 grid((unsigned)ceil_div(a.Sk, att::KB), (unsigned)a.H, (unsigned)B);
-      { TraceScope _ts(st, "attn_dkdv_kernel"); attn_dkdv_kernel<ELT, D, VM><<<grid, 256, lds, st>>>(a); }
-      if (int rc = check_launch("attn_dkdv_kernel")) return rc;
+      const dim3 grid((unsigned)ceil_div(a.Sk, att::KB), (unsigned)a.H, gz);
+      { TraceScope _ts(st, "attn_dkdv_kernel"); attn_dkdv_kernel<ELT, D, VM, SPLIT><<<grid, 256, lds, st>>>(a); }
+      return check_launch("attn_dkdv_kernel");
+    };
+    if (a.Sk > 0) {
+      if (int rc = plan.splits > 1 ? dkdv(std::true_type{}) : dkdv(std::false_type{})) return rc;
+      if (plan.splits > 1) {
+        const int64_t n = B * a.Sk * a.H * D;
+        { TraceScope _ts(st, "attn_dkdv_sum_kernel");
+          attn_dkdv_sum_kernel<ELT><<<(unsigned)ceil_div(n, 1024), 256, 0, st>>>(a, n); }
+        if (int rc = check_launch("attn_dkdv_sum_kernel")) return rc;
+      }
     }
     const int lds = 4 * att::KT * D * 2;
     if (hipError_t e = set_lds(attn_dq_kernel<ELT, D, VM>, lds))

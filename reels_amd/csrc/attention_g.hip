@@ -24,6 +24,7 @@
 // with single-element LDS reads: 610 / 1556); 2 x 1024 tokens, 16 heads x 80, bf16: 56 /
 // 152 us (460 / 1143). The f32 kernels are bound by their MFMAs and LDS fragment reads (6 MFMAs
 // per 3 fragments of 1 KiB), the 16-bit ones by the VALU work per score (exponential and split).
+#include <algorithm>
 #include <mutex>
 
 #include "attention_g.h"
@@ -492,7 +493,7 @@ __global__ __launch_bounds__(256) void attng_corr_kernel(AttgArgs a, int64_t B) 
 // S = Q K^T a lane holds queries 4 g + v of a 16-query tile for key kj, and the dV / dK products take
 // queries {4 g ..} and {16 + 4 g ..} of a 32-query block in its k slots: dV^T += dY^T P, dK^T += Q^T
 // dS with dS = P (dP - correction), dP = dY V^T.
-template <int ELT, int DP, int VM, int NW>
+template <int ELT, int DP, int VM, int NW, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, 2) void attng_dkdv_kernel(AttgArgs a, int vec) {
   using namespace attg;
   constexpr int NI = kParts<ELT>, QT = kTileRows<ELT>, NKB = DP / 32, NDT = DP / 16, WB = NW * QW;
@@ -501,7 +502,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dkdv_kernel(AttgArgs a, int 
   __shared__ __attribute__((aligned(16))) float slse[2][QT], scorr[2][QT];
   const int t = threadIdx.x, lane = t & 63, l16 = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int64_t b = blockIdx.z, h = blockIdx.y, H = a.H, Sq = a.Sq, Sk = a.Sk;
+  const int sp = SPLIT ? (int)blockIdx.z % a.qsplits : 0;
+  const int64_t b = SPLIT ? blockIdx.z / a.qsplits : blockIdx.z, h = blockIdx.y, H = a.H, Sq = a.Sq, Sk = a.Sk;
   const int D = (int)a.D;
   const int64_t kb0 = (int64_t)blockIdx.x * WB;
   const int64_t kj = kb0 + w * QW + l16;  // this lane's key
@@ -514,7 +516,12 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dkdv_kernel(AttgArgs a, int 
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) dka[dt] = dva[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   // causal: queries before the workgroup's first key see none of its keys
-  const int64_t qstart = a.causal ? kb0 / QT * QT : 0;
+  int64_t qstart = a.causal ? kb0 / QT * QT : 0, qend = Sq;
+  if constexpr (SPLIT) {  // this workgroup's range of tiles
+    const int64_t lo = (int64_t)sp * a.qper * QT, hi = lo + (int64_t)a.qper * QT;
+    qstart = qstart > lo ? qstart : lo;
+    qend = qend < hi ? qend : hi;
+  }
   float plse = 0.0f, pcorr = 0.0f;  // a tile's lse and correction on their way to LDS (threads 0 .. QT - 1)
   auto extra = [&](int stage, int64_t q0, bool load) {
     if (t >= QT) return;
@@ -589,9 +596,24 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dkdv_kernel(AttgArgs a, int 
         }
     }
   };
-  attg_stream<T>(rq, rdy, qstart, Sq, QT, D, vec, smem, w < NW / 2, step, extra);
+  attg_stream<T>(rq, rdy, qstart, qend, QT, D, vec, smem, w < NW / 2, step, extra);
   if (kj >= Sk) return;
   const int64_t ob = ((b * Sk + kj) * H + h) * D;
+  if constexpr (SPLIT) {
+    const int64_t plane = (int64_t)(gridDim.z / a.qsplits) * Sk * H * D;
+    float* p = a.part + sp * 2 * plane + ob;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int d = 16 * dt + 4 * g + v;
+        if (d < D) {
+          p[d] = dva[dt][v];
+          p[plane + d] = dka[dt][v];
+        }
+      }
+    return;
+  }
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
@@ -602,6 +624,22 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dkdv_kernel(AttgArgs a, int 
         attg_st<ELT>(a.dv, ob + d, dva[dt][v]);
       }
     }
+}
+
+// dv = sum over splits of dV's partials, dk = scale times the sum of dK's, in split order, rounded to
+// the element type (n elements per tensor)
+template <int ELT>
+__global__ __launch_bounds__(256) void attng_dkdv_sum_kernel(AttgArgs a, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  float v = 0.0f, k = 0.0f;
+#pragma unroll 4
+  for (int sp = 0; sp < a.qsplits; ++sp) {
+    v += a.part[2 * sp * n + i];
+    k += a.part[(2 * sp + 1) * n + i];
+  }
+  attg_st<ELT>(a.dv, i, v);
+  attg_st<ELT>(a.dk, i, k * a.scale);
 }
 
 // dQ: a workgroup takes 16 NW queries, 16 per wave, and streams the keys: dQ^T += K^T dS^T with
@@ -728,7 +766,8 @@ static int attg_waves(int64_t S, const AttgArgs& a, int64_t B, F&& f) {
 }
 
 template <auto KERN, int ELT, int DP, int NW>
-static int attg_launch(const char* name, int64_t S, const AttgArgs& a, int dtype, int64_t B, hipStream_t st) {
+static int attg_launch(const char* name, int64_t S, const AttgArgs& a, int dtype, int64_t B, hipStream_t st,
+                       int splits = 1) {
   constexpr int lds = 4 * GTile<ELT, kTileRows<ELT>, DP, NW * 64>::BYTES;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
@@ -737,7 +776,7 @@ static int attg_launch(const char* name, int64_t S, const AttgArgs& a, int dtype
   });
   if (attr_err != hipSuccess)
     return fail(REELS_HIP_EHIP, std::string(name) + ": hipFuncSetAttribute: " + hipGetErrorString(attr_err));
-  const dim3 grid((unsigned)ceil_div(S, NW * attg::QW), (unsigned)a.H, (unsigned)B);
+  const dim3 grid((unsigned)ceil_div(S, NW * attg::QW), (unsigned)a.H, (unsigned)(B * splits));
   { TraceScope _ts(st, name); KERN<<<grid, NW * 64, lds, st>>>(a, attg_vec(a, dtype)); }
   return check_launch(name);
 }
@@ -752,7 +791,24 @@ int attn_generic_fwd(const AttgArgs& a, int dtype, int64_t B, hipStream_t st) {
   });
 }
 
-int attn_generic_bwd(const AttgArgs& a, int dtype, int64_t B, hipStream_t st) {
+// Query splits of the dK / dV pass: with fewer key blocks than CUs, as many as fill them, while the
+// walk they shorten (about 2 us per tile at head dim 128) is worth the partials' traffic (16 bytes
+// per element of dK and dV and split at 5 TB/s) and a launch; the partials lie in dQ's buffer, as in
+// attention.hip. 2048 queries x 16 heads x 128 on 64 keys, f32:
+// 297 us unsplit, 38 + 7 us on 16 splits (forward and backward 338 -> 94 us).
+static int attg_splits(const AttgArgs& a, int64_t B, int dtype, int rows) {
+  const int64_t n = ceil_div(a.Sk, 4 * attg::QW) * a.H * B, tiles = ceil_div(a.Sq, rows);
+  const int64_t one = 2 * B * a.Sk * a.H * a.D * 4;
+  if (n <= 0 || n > 128) return 1;
+  const int64_t room = dq_scratch_bytes(a, B, a.D, dtype == REELS_HIP_F32 ? 4 : 2) / one;
+  const int64_t s = std::min<int64_t>({256 / n, room, tiles / 4, 16});
+  if (s < 2) return 1;
+  const double walk = tiles * 2.0 * a.D / 128, cost = s * one * 2 / 5e6 + 5.0;
+  return walk - walk / s > 1.5 * cost ? (int)s : 1;
+}
+
+int attn_generic_bwd(const AttgArgs& args, int dtype, int64_t B, hipStream_t st) {
+  AttgArgs a = args;
   return attg_dispatch(dtype, a.D, a, [&](auto e, auto dp, auto vm) {
     constexpr int ELT = decltype(e)::value, DP = decltype(dp)::value, VM = decltype(vm)::value;
     {
@@ -761,10 +817,24 @@ int attn_generic_bwd(const AttgArgs& a, int dtype, int64_t B, hipStream_t st) {
     }
     if (int rc = check_launch("attng_corr_kernel")) return rc;
     if (a.Sk > 0) {
-      const int rc = attg_waves(a.Sk, a, B, [&](auto nw) {
-        constexpr int NW = decltype(nw)::value;
-        return attg_launch<attng_dkdv_kernel<ELT, DP, VM, NW>, ELT, DP, NW>("attng_dkdv_kernel", a.Sk, a, dtype, B, st);
-      });
+      const int splits = attg_splits(a, B, dtype, kTileRows<ELT>);
+      int rc;
+      if (splits > 1) {  // fewer key blocks than CUs: four waves each
+        a.part = static_cast<float*>(a.o);
+        a.qsplits = splits;
+        a.qper = (int)ceil_div(ceil_div(a.Sq, kTileRows<ELT>), splits);
+        rc = attg_launch<attng_dkdv_kernel<ELT, DP, VM, 4, true>, ELT, DP, 4>("attng_dkdv_kernel", a.Sk, a, dtype, B, st, splits);
+        if (rc) return rc;
+        const int64_t n = B * a.Sk * a.H * a.D;
+        { TraceScope _ts(st, "attng_dkdv_sum_kernel");
+          attng_dkdv_sum_kernel<ELT><<<(unsigned)ceil_div(n, 256), 256, 0, st>>>(a, n); }
+        rc = check_launch("attng_dkdv_sum_kernel");
+      } else {
+        rc = attg_waves(a.Sk, a, B, [&](auto nw) {
+          constexpr int NW = decltype(nw)::value;
+          return attg_launch<attng_dkdv_kernel<ELT, DP, VM, NW, false>, ELT, DP, NW>("attng_dkdv_kernel", a.Sk, a, dtype, B, st);
+        });
+      }
       if (rc) return rc;
     }
     return attg_waves(a.Sq, a, B, [&](auto nw) {

@@ -383,3 +383,59 @@ def test_attention_generic_large_scores_and_values(dev):
     ro, _ = oracle.attention_forward(q[:, :, :1], k[:, keep, :1], v[:, keep, :1], elt="f32")
     assert np.isnan(out[0, ~low, 0]).all()
     assert_parity(out[0, low, 0], ro[0, low, 0], "the others of a key at -Inf", tol=1e-5)
+
+
+@pytest.mark.parametrize("keys", ["256", "64"])
+@pytest.mark.parametrize("B,Sq,Sk,H,D,causal,masked,dt", [
+    (1, 2100, 77, 2, 128, False, False, "bf16"),   # ragged last step and last split
+    (2, 1500, 130, 3, 64, False, True, "f16"),
+    (1, 1030, 65, 1, 128, True, False, "bf16"),    # causal: the later splits see every key
+    (1, 2100, 70, 2, 96, False, True, "f32"),      # the generic kernels
+    (2, 1100, 33, 3, 40, True, False, "bf16"),
+    (1, 1500, 65, 1, 128, False, False, "f32"),
+])
+def test_attention_split_queries(dev, monkeypatch, keys, B, Sq, Sk, H, D, causal, masked, dt):
+    """Few keys and many queries: the dK / dV pass splits the queries over workgroups (both kernels at
+    head dim 128) and adds the partials up in order."""
+    if keys == "64" and (D != 128 or dt == "f32"):
+        pytest.skip("one dK / dV kernel at this head dim and type")
+    monkeypatch.setenv("REELS_HIP_ATTN_DKDV_KEYS", keys)
+    mask = None
+    if masked:
+        mask = np.random.default_rng(300 + Sq).random((Sq, Sk)) < 0.7
+        mask[:, 0] = True
+    out, lse, ro, rl, grads = _run(B, Sq, Sk, H, D, causal, mask, dt, seed=Sq + Sk)
+    what = f"split {B}x{Sq}x{Sk}x{H}x{D} {dt}"
+    if dt == "f32":
+        for a, r in zip(*grads):
+            assert_parity(a, r, what, tol=1e-5)
+    else:
+        _check_bwd(grads, what)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+def test_attention_backward_writing_dq_over_q(dev, dt):
+    """dQ's buffer holds the split partials only where it overlaps no operand: written over q (each
+    workgroup reads its own queries before it writes them), every gradient stays right."""
+    import ctypes
+    import torch
+    from reels_amd import _lib, memory_efficient_attention
+    from reels_amd.attention import _DT
+    B, Sq, Sk, H, D = 1, 2100, 77, 2, 128
+    print(f"[case] attention backward, dq over q, {dt}", flush=True)
+    q, k, v, dy = _inputs(B, Sq, Sk, H, D, 41, dt)
+    tq, tk, tv, tdy = (_dev(a, dev, dt) for a in (q, k, v, dy))
+    res = memory_efficient_attention(tq, tk, tv)
+    L = _lib.lib()
+    n = L.reels_hip_attention_workspace_bytes(B, Sq, H)
+    ws = torch.empty((n,), dtype=torch.uint8, device=dev)
+    dk, dv = torch.empty_like(tk), torch.empty_like(tv)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    st = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    _lib.check("reels_hip_attention_bwd", L.reels_hip_attention_bwd(
+        p(tq), p(tk), p(tv), p(res.output), p(tdy), p(res.cache.logsumexp), None, 0, B, Sq, Sk, H, D,
+        _DT[tq.dtype], p(tq), p(dk), p(dv), p(ws), ctypes.c_size_t(n), st))
+    torch.cuda.synchronize()
+    ref = oracle.attention_backward(q, k, v, dy, elt=dt)
+    for t, r in zip((tq, dk, dv), ref):
+        assert_parity(_vals(_bits(t), dt), r, f"dq over q {dt}", tol=1e-5 if dt == "f32" else GTOL)
