@@ -21,6 +21,7 @@ struct AttgArgs {
   int64_t Sq, Sk, H, D;
   int causal;
   float scale;       // 1 / sqrt(Float32(D)) (attention.jl:129)
+  float ch, cl;      // scale log2(e) = ch + cl, ch rounded down so that cl > 0 (set by the launchers)
   // dK / dV with the queries split over qsplits workgroups per key block (qper query tiles each): the
   // f32 sums of split sp go to part[sp][dV, then dK][B][Sk][H][D] (dK unscaled)
   float* part;

@@ -25,6 +25,7 @@
 // 152 us (460 / 1143). The f32 kernels are bound by their MFMAs and LDS fragment reads (6 MFMAs
 // per 3 fragments of 1 KiB), the 16-bit ones by the VALU work per score (exponential and split).
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "attention_g.h"
@@ -102,28 +103,40 @@ __device__ __forceinline__ void split8(const float* x, u32x4 (&o)[3]) {
 }
 // the same for input elements: the first part by truncation (no finite value overflows); NaN stays
 // NaN. Of three parts an Inf is all in the last, which is only multiplied by first parts (nonzero
-// unless the element is); of two it is in the first.
+// unless the element is); of two it is in the first. That selection runs only where some lane of the
+// wave meets an Inf or NaN.
 template <int NI>
 __device__ __forceinline__ void split8_in(const float* x, u32x4 (&o)[NI]) {
+  uint32_t top = 0u;  // largest magnitude pattern of the 8
 #pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    float r[2];
-    uint32_t h[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const float v = x[2 * d + e];
-      const bool inf = __builtin_isinf(v);
-      h[e] = NI > 2 && inf ? 0u : __float_as_uint(v) & 0xffff0000u;
-      r[e] = NI > 2 || !inf ? v - __uint_as_float(h[e]) : 0.0f;
-    }
-    o[0][d] = __builtin_amdgcn_perm(h[1], h[0], 0x07060302u);
-    if constexpr (NI == 2) o[1][d] = pk_bf16(r[0], r[1]);
-    if constexpr (NI > 2) {
-      const float m0 = __builtin_isinf(r[0]) ? 0.0f : r[0], m1 = __builtin_isinf(r[1]) ? 0.0f : r[1];
-      o[1][d] = pk_bf16(m0, m1);
-      o[2][d] = pk_bf16(r[0] - bf16_lo(o[1][d]), r[1] - bf16_hi(o[1][d]));
-    }
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t u = __float_as_uint(x[e]) & 0x7fffffffu;
+    top = u > top ? u : top;
   }
+  auto parts = [&](auto special) {
+    constexpr bool SP = decltype(special)::value;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      float r[2];
+      uint32_t h[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float v = x[2 * d + e];
+        const bool inf = SP && __builtin_isinf(v);
+        h[e] = NI > 2 && inf ? 0u : __float_as_uint(v) & 0xffff0000u;
+        r[e] = NI > 2 || !inf ? v - __uint_as_float(h[e]) : 0.0f;
+      }
+      o[0][d] = __builtin_amdgcn_perm(h[1], h[0], 0x07060302u);
+      if constexpr (NI == 2) o[1][d] = pk_bf16(r[0], r[1]);
+      if constexpr (NI > 2) {
+        const float m0 = SP && __builtin_isinf(r[0]) ? 0.0f : r[0], m1 = SP && __builtin_isinf(r[1]) ? 0.0f : r[1];
+        o[1][d] = pk_bf16(m0, m1);
+        o[2][d] = pk_bf16(r[0] - bf16_lo(o[1][d]), r[1] - bf16_hi(o[1][d]));
+      }
+    }
+  };
+  if (__builtin_amdgcn_ballot_w64(top >= 0x7f800000u)) parts(std::true_type{});
+  else parts(std::false_type{});
 }
 
 // 8 consecutive elements of a row: raw from memory, then as bf16 parts. Buffer loads, so rows and
@@ -249,13 +262,14 @@ __device__ __forceinline__ void mfma_parts2(const u32x4 (&a)[NA], const u32x4 (&
   hi = mfma_bf(a[0], b[0], hi);
 }
 
-// exp(x) for x <= about 90, to about an ulp: 2^t with t = x log2(e) rounded, corrected by what the
-// rounding left over (results below the f32 normal range are zero)
-__device__ __forceinline__ float exp_f(float x) {
-  const float t = x * 1.44269504f;
-  const float e = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269504f, -t));
-  const float y = __builtin_amdgcn_exp2f(t);
-  return fmaf(y * e, 0.693147181f, y);
+// Probabilities are powers of two: 2^(s ch + s cl - off) of a raw score s, scale log2(e) in two parts
+// (one f32 constant would be off by up to 2^-24 of the exponent for every score alike). cl > 0, so a
+// score of -Inf stays -Inf. v_exp_f32 is within an ulp (results below the f32 normal range are zero).
+__device__ __forceinline__ float exp2_f(float x) { return __builtin_amdgcn_exp2f(x); }
+// lse log2(e) in two parts, for the exponents of the backward
+__device__ __forceinline__ float lse2_hi(float lse) { return lse * 1.44269502f; }
+__device__ __forceinline__ float lse2_lo(float lse, float hi) {
+  return fmaf(lse, 1.92596299e-8f, fmaf(lse, 1.44269502f, -hi));
 }
 
 // own rows of a wave as MFMA operands: row of lane l16, parts x 32-element blocks
@@ -336,14 +350,16 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_fwd_kernel(AttgArgs a, int v
   f32x4 oacc[NDT];  // O^T: lane holds d = 16 dt + 4 g + v of query qi
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) oacc[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  float m = -INFINITY, l = 0.0f;  // l: this lane's part
+  // the running maximum of the raw scores, the exponents' offset, this lane's part of the sum
+  float m = -INFINITY, off = 0.0f, l = 0.0f;
   // keys past the last one any query of this workgroup can see (causal) need no tile
   const int64_t kvis = (int64_t)(blockIdx.x + 1) * WB;
   const int64_t kend = a.causal && kvis < Sk ? kvis : Sk;
   // FIRST: the pass over the keys; else the second one (below), which keeps m and adds the first
   // parts of P only
-  auto step = [&](const uint8_t* sk, const uint8_t* sv, int64_t k0, auto first) {
-    constexpr bool FIRST = decltype(first)::value;
+  // FULL: every key of the tile exists and is visible (no mask, not causal)
+  auto step = [&](const uint8_t* sk, const uint8_t* sv, int64_t k0, auto first, auto full) {
+    constexpr bool FIRST = decltype(first)::value, FULL = decltype(full)::value;
     uint32_t mk[KT / 16];
 #pragma unroll
     for (int u = 0; u < KT / 16; ++u) mk[u] = VM == 2 ? mask_keys(a, qi, k0 + 16 * u + 4 * g) : 0u;
@@ -370,7 +386,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_fwd_kernel(AttgArgs a, int v
         for (int v = 0; v < 4; ++v) {
           const int64_t kj = k0 + 16 * (u0 + u) + 4 * g + v;
           const float s = NI > 1 ? sh[u][v] + sl[u][v] : sh[u][v];
-          sc[u0 + u][v] = attg_visible<VM>(a, qi, kj, (mk[u0 + u] >> (8 * v)) & 0xffu) ? s * a.scale : -INFINITY;
+          sc[u0 + u][v] = FULL || attg_visible<VM>(a, qi, kj, (mk[u0 + u] >> (8 * v)) & 0xffu) ? s : -INFINITY;
           bmax = fmaxf(bmax, sc[u0 + u][v]);
         }
     }
@@ -378,8 +394,10 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_fwd_kernel(AttgArgs a, int v
     // exp(-Inf - -Inf) = NaN there would only reach queries that see no key at all
     if (FIRST && __builtin_amdgcn_ballot_w64(bmax > m)) {
       const float nmax = fmaxf(m, wave_max16(bmax));
-      const float ps = nmax == -INFINITY ? 1.0f : exp_f(m == -INFINITY ? -1e30f : m - nmax);
+      const float noff = nmax * a.ch;  // the exponents' offset: about the new maximum's exponent
+      const float ps = nmax == -INFINITY || m == -INFINITY ? (nmax == -INFINITY ? 1.0f : 0.0f) : exp2_f(off - noff);
       m = nmax;
+      off = noff;
       l *= ps;
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt)
@@ -392,7 +410,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_fwd_kernel(AttgArgs a, int v
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float x = sc[2 * kb + (e >> 2)][e & 3];
-        p[e] = x == -INFINITY ? 0.0f : exp_f(x - m);
+        const float pe = exp2_f(fmaf(x, a.ch, fmaf(x, a.cl, -off)));
+        p[e] = !FULL && x == -INFINITY ? 0.0f : pe;
         if (FIRST) l += p[e];
       }
       u32x4 pb[3];
@@ -420,7 +439,10 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_fwd_kernel(AttgArgs a, int v
   };
   const auto none_extra = [](int, int64_t, bool) {};
   attg_stream<T>(rk, rv, 0, kend, KT, D, vec, smem, w < NW / 2,
-                 [&](const uint8_t* sk, const uint8_t* sv, int, int64_t k0) { step(sk, sv, k0, std::true_type{}); },
+                 [&](const uint8_t* sk, const uint8_t* sv, int, int64_t k0) {
+                   if (VM == 0 && k0 + KT <= Sk) step(sk, sv, k0, std::true_type{}, std::true_type{});
+                   else step(sk, sv, k0, std::true_type{}, std::false_type{});
+                 },
                  none_extra);
   // An infinite value times a low part of P (zero or negative) is NaN where P times it is that
   // infinity. If any output of the workgroup is NaN, its keys are walked again with P rounded to its
@@ -438,7 +460,10 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_fwd_kernel(AttgArgs a, int v
       oacc[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
     attg_stream<T>(rk, rv, 0, kend, KT, D, vec, smem, w < NW / 2,
-                   [&](const uint8_t* sk, const uint8_t* sv, int, int64_t k0) { step(sk, sv, k0, std::false_type{}); },
+                   [&](const uint8_t* sk, const uint8_t* sv, int, int64_t k0) {
+                   if (VM == 0 && k0 + KT <= Sk) step(sk, sv, k0, std::false_type{}, std::true_type{});
+                   else step(sk, sv, k0, std::false_type{}, std::false_type{});
+                 },
                    none_extra);
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
@@ -448,7 +473,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_fwd_kernel(AttgArgs a, int v
   }
   l = wave_sum16(l);
   if (qi >= Sq) return;
-  // out = acc / l, lse = m + log(l); a query without a visible key: NaN output, lse NaN (-Inf
+  // out = acc / l, lse = off ln(2) + log(l); a query without a visible key: NaN output, lse NaN (-Inf
   // without keys: the reference's -Inf + log(0))
   const bool none = m == -INFINITY;
   const int64_t ob = ((b * Sq + qi) * H + h) * D;
@@ -459,7 +484,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_fwd_kernel(AttgArgs a, int v
       const int d = 16 * dt + 4 * g + v;
       if (d < D) attg_st<ELT>(a.o, ob + d, none ? NAN : oacc[dt][v] / l);
     }
-  if (g == 0 && a.lse_out) a.lse_out[(b * H + h) * Sq + qi] = none ? (Sk == 0 ? -INFINITY : NAN) : m + logf(l);
+  if (g == 0 && a.lse_out) a.lse_out[(b * H + h) * Sq + qi] = none ? (Sk == 0 ? -INFINITY : NAN) : fmaf(off, 0.693147182f, fmaf(off, -1.90465421e-9f, logf(l)));
 }
 
 // correction[q] = sum(dy .* out) over the head dim (attention.jl:190), in f32: 16 lanes per row,
@@ -499,7 +524,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dkdv_kernel(AttgArgs a, int 
   constexpr int NI = kParts<ELT>, QT = kTileRows<ELT>, NKB = DP / 32, NDT = DP / 16, WB = NW * QW;
   using T = GTile<ELT, QT, DP, NW * 64>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  __shared__ __attribute__((aligned(16))) float slse[2][QT], scorr[2][QT];
+  __shared__ __attribute__((aligned(16))) float slse[2][2][QT], scorr[2][QT];  // lse log2(e): high, low part
   const int t = threadIdx.x, lane = t & 63, l16 = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int sp = SPLIT ? (int)blockIdx.z % a.qsplits : 0;
@@ -530,7 +555,9 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dkdv_kernel(AttgArgs a, int 
       plse = in ? a.lse[(b * H + h) * Sq + q0 + t] : 0.0f;
       pcorr = in ? a.corr[(b * H + h) * Sq + q0 + t] : 0.0f;
     } else {
-      slse[stage][t] = plse;
+      const float hi = lse2_hi(plse);
+      slse[stage][0][t] = hi;
+      slse[stage][1][t] = lse2_lo(plse, hi);
       scorr[stage][t] = pcorr;
     }
   };
@@ -562,9 +589,11 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dkdv_kernel(AttgArgs a, int 
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int qq = qb + 16 * u + 4 * g + v;
-          const bool vis = attg_visible<VM>(a, q0 + qq, kj, (mk[qb / 16 + u] >> (8 * v)) & 0xffu);
+          // without a mask nothing needs hiding: a query past Sq has zero Q and dY rows and zero
+          // statistics (P = 1, dS = 0: both products add zeros), a key past Sk is not stored
+          const bool vis = VM == 0 || attg_visible<VM>(a, q0 + qq, kj, (mk[qb / 16 + u] >> (8 * v)) & 0xffu);
           const float s = NI > 1 ? sh[v] + sl[v] : sh[v], dp = NI > 1 ? dh[v] + dl[v] : dh[v];
-          const float pv = exp_f(s * a.scale - slse[stage][qq]);
+          const float pv = exp2_f(fmaf(s, a.ch, -slse[stage][0][qq]) + fmaf(s, a.cl, -slse[stage][1][qq]));
           p[4 * u + v] = vis ? pv : 0.0f;
           ds[4 * u + v] = vis ? pv * (dp - scorr[stage][qq]) : 0.0f;
         }
@@ -661,6 +690,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dq_kernel(AttgArgs a, int ve
   attg_frags<ELT, DP>(rq, qi, g, D, vec, qf);
   attg_frags<ELT, DP>(rdy, qi, g, D, vec, df);
   const float lse = qi < Sq ? a.lse[(b * H + h) * Sq + qi] : 0.0f;
+  const float lh = lse2_hi(lse), ll = lse2_lo(lse, lh);
   const float corr = qi < Sq ? a.corr[(b * H + h) * Sq + qi] : 0.0f;
   f32x4 dqa[NDT];
 #pragma unroll
@@ -668,7 +698,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dq_kernel(AttgArgs a, int ve
   // causal: keys past the workgroup's last query are seen by none of its queries
   const int64_t kvis = (int64_t)(blockIdx.x + 1) * WB;
   const int64_t kend = a.causal && kvis < Sk ? kvis : Sk;
-  auto step = [&](const uint8_t* sk, const uint8_t* sv, int, int64_t k0) {
+  auto step = [&](const uint8_t* sk, const uint8_t* sv, int64_t k0, auto full) {
+    constexpr bool FULL = decltype(full)::value;
     uint32_t mk[KT / 16];
 #pragma unroll
     for (int u = 0; u < KT / 16; ++u) mk[u] = VM == 2 ? mask_keys(a, qi, k0 + 16 * u + 4 * g) : 0u;
@@ -693,7 +724,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dq_kernel(AttgArgs a, int ve
         for (int v = 0; v < 4; ++v) {
           const int64_t kk = k0 + kb2 + 16 * u + 4 * g + v;
           const float s = NI > 1 ? sh[v] + sl[v] : sh[v], dp = NI > 1 ? dh[v] + dl[v] : dh[v];
-          ds[4 * u + v] = attg_visible<VM>(a, qi, kk, (mk[kb2 / 16 + u] >> (8 * v)) & 0xffu) ? exp_f(s * a.scale - lse) * (dp - corr) : 0.0f;
+          const float x = exp2_f(fmaf(s, a.ch, -lh) + fmaf(s, a.cl, -ll)) * (dp - corr);
+          ds[4 * u + v] = FULL || attg_visible<VM>(a, qi, kk, (mk[kb2 / 16 + u] >> (8 * v)) & 0xffu) ? x : 0.0f;
         }
       }
       u32x4 db[3];
@@ -717,7 +749,12 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dq_kernel(AttgArgs a, int ve
       }
     }
   };
-  attg_stream<T>(rk, rv, 0, kend, KT, D, vec, smem, w < NW / 2, step, [](int, int64_t, bool) {});
+  attg_stream<T>(rk, rv, 0, kend, KT, D, vec, smem, w < NW / 2,
+                 [&](const uint8_t* sk, const uint8_t* sv, int, int64_t k0) {
+                   if (VM == 0 && k0 + KT <= Sk) step(sk, sv, k0, std::true_type{});
+                   else step(sk, sv, k0, std::false_type{});
+                 },
+                 [](int, int64_t, bool) {});
   if (qi >= Sq) return;
   const int64_t ob = ((b * Sq + qi) * H + h) * D;
 #pragma unroll
@@ -781,7 +818,17 @@ static int attg_launch(const char* name, int64_t S, const AttgArgs& a, int dtype
   return check_launch(name);
 }
 
-int attn_generic_fwd(const AttgArgs& a, int dtype, int64_t B, hipStream_t st) {
+// scale log2(e) in two f32 parts, the first rounded down
+static void set_exponent(AttgArgs& a) {
+  const double c = (double)a.scale * 1.4426950408889634;
+  a.ch = (float)c;
+  if ((double)a.ch >= c) a.ch = nextafterf(a.ch, 0.0f);
+  a.cl = (float)(c - (double)a.ch);
+}
+
+int attn_generic_fwd(const AttgArgs& args, int dtype, int64_t B, hipStream_t st) {
+  AttgArgs a = args;
+  set_exponent(a);
   return attg_dispatch(dtype, a.D, a, [&](auto e, auto dp, auto vm) {
     constexpr int ELT = decltype(e)::value, DP = decltype(dp)::value, VM = decltype(vm)::value;
     return attg_waves(a.Sq, a, B, [&](auto nw) {
@@ -809,6 +856,7 @@ static int attg_splits(const AttgArgs& a, int64_t B, int dtype, int rows) {
 
 int attn_generic_bwd(const AttgArgs& args, int dtype, int64_t B, hipStream_t st) {
   AttgArgs a = args;
+  set_exponent(a);
   return attg_dispatch(dtype, a.D, a, [&](auto e, auto dp, auto vm) {
     constexpr int ELT = decltype(e)::value, DP = decltype(dp)::value, VM = decltype(vm)::value;
     {
