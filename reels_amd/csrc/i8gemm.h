@@ -96,15 +96,18 @@ struct SkinnyPlan {
 bool skinny_supported(int64_t M, int64_t K, int64_t N, int rp);
 // mode 0: the forward (Kred = K, Ncols = N); 1: dX (Kred = N, Ncols = K)
 SkinnyPlan skinny_plan(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode);
-// workspace of one launch: the split partials and l [M][rp]
-size_t skinny_ws_bytes(const SkinnyPlan& p, int64_t M, int64_t Ncols, int rp);
+// tokens per launch for the token counts skinny_supported leaves to the GEMM (0: the GEMM)
+int64_t skinny_chunk(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode);
+// workspace of launches over chunks of M tokens: the split partials and l [chunk][rp]
+size_t skinny_ws_bytes(int64_t chunk, int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode);
+// One launch per chunk tokens (a multiple of 16 unless it is M):
 // out = rnd(colscale * act W + c l R + bias) with l = rnd(act L) (h or u), written to lsave
 // ([M][ld_lsave], lsave_cols columns, zeros past r) when not NULL; R(o, j) = R[j][o] (mode 0,
 // row stride ldr) or R[o][j] (mode 1, rows of ldr >= rp elements, zeros past r). adapter_only: l
 // alone, from the same blocks and split order as a full launch (so a recomputed h equals the
 // forward's bit for bit). The launch's counters live in ws (cleared by a kernel before it), so
 // launches with their own workspaces may run concurrently.
-int launch_skinny(int mode, int elt, const SkinnyPlan& p, const uint16_t* act, const int8_t* q,
+int launch_skinny(int mode, int elt, int64_t chunk, const uint16_t* act, const int8_t* q,
                   int64_t ldq, const float* s, const uint16_t* lw, void* ws, int64_t M,
                   int64_t Kred, int64_t Ncols, int r, int rp, const float* colscale,
                   const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,

@@ -893,12 +893,14 @@ static Split split_for(int64_t M, int64_t Od) {
 struct Plan {
   bool fast;
   bool deq;     // fast and K, N multiples of 64: dequantized weight + bf16 GEMM
-  bool skinny;  // few tokens: the int8 codes streamed into registers (skinny.hip), both directions
+  bool few;     // few tokens: the int8 codes streamed into registers (skinny.hip), both directions
+  // tokens per launch of that path in the forward (reduction K) and dX (reduction N): M when few,
+  // chunks of M or 0 (the GEMMs) beyond
+  int64_t cf, cb;
   int rp;       // row stride of the h/u panels and padded adapter operands: round_up(r, 16)
   bool padded;  // rp != r: h, h_save and A go through padded copies in the workspace
   Split sa;     // dA: columns of x (K)
   Split sb;     // dB: columns of dy (N)
-  SkinnyPlan skf, skb;  // the few-token forward (reduction K) and dX (reduction N)
   int ksf, ksb;  // reduction splits of the forward and dX GEMMs (1 = none)
   bool i8f;      // deq shapes with a split forward: the forward multiplies the int8 codes (no
                  // weight copy; faster there), dX keeps the dequantized weight (faster there)
@@ -926,6 +928,7 @@ static void noalloc_plan(Plan& p) {
   p.deq = false;
   p.i8f = false;
   p.ksf = p.ksb = 1;
+  if (!p.few) p.cf = p.cb = 0;  // the int8 GEMM, as its scratch bound was made for
 }
 
 static Plan make_plan(int64_t M, int64_t K, int64_t N, int64_t r, bool ptrs_aligned) {
@@ -937,15 +940,14 @@ static Plan make_plan(int64_t M, int64_t K, int64_t N, int64_t r, bool ptrs_alig
   p.deq = p.fast && bfgemm_supported(M, N, K) && bfgemm_supported(M, K, N);
   p.rp = (int)((r + 15) / 16 * 16);
   p.padded = p.fast && p.rp != r;
-  p.skinny = p.fast && skinny_supported(M, K, N, p.rp);
-  if (p.skinny) {
-    p.skf = skinny_plan(M, K, N, r > 0 ? p.rp : 0, 0);
-    p.skb = skinny_plan(M, N, K, r > 0 ? p.rp : 0, 1);
-  }
+  p.few = p.fast && skinny_supported(M, K, N, p.rp);
+  const int rpl = r > 0 ? p.rp : 0;
+  p.cf = p.few ? M : (p.deq ? skinny_chunk(M, K, N, rpl, 0) : 0);
+  p.cb = p.few ? M : (p.deq ? skinny_chunk(M, N, K, rpl, 1) : 0);
   p.sa = split_for(M, K);
   p.sb = split_for(M, N);
-  p.ksf = p.fast && !p.skinny ? bfgemm_splits(M, N, K) : 1;
-  p.ksb = p.fast && !p.skinny ? bfgemm_splits(M, K, N) : 1;
+  p.ksf = p.fast && p.cf == 0 ? bfgemm_splits(M, N, K) : 1;
+  p.ksb = p.fast && p.cb == 0 ? bfgemm_splits(M, K, N) : 1;
   p.i8f = p.deq && p.ksf > 1;
   return p;
 }
@@ -961,20 +963,26 @@ static WsLayout ws_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which,
   auto take = [&](size_t bytes) { size_t o = off; off = align_up(off + bytes, 256); return o; };
   const size_t rp = (size_t)p.rp;
   const int rpl = r > 0 ? p.rp : 0;
-  if (p.skinny) {
+  if (which == REELS_HIP_WS_FWD ? p.cf > 0 : p.cf > 0 || p.cb > 0) {
     // few tokens: the f32 split partials instead of a dequantized weight; A zero-padded to rp for
     // the forward's adapter blocks; u (and h for the dB pass) as in the other plans
     if (which == REELS_HIP_WS_FWD) {
       w.ap = take(p.padded && r > 0 ? (size_t)K * rp * 2 : 0);
-      w.pa = take(skinny_ws_bytes(p.skf, M, N, rpl));
+      w.pa = take(skinny_ws_bytes(p.cf, M, K, N, rpl, 0));
     } else {
       w.h = take((size_t)M * rp * 2);
       w.at = take(r > 0 ? (size_t)K * rp * 2 : 0);  // A^T, or A padded to rp for recomputing h
       w.ap = take(p.padded && r > 0 ? (size_t)K * rp * 2 : 0);  // A [K][rp] for the dX epilogue
       w.u = take((size_t)M * rp * 2);
-      // dX partials, or the forward's when h is recomputed
-      const size_t pb = skinny_ws_bytes(p.skb, M, K, rpl), pf = skinny_ws_bytes(p.skf, M, N, rpl);
+      // dX's partials or its weight copy; the forward's partials when h is recomputed after it
+      const size_t pb = p.cb > 0 ? skinny_ws_bytes(p.cb, M, N, K, rpl, 1) : (size_t)N * K * 2;
+      const size_t pf = p.cf > 0 ? skinny_ws_bytes(p.cf, M, K, N, rpl, 0) : 0;
       w.wd = take(pb > pf ? pb : pf);
+      if (!p.few && r > 0) {  // rank projections of the direction that runs on the GEMM
+        const int rs = std::max(rowproj_splits(M, K, p.rp), rowproj_splits(M, N, p.rp));
+        w.rq = take(rs > 1 ? (size_t)rs * M * rp * 4 : 0);
+      }
+      w.kp = take(p.ksb > 1 ? (size_t)p.ksb * M * K * 4 : 0);
       w.pa = take(r > 0 ? (size_t)p.sa.splits * K * rp * 4 : 0);
       w.pb = take(r > 0 ? (size_t)p.sb.splits * N * rp * 4 : 0);
       w.pbias = take(colsum_partial_bytes(M, N));
@@ -1006,12 +1014,20 @@ static WsLayout ws_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which,
   return w;
 }
 
+// Padded width: multiples of 64, or of 128 at the token counts whose few-token path then takes its
+// row-wave tiles in both directions (their reduction steps are 128 deep): dX of 777 tokens, 1000 ->
+// 3000, on split tiles at 3008 outputs and on row-wave tiles at 3072: 88 -> 65 us forward and backward.
+static int64_t pad_width(int64_t M, int64_t d) {
+  const int64_t to = M <= kSkinnySmallWeightTokens ? 128 : 64;
+  return (d + to - 1) / to * to;
+}
+
 // Widths that are no multiples of 64: the call runs on copies zero-padded to the next multiples
 // (Kp, Np) in the workspace, so it meets the same kernels as any other shape, and the outputs'
 // valid parts are copied out. The forward then multiplies the int8 codes (s on the f32 sum), as
 // the direct kernels do for these widths; dX multiplies the dequantized weight. The copies cost a
-// read and a write of each operand, four launches of 5-9 us in 88 us forward and backward for 777
-// tokens, 1000 -> 3000; the one-output-per-thread kernels took 11.0 ms there, and widths that are
+// read and a write of each operand, four launches of 5-9 us in 65 us forward and backward for 777
+// tokens, 1000 -> 3000 (rank 8); the one-output-per-thread kernels took 11.0 ms there, and widths that are
 // multiples of 16 ran unsplit 256 x 256 tiles (1000 tokens, 528 -> 2064: 236 against 89 us). dX's
 // error against 64 bits stays: 2.341e-3 to 2.349e-3 with rnd(dy s) times the codes, 2.343e-3 to
 // 2.347e-3 with rnd(q s), over seven shapes.
@@ -1021,7 +1037,7 @@ static bool pad_shape(int64_t M, int64_t K, int64_t N) {
   // 100 -> 100 forward 14 against 21 us; 64 tokens forward and backward 60 us either way; 256 tokens
   // 91 against 63, 16 tokens 200 -> 200 78 against 65, 300 -> 100 forward 26 against 21)
   if (M <= 64 && K <= 128 && N <= 128) return false;
-  const int64_t Kp = (K + 63) / 64 * 64, Np = (N + 63) / 64 * 64, most = (int64_t)1 << 31;
+  const int64_t Kp = pad_width(M, K), Np = pad_width(M, N), most = (int64_t)1 << 31;
   return Kp < ((int64_t)1 << 22) && Np < ((int64_t)1 << 22) && Kp * Np * 2 < most &&
          M * std::max(Kp, Np) / 8 < most;  // the copies count their 16-byte pieces in 32 bits
 }
@@ -1034,8 +1050,8 @@ struct PadLayout {
 
 static PadLayout pad_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which) {
   PadLayout w{};
-  w.Kp = (K + 63) / 64 * 64;
-  w.Np = (N + 63) / 64 * 64;
+  w.Kp = pad_width(M, K);
+  w.Np = pad_width(M, N);
   w.rp = (r + 15) / 16 * 16;
   r = w.rp;
   size_t off = 0;
@@ -1057,7 +1073,7 @@ static PadLayout pad_layout(int64_t M, int64_t K, int64_t N, int64_t r, int whic
     w.db = take((size_t)w.Np * 4);
   }
   w.p = make_plan(M, w.Kp, w.Np, r, true);
-  if (which == REELS_HIP_WS_FWD && !w.p.skinny) w.p.i8f = w.p.deq;
+  if (which == REELS_HIP_WS_FWD && w.p.cf == 0) w.p.i8f = w.p.deq;
   w.inner = off;
   w.total = off + ws_layout(M, w.Kp, w.Np, r, which, w.p).total;
   return w;
@@ -1360,7 +1376,9 @@ extern "C" size_t reels_hip_i8lora_workspace_bytes(int64_t M, int64_t K, int64_t
     noalloc_plan(p);
     which = REELS_HIP_WS_FWD;
   }
-  return ws_layout(M, K, N, r, which, p).total;
+  // unaligned buffers take the generic layout
+  return std::max(ws_layout(M, K, N, r, which, p).total,
+                  ws_layout(M, K, N, r, which, make_plan(M, K, N, r, false)).total);
 }
 
 static bool all_aligned(std::initializer_list<const void*> ps) {
@@ -1444,7 +1462,7 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
                   (bias == nullptr || (reinterpret_cast<uintptr_t>(bias) & 7u) == 0);
   Plan p = make_plan(M, K, N, r, al);
   if (noalloc) noalloc_plan(p);
-  if (codes && !p.skinny) p.i8f = p.deq;  // the forward of a padded call multiplies the codes
+  if (codes && p.cf == 0) p.i8f = p.deq;  // the forward of a padded call multiplies the codes
   WsLayout w = ws_layout(M, K, N, r, REELS_HIP_WS_FWD, p);
   if (noalloc) {
     if (w.total > kScratchBytes)
@@ -1463,7 +1481,7 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   const uint16_t* xb = static_cast<const uint16_t*>(x);
   int rc;
-  if (p.skinny) {
+  if (p.cf > 0) {
     // few tokens: y and h from the int8 codes in one launch
     const uint16_t* Ap = static_cast<const uint16_t*>(A);
     if (r > 0 && p.padded) {
@@ -1471,7 +1489,7 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
       if ((rc = launch_pad_cols(Ap, K, (int)r, r, ap, p.rp, p.rp, st))) return rc;
       Ap = ap;
     }
-    return launch_skinny(0, elt, p.skf, xb, q, K, nullptr, r > 0 ? Ap : nullptr,
+    return launch_skinny(0, elt, p.cf, xb, q, K, nullptr, r > 0 ? Ap : nullptr,
                          reinterpret_cast<float*>(ws + w.pa), M, K, N, (int)r, p.rp, scales,
                          static_cast<const uint16_t*>(B), N, static_cast<const uint16_t*>(bias),
                          lora_scale, static_cast<uint16_t*>(y), static_cast<uint16_t*>(h_save), r,
@@ -1622,17 +1640,18 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
     if ((rc = launch_pad_cols(hh, M, (int)r, r, hw, p.rp, p.rp, st))) return rc;
     hh = hw;
   }
-  if (p.skinny && dx) {
+  if (p.cb > 0 && dx) {
     // few tokens: dx and u = rnd(dy B^T) from one launch over the int8 codes (u lands in the
     // workspace for the dA pass)
-    if ((rc = launch_skinny(1, elt, p.skb, dyb, q, K, scales, r > 0 ? Bb : nullptr,
+    if ((rc = launch_skinny(1, elt, p.cb, dyb, q, K, scales, r > 0 ? Bb : nullptr,
                             reinterpret_cast<float*>(ws + w.wd), M, N, K, (int)r, p.rp, nullptr,
                             Ar, p.rp, nullptr, lora_scale, static_cast<uint16_t*>(dx),
                             r > 0 ? u : nullptr, p.rp, p.rp, st)))
       return rc;
-  } else if (p.skinny) {
+  } else if (p.cb > 0) {
     if (r > 0 && dA &&
-        (rc = launch_rowproj(elt, dyb, M, N, Bb, (int)r, p.rp, u, nullptr, nullptr, st)))
+        (rc = launch_rowproj(elt, dyb, M, N, Bb, (int)r, p.rp, u, nullptr, nullptr, st,
+                             p.few ? nullptr : reinterpret_cast<float*>(ws + w.rq))))
       return rc;
   } else if (p.deq) {
     // 1. u = dy B^T; 2. dx = dy wt^T + c u A^T with wt[k][n] = bf16(q[n][k] s[n])
@@ -1666,7 +1685,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
     }
   }
   // 2. dx = dys q + c u A^T (bf16), dx = dy f16(q f16(s)) + c u A^T (f16)
-  if (dx && !p.deq && !p.skinny) {
+  if (dx && !p.deq && p.cb == 0) {
     GemmArgs g{};
     g.act = f16 ? dyb : dys; g.q = q; g.colscale = nullptr; g.redscale = f16 ? scales : nullptr;
     g.L = r > 0 ? u : nullptr; g.R = Ar; g.bias = nullptr;
@@ -1677,7 +1696,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
   }
   // 3. dA = c x^T u ; dB = c (dy^T h)^T, in one launch (h recomputed first when not given)
   if (dB) {
-    if (!hh && p.skinny) {
+    if (!hh && p.cf > 0) {
       // recompute h exactly as the few-token forward computed it (same blocks, same split order)
       uint16_t* hw = reinterpret_cast<uint16_t*>(ws + w.h);
       const uint16_t* Ap = Ab;
@@ -1686,7 +1705,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
         if ((rc = launch_pad_cols(Ab, K, (int)r, r, ap, p.rp, p.rp, st))) return rc;
         Ap = ap;
       }
-      if ((rc = launch_skinny(0, elt, p.skf, xb, q, K, nullptr, Ap, reinterpret_cast<float*>(ws + w.wd),
+      if ((rc = launch_skinny(0, elt, p.cf, xb, q, K, nullptr, Ap, reinterpret_cast<float*>(ws + w.wd),
                               M, K, N, (int)r, p.rp, nullptr, nullptr, N, nullptr, lora_scale, nullptr,
                               hw, p.rp, p.rp, st, true)))
         return rc;

@@ -1302,6 +1302,36 @@ SkinnyPlan skinny_plan(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode)
   return p;
 }
 
+// Beyond the sizes of skinny_supported a direction may still run here, as consecutive launches over
+// token chunks that each fill one round of row-wave tiles, where the 256 x 256-tile GEMM would leave
+// most CUs idle or split its reduction through f32 partials (bound by their traffic and by five or
+// six launches). Both sides in us, fitted to bf16 at 64 to 11008 tokens on 1536 to 13824 wide layers:
+// a launch here takes 8.5 plus 0.6 (forward) or 0.76 (dX) per 128-deep step, 1.15 times that with 96-
+// token tiles; the GEMM path 36, its weight copy at 4 bytes a ns, 0.8 per 64-deep step and round, and
+// partials at 6 bytes a ns. Returns the tokens per launch, 0 if the GEMM is the better one.
+// Forward / backward with dA and dB, bf16, the GEMM before and chunks now: 1536 tokens on 1536 x 1536
+// 49.5 / 58.7 -> 15.7 / 28.5 us (one launch), 4096 there 75.6 / 86.4 -> 45.2 / 66.1, 1536 on 3072 x
+// 3072 96.4 / 102.3 -> 46.3 / 68.6, 333 on 1536 -> 8960 forward 63.3 -> 25.7, 1024 on 5120 x 5120
+// 87.5 / 106.4 -> 67.0 / 95.6; from there on up (1536 on 5120 x 5120: 111.4 / 128.9) the GEMM stays.
+// The errors against 64 bits are the same to four digits: both multiply the codes, or rnd(q s) in dX.
+int64_t skinny_chunk(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode) {
+  constexpr int64_t kMaxChunks = 6;
+  const int64_t tiles = ceil_div(M, 256) * ceil_div(Ncols, 256);
+  const int64_t ks = bfgemm_splits(M, Ncols, Kred);
+  double gemm = 36.0 + 0.8 * (double)ceil_div(Kred / 64, ks) * (double)ceil_div(tiles * ks, 256);
+  if (ks > 1) gemm += (double)(2 * ks * M * Ncols * 4) / 6e6;
+  if (ks == 1 || mode == 1) gemm += (double)(3 * Ncols * Kred) / 4e6;
+  for (int64_t n = 1; n <= kMaxChunks; ++n) {
+    const int64_t chunk = ceil_div(ceil_div(M, n), 16) * 16;
+    SkinnyPlan p;
+    if (!skinny_limits(chunk, Kred, Ncols, rp) || !rw_choose(chunk, Kred, Ncols, rp, mode, p)) continue;
+    const double step = (mode == 0 ? 0.6 : 0.76) * (p.To == 6 ? 1.15 : 1.0);
+    const double t = (double)ceil_div(M, chunk) * (8.5 + step * (double)(Kred / 128));
+    return t < 0.95 * gemm ? chunk : 0;  // more chunks only take longer
+  }
+  return 0;
+}
+
 // workspace of one launch: split partials, l [M][rp], then the keys; the offsets are the same in
 // sizing and use
 struct SkWs {
@@ -1325,8 +1355,11 @@ static SkWs skinny_ws(const SkinnyPlan& p, int64_t M, int64_t Ncols, int rp) {
   return w;
 }
 
-size_t skinny_ws_bytes(const SkinnyPlan& p, int64_t M, int64_t Ncols, int rp) {
-  return skinny_ws(p, M, Ncols, rp).total;
+size_t skinny_ws_bytes(int64_t chunk, int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode) {
+  size_t most = 0;
+  for (int64_t m : {std::min(chunk, M), M % chunk})  // the launches follow one another in one stream
+    if (m > 0) most = std::max(most, skinny_ws(skinny_plan(m, Kred, Ncols, rp, mode), m, Ncols, rp).total);
+  return most;
 }
 
 template <int MODE, int ELT, int T>
@@ -1366,12 +1399,12 @@ static uint64_t sk_next_nonce() {
   return next.fetch_add(1, std::memory_order_relaxed);
 }
 
-int launch_skinny(int mode, int elt, const SkinnyPlan& p, const uint16_t* act, const int8_t* q,
-                  int64_t ldq, const float* s, const uint16_t* lw, void* ws, int64_t M,
-                  int64_t Kred, int64_t Ncols, int r, int rp, const float* colscale,
-                  const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,
-                  uint16_t* lsave, int64_t ld_lsave, int lsave_cols, hipStream_t st,
-                  bool adapter_only) {
+static int launch_skinny_once(int mode, int elt, const SkinnyPlan& p, const uint16_t* act, const int8_t* q,
+                              int64_t ldq, const float* s, const uint16_t* lw, void* ws, int64_t M,
+                              int64_t Kred, int64_t Ncols, int r, int rp, const float* colscale,
+                              const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,
+                              uint16_t* lsave, int64_t ld_lsave, int lsave_cols, hipStream_t st,
+                              bool adapter_only) {
   SkArgs a;
   a.act = act; a.q = q; a.s = s; a.lw = lw;
   a.M = M; a.Kred = Kred; a.Ncols = Ncols; a.ldq = ldq;
@@ -1440,6 +1473,24 @@ int launch_skinny(int mode, int elt, const SkinnyPlan& p, const uint16_t* act, c
   if (attr != hipSuccess)
     return fail(REELS_HIP_EHIP, std::string("skinny_kernel: hipFuncSetAttribute: ") + hipGetErrorString(attr));
   return check_launch("skinny_kernel");
+}
+
+int launch_skinny(int mode, int elt, int64_t chunk, const uint16_t* act, const int8_t* q,
+                  int64_t ldq, const float* s, const uint16_t* lw, void* ws, int64_t M,
+                  int64_t Kred, int64_t Ncols, int r, int rp, const float* colscale,
+                  const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,
+                  uint16_t* lsave, int64_t ld_lsave, int lsave_cols, hipStream_t st,
+                  bool adapter_only) {
+  for (int64_t m0 = 0; m0 < M; m0 += chunk) {
+    const int64_t m = std::min(chunk, M - m0);
+    const SkinnyPlan p = skinny_plan(m, Kred, Ncols, r > 0 ? rp : 0, mode);
+    if (int rc = launch_skinny_once(mode, elt, p, act + m0 * Kred, q, ldq, s, lw, ws, m, Kred, Ncols, r, rp,
+                                    colscale, R, ldr, bias, c, out ? out + m0 * Ncols : nullptr,
+                                    lsave ? lsave + m0 * ld_lsave : nullptr, ld_lsave, lsave_cols, st,
+                                    adapter_only))
+      return rc;
+  }
+  return REELS_HIP_OK;
 }
 
 }  // namespace reels

@@ -255,6 +255,65 @@ def test_row_wave_tiles_on_narrow_weights(dev, M, K, N, r):
     assert_parity(dA.cpu().numpy(), go["dA"], f"M={M} dA")
     assert_parity(dB.cpu().numpy(), go["dB"], f"M={M} dB")
 
+
+@pytest.mark.parametrize("M,K,N,r", [
+    (1030, 1536, 1536, 32),   # just past the few-token path, still one launch
+    (1553, 1536, 1536, 24),   # two launches in both directions, the last of an odd length
+    (4096, 1536, 1536, 16),   # three launches, the last a shorter one
+    (1537, 3072, 3072, 8),    # rank below a tile, 96-token tiles
+    (600, 1536, 8960, 24),    # the two directions with chunks of their own
+    (1100, 8960, 1536, 32),   # a long reduction forward; dX on the GEMM
+    (1100, 1536, 8960, 40),   # the forward on the GEMM; a long reduction in dX
+    (2000, 1536, 2048, 0),    # no adapter
+])
+def test_token_chunks(dev, M, K, N, r):
+    """Token counts that run as consecutive row-wave launches over token chunks, in one direction or
+    both: y, h, dx, dA, dB against the oracle, the same bits when h is recomputed, and on replays of
+    a captured graph with eager calls between them."""
+    import torch
+    from reels_amd import i8lora_backward, i8lora_forward
+    host, d = _case(dev, M, K, N, max(r, 16), 6100 + M)
+    A, B = (d["A"][:, :r].contiguous(), d["B"][:r].contiguous()) if r else (None, None)
+    c = 0.5
+    print(f"[skinny] token chunks M={M} K={K} N={N} r={r}", flush=True)
+
+    def both(keep_h):
+        y, h = i8lora_forward(d["x"], d["W"], A, B, None, c, save_h=r > 0)
+        return (y, h) + tuple(i8lora_backward(d["dy"], d["x"], d["W"], A, B, c, h=h if keep_h else None))
+    first = both(True)
+    for a, b in zip(first, both(False)):
+        assert a is None or torch.equal(a, b)
+    side = torch.cuda.Stream(dev)
+    side.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(side):
+        both(True)
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize(dev)
+        with torch.cuda.graph(graph, stream=side):
+            out = both(True)
+    for _ in range(3):
+        for t in out:
+            if t is not None:
+                t.zero_()
+        graph.replay()
+        both(False)
+        torch.cuda.synchronize(dev)
+        for a, b in zip(first, out):
+            assert a is None or torch.equal(a, b)
+    hA, hB = (np.ascontiguousarray(host["A"][:, :r]), np.ascontiguousarray(host["B"][:r])) if r else (None, None)
+    yo, ho = oracle.lora_forward(host["x"], host["q"], host["s"], hA, hB, c)
+    go = oracle.lora_backward(host["dy"], host["x"], host["q"], host["s"],
+                              hA if r else np.zeros((K, 0), np.uint16), hB if r else np.zeros((0, N), np.uint16),
+                              c, want=("dx", "dA", "dB") if r else ("dx",))
+    y, h, dx, dA, dB = first
+    assert_parity(bf16_f32(y), yo, f"M={M} y")
+    assert_parity(bf16_f32(dx), go["dx"], f"M={M} dx")
+    if r:
+        assert_parity(bf16_f32(h), ho, f"M={M} h")
+        assert_parity(dA.cpu().numpy(), go["dA"], f"M={M} dA")
+        assert_parity(dB.cpu().numpy(), go["dB"], f"M={M} dB")
+
+
 def _abi_calls(dev, M, K, N, r, c, ws):
     """Forward and backward through the C-ABI on an explicit workspace ws (uint8, large enough
     for both)."""
