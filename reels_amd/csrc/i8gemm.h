@@ -98,6 +98,8 @@ bool skinny_supported(int64_t M, int64_t K, int64_t N, int rp);
 SkinnyPlan skinny_plan(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode);
 // tokens per launch for the token counts skinny_supported leaves to the GEMM (0: the GEMM)
 int64_t skinny_chunk(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode);
+// tokens the GEMM keeps of M, the others run here in launches of chunk (M: all on the GEMM)
+int64_t skinny_tail(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode, int64_t& chunk);
 // workspace of launches over chunks of M tokens: the split partials and l [chunk][rp]
 size_t skinny_ws_bytes(int64_t chunk, int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode);
 // One launch per chunk tokens (a multiple of 16 unless it is M):

@@ -897,6 +897,9 @@ struct Plan {
   // tokens per launch of that path in the forward (reduction K) and dX (reduction N): M when few,
   // chunks of M or 0 (the GEMMs) beyond
   int64_t cf, cb;
+  // tokens of the dequantized-weight GEMMs of the two directions; the others, past their whole
+  // rounds, follow on the few-token path in launches of tf, tb tokens
+  int64_t mf, mb, tf = 0, tb = 0;
   int rp;       // row stride of the h/u panels and padded adapter operands: round_up(r, 16)
   bool padded;  // rp != r: h, h_save and A go through padded copies in the workspace
   Split sa;     // dA: columns of x (K)
@@ -928,6 +931,7 @@ static void noalloc_plan(Plan& p) {
   p.deq = false;
   p.i8f = false;
   p.ksf = p.ksb = 1;
+  p.tf = p.tb = 0;
   if (!p.few) p.cf = p.cb = 0;  // the int8 GEMM, as its scratch bound was made for
 }
 
@@ -949,12 +953,17 @@ static Plan make_plan(int64_t M, int64_t K, int64_t N, int64_t r, bool ptrs_alig
   p.ksf = p.fast && p.cf == 0 ? bfgemm_splits(M, N, K) : 1;
   p.ksb = p.fast && p.cb == 0 ? bfgemm_splits(M, K, N) : 1;
   p.i8f = p.deq && p.ksf > 1;
+  p.mf = p.mb = M;
+  if (p.deq && p.cf == 0 && p.ksf == 1) p.mf = skinny_tail(M, K, N, rpl, 0, p.tf);
+  if (p.deq && p.cb == 0 && p.ksb == 1) p.mb = skinny_tail(M, N, K, rpl, 1, p.tb);
+  if (p.mf == M) p.tf = 0;
+  if (p.mb == M) p.tb = 0;
   return p;
 }
 
 // workspace layout (byte offsets, 256-aligned); identical computation for sizing and use
 struct WsLayout {
-  size_t h, u, dys, wd, at, bt, ap, pa, pb, pbias, kp, rq, total;
+  size_t h, u, dys, wd, at, bt, ap, pa, pb, pbias, kp, rq, tl, total;
 };
 
 static WsLayout ws_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which, const Plan& p) {
@@ -983,6 +992,7 @@ static WsLayout ws_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which,
         w.rq = take(rs > 1 ? (size_t)rs * M * rp * 4 : 0);
       }
       w.kp = take(p.ksb > 1 ? (size_t)p.ksb * M * K * 4 : 0);
+      w.tl = take(p.tb > 0 ? skinny_ws_bytes(p.tb, M - p.mb, N, K, rpl, 1) : 0);
       w.pa = take(r > 0 ? (size_t)p.sa.splits * K * rp * 4 : 0);
       w.pb = take(r > 0 ? (size_t)p.sb.splits * N * rp * 4 : 0);
       w.pbias = take(colsum_partial_bytes(M, N));
@@ -1001,8 +1011,11 @@ static WsLayout ws_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which,
   if (which == REELS_HIP_WS_FWD) {
     w.bt = take(p.fast ? (size_t)N * rp * 2 : 0);
     w.kp = take(p.ksf > 1 ? (size_t)p.ksf * M * N * 4 : 0);  // split GEMM partials
+    w.ap = take(p.tf > 0 && p.padded ? (size_t)K * rp * 2 : 0);  // the tail's A [K][rp]
+    w.tl = take(p.tf > 0 ? skinny_ws_bytes(p.tf, M - p.mf, K, N, rpl, 0) : 0);
   } else {
     w.kp = take(p.ksb > 1 ? (size_t)p.ksb * M * K * 4 : 0);
+    w.tl = take(p.tb > 0 ? skinny_ws_bytes(p.tb, M - p.mb, N, K, rpl, 1) : 0);
     w.u = take((size_t)M * rp * 2);
     w.ap = take(p.padded ? (size_t)K * rp * 2 : 0);  // A [K][rp], zeros past r
     w.dys = take(p.fast && !p.deq ? (size_t)M * N * 2 : 0);
@@ -1432,7 +1445,7 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
                            const float* scales, const void* A, const void* B, const void* bias,
                            int64_t M, int64_t K, int64_t N, int64_t r, float lora_scale, void* y,
                            void* h_save, void* workspace, size_t ws_bytes, void* stream,
-                           bool noalloc = false, void* gout = nullptr, bool* gelu_fused = nullptr,
+                           bool noalloc = false, void* gout = nullptr, int64_t* gelu_rows = nullptr,
                            bool codes = false) {
   clear_error();
   if (M < 0 || K <= 0 || N <= 0 || r < 0 || r > 4096)
@@ -1535,8 +1548,20 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
     g.q = nullptr; g.colscale = nullptr;
     g.gout = static_cast<uint16_t*>(gout);
     if (g.gout && !bfgemm_fuses_gelu_fwd(g)) g.gout = nullptr;
-    if (g.gout && gelu_fused) *gelu_fused = true;
-    return launch_bfgemm(0, elt, g, wd, st);
+    if (p.tf > 0) g.M = p.mf;
+    if (g.gout && gelu_rows) *gelu_rows = g.M;
+    if ((rc = launch_bfgemm(0, elt, g, wd, st)) || p.tf == 0) return rc;
+    // the tokens past the whole rounds (their h is the projection's)
+    const uint16_t* Ap = static_cast<const uint16_t*>(A);
+    if (r > 0 && p.padded) {
+      uint16_t* ap = reinterpret_cast<uint16_t*>(ws + w.ap);
+      if ((rc = launch_pad_cols(Ap, K, (int)r, r, ap, p.rp, p.rp, st))) return rc;
+      Ap = ap;
+    }
+    return launch_skinny(0, elt, p.tf, xb + p.mf * K, q, K, nullptr, r > 0 ? Ap : nullptr, ws + w.tl,
+                         M - p.mf, K, N, (int)r, p.rp, scales, static_cast<const uint16_t*>(B), N,
+                         static_cast<const uint16_t*>(bias), lora_scale,
+                         static_cast<uint16_t*>(y) + p.mf * N, nullptr, r, (int)r, st);
   }
   return launch_i8gemm(0, elt, g, st);
 }
@@ -1545,7 +1570,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
                            const int8_t* q, const float* scales, const void* A, const void* B,
                            int64_t M, int64_t K, int64_t N, int64_t r, float lora_scale, void* dx,
                            float* dA, float* dB, float* dbias, void* workspace, size_t ws_bytes,
-                           void* stream, const void* gx = nullptr, bool* gelu_fused = nullptr) {
+                           void* stream, const void* gx = nullptr, int64_t* gelu_rows = nullptr) {
   clear_error();
   if (M < 0 || K <= 0 || N <= 0 || r < 0 || r > 4096)
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": " "need M >= 0, K > 0, N > 0, 0 <= r <= 4096");
@@ -1669,8 +1694,14 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
       g.ksplit = p.ksb; g.part = reinterpret_cast<float*>(ws + w.kp);
       g.gx = static_cast<const uint16_t*>(gx);
       if (g.gx && !bfgemm_fuses_gelu(g)) g.gx = nullptr;
-      if (g.gx && gelu_fused) *gelu_fused = true;
+      if (p.tb > 0) g.M = p.mb;
+      if (g.gx && gelu_rows) *gelu_rows = g.M;
       if ((rc = launch_bfgemm(1, elt, g, wt, st))) return rc;
+      if (p.tb > 0 &&  // the tokens past the whole rounds (their u is the projection's)
+          (rc = launch_skinny(1, elt, p.tb, dyb + p.mb * N, q, K, scales, r > 0 ? Bb : nullptr, ws + w.tl,
+                              M - p.mb, N, K, (int)r, p.rp, nullptr, Ar, p.rp, nullptr, lora_scale,
+                              static_cast<uint16_t*>(dx) + p.mb * K, nullptr, p.rp, p.rp, st)))
+        return rc;
     }
   } else if (r > 0 || (dx && !f16)) {
     // 1. u = dy B^T and (bf16) dys = dy * s in one pass over dy (the scaled copy only when dx is
@@ -1918,12 +1949,13 @@ static int i8lora_fwd_gelu_impl(int elt, const char* fn, const void* x, const in
     clear_error();
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": NULL g");
   }
-  bool fused = false;
+  int64_t done = 0;  // rows whose GELU the GEMM's epilogue took
   if (int rc = i8lora_fwd_impl(elt, fn, x, q, scales, A, B, bias, M, K, N, r, lora_scale, y, h_save,
-                               workspace, ws_bytes, stream, false, g, &fused))
+                               workspace, ws_bytes, stream, false, g, &done))
     return rc;
-  if (fused || M == 0) return REELS_HIP_OK;
-  return gelu_impl(elt, fn, y, g, M * N, stream);
+  if (done >= M) return REELS_HIP_OK;
+  return gelu_impl(elt, fn, static_cast<const uint16_t*>(y) + done * N, static_cast<uint16_t*>(g) + done * N,
+                   (M - done) * N, stream);
 }
 
 extern "C" int reels_hip_i8lora_fwd_gelu(const void* x, const int8_t* q, const float* scales,
@@ -1957,12 +1989,13 @@ static int i8lora_bwd_gelu_impl(int elt, const char* fn, const void* dy, const v
     clear_error();
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": NULL gx with dx");
   }
-  bool fused = false;
+  int64_t done = 0;  // rows whose GELU the GEMM's epilogue took
   if (int rc = i8lora_bwd_impl(elt, fn, dy, x, h, q, scales, A, B, M, K, N, r, lora_scale, dx, dA,
-                               dB, dbias, workspace, ws_bytes, stream, dx ? gx : nullptr, &fused))
+                               dB, dbias, workspace, ws_bytes, stream, dx ? gx : nullptr, &done))
     return rc;
-  if (fused || M == 0 || !dx) return REELS_HIP_OK;
-  return gelu_bwd_impl(elt, fn, gx, dx, dx, M * K, stream);
+  if (done >= M || !dx) return REELS_HIP_OK;
+  uint16_t* rest = static_cast<uint16_t*>(dx) + done * K;
+  return gelu_bwd_impl(elt, fn, static_cast<const uint16_t*>(gx) + done * K, rest, rest, (M - done) * K, stream);
 }
 
 extern "C" int reels_hip_i8lora_bwd_gelu(const void* dy, const void* x, const void* h,

@@ -1302,12 +1302,25 @@ SkinnyPlan skinny_plan(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode)
   return p;
 }
 
+// Estimated time (us) of row-wave launches over chunks of M tokens, each chunk (out) filling one
+// round: 8.5 and per 128-deep step 0.6 (forward) or 0.76 (dX), 1.15 times that with 96-token tiles
+static double chunk_time(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode, int64_t& chunk) {
+  constexpr int64_t kMaxChunks = 6;
+  for (int64_t n = 1; n <= kMaxChunks; ++n) {
+    chunk = ceil_div(ceil_div(M, n), 16) * 16;
+    SkinnyPlan p;
+    if (!skinny_limits(chunk, Kred, Ncols, rp) || !rw_choose(chunk, Kred, Ncols, rp, mode, p)) continue;
+    const double step = (mode == 0 ? 0.6 : 0.76) * (p.To == 6 ? 1.15 : 1.0);
+    return (double)ceil_div(M, chunk) * (8.5 + step * (double)(Kred / 128));
+  }
+  return 1e30;
+}
+
 // Beyond the sizes of skinny_supported a direction may still run here, as consecutive launches over
 // token chunks that each fill one round of row-wave tiles, where the 256 x 256-tile GEMM would leave
 // most CUs idle or split its reduction through f32 partials (bound by their traffic and by five or
-// six launches). Both sides in us, fitted to bf16 at 64 to 11008 tokens on 1536 to 13824 wide layers:
-// a launch here takes 8.5 plus 0.6 (forward) or 0.76 (dX) per 128-deep step, 1.15 times that with 96-
-// token tiles; the GEMM path 36, its weight copy at 4 bytes a ns, 0.8 per 64-deep step and round, and
+// six launches). Both sides are fitted to bf16 at 64 to 11008 tokens on 1536 to 13824 wide layers:
+// the GEMM path takes 36 us, its weight copy at 4 bytes a ns, 0.8 us per 64-deep step and round, and
 // partials at 6 bytes a ns. Returns the tokens per launch, 0 if the GEMM is the better one.
 // Forward / backward with dA and dB, bf16, the GEMM before and chunks now: 1536 tokens on 1536 x 1536
 // 49.5 / 58.7 -> 15.7 / 28.5 us (one launch), 4096 there 75.6 / 86.4 -> 45.2 / 66.1, 1536 on 3072 x
@@ -1315,21 +1328,27 @@ SkinnyPlan skinny_plan(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode)
 // 87.5 / 106.4 -> 67.0 / 95.6; from there on up (1536 on 5120 x 5120: 111.4 / 128.9) the GEMM stays.
 // The errors against 64 bits are the same to four digits: both multiply the codes, or rnd(q s) in dX.
 int64_t skinny_chunk(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode) {
-  constexpr int64_t kMaxChunks = 6;
   const int64_t tiles = ceil_div(M, 256) * ceil_div(Ncols, 256);
   const int64_t ks = bfgemm_splits(M, Ncols, Kred);
   double gemm = 36.0 + 0.8 * (double)ceil_div(Kred / 64, ks) * (double)ceil_div(tiles * ks, 256);
   if (ks > 1) gemm += (double)(2 * ks * M * Ncols * 4) / 6e6;
   if (ks == 1 || mode == 1) gemm += (double)(3 * Ncols * Kred) / 4e6;
-  for (int64_t n = 1; n <= kMaxChunks; ++n) {
-    const int64_t chunk = ceil_div(ceil_div(M, n), 16) * 16;
-    SkinnyPlan p;
-    if (!skinny_limits(chunk, Kred, Ncols, rp) || !rw_choose(chunk, Kred, Ncols, rp, mode, p)) continue;
-    const double step = (mode == 0 ? 0.6 : 0.76) * (p.To == 6 ? 1.15 : 1.0);
-    const double t = (double)ceil_div(M, chunk) * (8.5 + step * (double)(Kred / 128));
-    return t < 0.95 * gemm ? chunk : 0;  // more chunks only take longer
-  }
-  return 0;
+  int64_t chunk = 0;
+  return chunk_time(M, Kred, Ncols, rp, mode, chunk) < 0.95 * gemm ? chunk : 0;
+}
+
+// Tokens that the GEMM leaves to row-wave launches after it: with 256 x 256 tiles a little past whole
+// rounds of the 256 CUs, the last round is nearly empty and takes as long as a full one (1.05 us per
+// 64-deep step and 4 for its epilogue, measured with 222 against 258 tiles and 240 against 320). The
+// GEMM then takes the tokens of the whole rounds only. Returns M for no tail. Forward / backward, bf16:
+// 11008 tokens on 8960 -> 1536 390.7 / 323.7 -> 274.6 / 300.3 us, on 1536 x 1536 90.9 / 108.9 -> 70.7 /
+// 91.2, 6144 on 3072 x 3072 147.2 / 168.1 -> 117.5 / 143.5, 9360 on 1536 -> 8960 forward 252 -> 230.5.
+int64_t skinny_tail(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode, int64_t& chunk) {
+  const int64_t tn = ceil_div(Ncols, 256), tiles = ceil_div(M, 256) * tn, rounds = tiles / 256;
+  const int64_t rows = rounds * 256 / tn * 256;
+  if (rounds < 1 || tiles % 256 == 0 || rows <= 0 || rows >= M) return M;
+  const double saved = 4.0 + 1.05 * (double)(Kred / 64);
+  return chunk_time(M - rows, Kred, Ncols, rp, mode, chunk) + 3.0 < 0.85 * saved ? rows : M;
 }
 
 // workspace of one launch: split partials, l [M][rp], then the keys; the offsets are the same in

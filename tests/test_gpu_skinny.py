@@ -265,10 +265,12 @@ def test_row_wave_tiles_on_narrow_weights(dev, M, K, N, r):
     (1100, 8960, 1536, 32),   # a long reduction forward; dX on the GEMM
     (1100, 1536, 8960, 40),   # the forward on the GEMM; a long reduction in dX
     (2000, 1536, 2048, 0),    # no adapter
+    (11001, 1536, 1536, 24),  # the GEMM's whole round and the 249 tokens past it, both directions
+    (4900, 1536, 3584, 16),   # the GEMM's whole round in the forward; dX on the GEMM alone
 ])
 def test_token_chunks(dev, M, K, N, r):
     """Token counts that run as consecutive row-wave launches over token chunks, in one direction or
-    both: y, h, dx, dA, dB against the oracle, the same bits when h is recomputed, and on replays of
+    both, or on the GEMM with such launches past its whole rounds: y, h, dx, dA, dB against the oracle, the same bits when h is recomputed, and on replays of
     a captured graph with eager calls between them."""
     import torch
     from reels_amd import i8lora_backward, i8lora_forward
@@ -403,3 +405,23 @@ def test_graph_replays_on_changing_inputs(dev):
         torch.cuda.synchronize(dev)
         for name, a, b in zip(("y", "h", "dx", "dA", "dB"), out, refs[k]):
             assert torch.equal(a, b), f"replay {rnd} (inputs {k}): {name} differs from eager"
+
+
+def test_gelu_past_the_whole_rounds(dev):
+    """The feed-forward entry points where the GEMM takes 4608 of 4900 tokens with the GELU in its
+    epilogue and the rest follow on row-wave tiles: the bits of the separate GELU passes."""
+    import torch
+    from reels_amd import (gelu_tanh, gelu_tanh_backward, i8lora_backward, i8lora_backward_gelu,
+                           i8lora_forward, i8lora_forward_gelu)
+    M, K, N, r = 4900, 1536, 3584, 16
+    print("[skinny] GELU past the whole rounds", flush=True)
+    _, d = _case(dev, M, K, N, r, 7100)
+    z, a, _ = i8lora_forward_gelu(d["x"], d["W"], d["A"], d["B"], None, 1.0, save_h=True)
+    z2, _ = i8lora_forward(d["x"], d["W"], d["A"], d["B"], None, 1.0, save_h=True)
+    assert torch.equal(z, z2) and torch.equal(a, gelu_tanh(z))
+    _, e = _case(dev, M, N, K, r, 7200)  # the second projection N -> K
+    g = i8lora_backward_gelu(e["dy"], a, z, e["W"], e["A"], e["B"], 1.0)
+    p = i8lora_backward(e["dy"], a, e["W"], e["A"], e["B"], 1.0)
+    torch.cuda.synchronize(dev)
+    assert torch.equal(g[0], gelu_tanh_backward(z, p[0]))
+    assert torch.equal(g[1], p[1]) and torch.equal(g[2], p[2])
