@@ -11,8 +11,9 @@
 //      (no float atomics: bitwise reproducible)                          (HBM-bound)
 // Every rank takes the fast kernels: the LoRA panels h, u and the adapter operands live in the
 // workspace with rp = round_up(r, 16) columns (zeros past r), and the projection and gradient
-// kernels run in rank chunks of up to 128. Widths that are no multiples of 64 run on operands
-// zero-padded to the next multiples in the workspace (pad_shape). What neither takes (unaligned
+// kernels run in rank chunks of up to 128. Few tokens, and where it is faster token chunks of larger
+// calls and the tokens past the GEMM's whole rounds, run on the kernels of skinny.hip instead of 1 to 3
+// and of 1 and 2. Widths that are no multiples of 64 run on operands zero-padded to the next multiples in the workspace (pad_shape). What neither takes (unaligned
 // pointers, widths of 2^22 and more) runs through the generic kernels at the bottom, which compute
 // the same formulas with the same bf16 rounding points, one output element per thread.
 #include "i8gemm.h"
@@ -931,8 +932,8 @@ static void noalloc_plan(Plan& p) {
   p.deq = false;
   p.i8f = false;
   p.ksf = p.ksb = 1;
-  p.tf = p.tb = 0;
-  if (!p.few) p.cf = p.cb = 0;  // the int8 GEMM, as its scratch bound was made for
+  p.tf = p.tb = 0;  // token chunks stay: at most 256 adapter blocks' partials (10 KiB each) and one
+                    // chunk's l, less than the scratch at every rank they take, and h keeps its bits
 }
 
 static Plan make_plan(int64_t M, int64_t K, int64_t N, int64_t r, bool ptrs_aligned) {
@@ -1387,7 +1388,7 @@ extern "C" size_t reels_hip_i8lora_workspace_bytes(int64_t M, int64_t K, int64_t
   Plan p = make_plan(M, K, N, r, true);
   if (which == REELS_HIP_WS_FWD_NOALLOC) {
     noalloc_plan(p);
-    which = REELS_HIP_WS_FWD;
+    return ws_layout(M, K, N, r, REELS_HIP_WS_FWD, p).total;
   }
   // unaligned buffers take the generic layout
   return std::max(ws_layout(M, K, N, r, which, p).total,
