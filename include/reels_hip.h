@@ -101,8 +101,10 @@ size_t reels_hip_i8lora_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t
  * zero-padded copies in the workspace), and the
  * few-token path (M <= 240, or M <= 1024 with N * K <= 2^22; K and N multiples of 64), which
  * reads the int8 codes without a weight copy. Up to a few thousand tokens that path also runs over
- * chunks of the tokens where it is faster than the GEMM, and behind the GEMM over the tokens past
- * its whole rounds of 256 x 256 output tiles. With few 256 x 256 output tiles (a few hundred
+ * chunks of the tokens where it is faster than the GEMM. One call multiplies one weight: the tokens
+ * past the GEMM's whole rounds of 256 x 256 output tiles run on other kernels, with the same W and h
+ * (their sums are taken in another f32 order, so equal rows of x may differ in the last bit of y by
+ * their position, here as between the tiles of the few-token path). With few 256 x 256 output tiles (a few hundred
  * tokens) the GEMM splits its reduction over several workgroups and sums their f32 partials in a
  * fixed order before the one rounding (the workspace holds them); the forward then multiplies the
  * int8 codes with s on the f32 sum, no weight copy. bias may be NULL. r = 0 (A, B NULL) gives the base-only
@@ -121,9 +123,9 @@ int reels_hip_i8lora_fwd(const void* x, const int8_t* q, const float* scales, co
  * rounding above becomes an f16 rounding (nearest even). The weight is the one the bf16 entry
  * point's shape rules pick, in binary16: where that entry point multiplies a dequantized copy
  * (K and N multiples of 64, many tokens), W = f16(q * f16(s)) as _dequantize_for_compute
- * computes it; where it multiplies the int8 codes (the few-token path, whole calls or their last
- * tokens, the split-reduction forward over a few hundred tokens, K or N not a multiple of 64),
- * s[n] is applied to the f32 sum of x * q, so y can differ from the f16(q * f16(s)) product in the last f16 bit. The
+ * computes it; where it multiplies the int8 codes (the few-token path, the split-reduction
+ * forward over a few hundred tokens, K or N not a multiple of 64), s[n] is applied to the f32
+ * sum of x * q, so y can differ from the f16(q * f16(s)) product in the last f16 bit. The
  * backward (reels_hip_i8lora_bwd_f16) always multiplies f16(q * f16(s)). Same workspace size.
  */
 int reels_hip_i8lora_fwd_f16(const void* x, const int8_t* q, const float* scales, const void* A,

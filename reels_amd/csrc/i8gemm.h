@@ -98,8 +98,9 @@ bool skinny_supported(int64_t M, int64_t K, int64_t N, int rp);
 SkinnyPlan skinny_plan(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode);
 // tokens per launch for the token counts skinny_supported leaves to the GEMM (0: the GEMM)
 int64_t skinny_chunk(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode);
-// tokens the GEMM keeps of M, the others run here in launches of chunk (M: all on the GEMM)
-int64_t skinny_tail(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode, int64_t& chunk);
+// tokens the GEMM keeps of M, the others run on launch_skinny_tail in launches of chunk (M: all on
+// the GEMM)
+int64_t skinny_tail(int64_t M, int64_t Kred, int64_t Ncols, int mode, int64_t& chunk);
 // workspace of launches over chunks of M tokens: the split partials and l [chunk][rp]
 size_t skinny_ws_bytes(int64_t chunk, int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode);
 // One launch per chunk tokens (a multiple of 16 unless it is M):
@@ -107,7 +108,7 @@ size_t skinny_ws_bytes(int64_t chunk, int64_t M, int64_t Kred, int64_t Ncols, in
 // ([M][ld_lsave], lsave_cols columns, zeros past r) when not NULL; R(o, j) = R[j][o] (mode 0,
 // row stride ldr) or R[o][j] (mode 1, rows of ldr >= rp elements, zeros past r). adapter_only: l
 // alone, from the same blocks and split order as a full launch (so a recomputed h equals the
-// forward's bit for bit). The launch's counters live in ws (cleared by a kernel before it), so
+// forward's bit for bit). What the blocks hand to each other lies in ws under keys of the launch, so
 // launches with their own workspaces may run concurrently.
 int launch_skinny(int mode, int elt, int64_t chunk, const uint16_t* act, const int8_t* q,
                   int64_t ldq, const float* s, const uint16_t* lw, void* ws, int64_t M,
@@ -115,6 +116,13 @@ int launch_skinny(int mode, int elt, int64_t chunk, const uint16_t* act, const i
                   const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,
                   uint16_t* lsave, int64_t ld_lsave, int lsave_cols, hipStream_t st,
                   bool adapter_only = false);
+// The GEMM's products for the tokens it leaves: out = rnd(act rnd(q s)^T + c l R + bias) with the
+// weight the GEMM multiplies (s of the output row in mode 0, of the reduction in mode 1) and the l it
+// reads ([M][rp], zeros past r; NULL with r = 0). No workspace.
+int launch_skinny_tail(int mode, int elt, int64_t chunk, const uint16_t* act, const int8_t* q, int64_t ldq,
+                       const float* s, const uint16_t* l, int64_t M, int64_t Kred, int64_t Ncols, int r, int rp,
+                       const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,
+                       hipStream_t st);
 
 // out = c * sum over splits of part[sp][o][j] (split order): out[o][j], or out[j][o] with trans
 int launch_reduce_partials(const float* part, int splits, int64_t Od, int rp, int r, float c,

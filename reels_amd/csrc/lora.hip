@@ -12,10 +12,11 @@
 // Every rank takes the fast kernels: the LoRA panels h, u and the adapter operands live in the
 // workspace with rp = round_up(r, 16) columns (zeros past r), and the projection and gradient
 // kernels run in rank chunks of up to 128. Few tokens, and where it is faster token chunks of larger
-// calls and the tokens past the GEMM's whole rounds, run on the kernels of skinny.hip instead of 1 to 3
-// and of 1 and 2. Widths that are no multiples of 64 run on operands zero-padded to the next multiples in the workspace (pad_shape). What neither takes (unaligned
-// pointers, widths of 2^22 and more) runs through the generic kernels at the bottom, which compute
-// the same formulas with the same bf16 rounding points, one output element per thread.
+// calls, run on the kernels of skinny.hip instead; the tokens past the GEMM's whole rounds run on them
+// instead of the GEMM. Widths that are no multiples of 64 run on operands zero-padded to the next
+// multiples in the workspace (pad_shape). What neither takes (unaligned pointers, widths of 2^22 and
+// more) runs through the generic kernels at the bottom, which compute the same formulas with the same
+// bf16 rounding points, one output element per thread.
 #include "i8gemm.h"
 
 #include <algorithm>
@@ -955,8 +956,8 @@ static Plan make_plan(int64_t M, int64_t K, int64_t N, int64_t r, bool ptrs_alig
   p.ksb = p.fast && p.cb == 0 ? bfgemm_splits(M, K, N) : 1;
   p.i8f = p.deq && p.ksf > 1;
   p.mf = p.mb = M;
-  if (p.deq && p.cf == 0 && p.ksf == 1) p.mf = skinny_tail(M, K, N, rpl, 0, p.tf);
-  if (p.deq && p.cb == 0 && p.ksb == 1) p.mb = skinny_tail(M, N, K, rpl, 1, p.tb);
+  if (p.deq && p.cf == 0 && p.ksf == 1) p.mf = skinny_tail(M, K, N, 0, p.tf);
+  if (p.deq && p.cb == 0 && p.ksb == 1) p.mb = skinny_tail(M, N, K, 1, p.tb);
   if (p.mf == M) p.tf = 0;
   if (p.mb == M) p.tb = 0;
   return p;
@@ -964,7 +965,7 @@ static Plan make_plan(int64_t M, int64_t K, int64_t N, int64_t r, bool ptrs_alig
 
 // workspace layout (byte offsets, 256-aligned); identical computation for sizing and use
 struct WsLayout {
-  size_t h, u, dys, wd, at, bt, ap, pa, pb, pbias, kp, rq, tl, total;
+  size_t h, u, dys, wd, at, bt, ap, pa, pb, pbias, kp, rq, total;
 };
 
 static WsLayout ws_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which, const Plan& p) {
@@ -993,7 +994,6 @@ static WsLayout ws_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which,
         w.rq = take(rs > 1 ? (size_t)rs * M * rp * 4 : 0);
       }
       w.kp = take(p.ksb > 1 ? (size_t)p.ksb * M * K * 4 : 0);
-      w.tl = take(p.tb > 0 ? skinny_ws_bytes(p.tb, M - p.mb, N, K, rpl, 1) : 0);
       w.pa = take(r > 0 ? (size_t)p.sa.splits * K * rp * 4 : 0);
       w.pb = take(r > 0 ? (size_t)p.sb.splits * N * rp * 4 : 0);
       w.pbias = take(colsum_partial_bytes(M, N));
@@ -1012,11 +1012,8 @@ static WsLayout ws_layout(int64_t M, int64_t K, int64_t N, int64_t r, int which,
   if (which == REELS_HIP_WS_FWD) {
     w.bt = take(p.fast ? (size_t)N * rp * 2 : 0);
     w.kp = take(p.ksf > 1 ? (size_t)p.ksf * M * N * 4 : 0);  // split GEMM partials
-    w.ap = take(p.tf > 0 && p.padded ? (size_t)K * rp * 2 : 0);  // the tail's A [K][rp]
-    w.tl = take(p.tf > 0 ? skinny_ws_bytes(p.tf, M - p.mf, K, N, rpl, 0) : 0);
   } else {
     w.kp = take(p.ksb > 1 ? (size_t)p.ksb * M * K * 4 : 0);
-    w.tl = take(p.tb > 0 ? skinny_ws_bytes(p.tb, M - p.mb, N, K, rpl, 1) : 0);
     w.u = take((size_t)M * rp * 2);
     w.ap = take(p.padded ? (size_t)K * rp * 2 : 0);  // A [K][rp], zeros past r
     w.dys = take(p.fast && !p.deq ? (size_t)M * N * 2 : 0);
@@ -1496,7 +1493,7 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
   const uint16_t* xb = static_cast<const uint16_t*>(x);
   int rc;
   if (p.cf > 0) {
-    // few tokens: y and h from the int8 codes in one launch
+    // few tokens: y and h from the int8 codes, one launch per chunk of tokens
     const uint16_t* Ap = static_cast<const uint16_t*>(A);
     if (r > 0 && p.padded) {
       uint16_t* ap = reinterpret_cast<uint16_t*>(ws + w.ap);
@@ -1552,17 +1549,11 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
     if (p.tf > 0) g.M = p.mf;
     if (g.gout && gelu_rows) *gelu_rows = g.M;
     if ((rc = launch_bfgemm(0, elt, g, wd, st)) || p.tf == 0) return rc;
-    // the tokens past the whole rounds (their h is the projection's)
-    const uint16_t* Ap = static_cast<const uint16_t*>(A);
-    if (r > 0 && p.padded) {
-      uint16_t* ap = reinterpret_cast<uint16_t*>(ws + w.ap);
-      if ((rc = launch_pad_cols(Ap, K, (int)r, r, ap, p.rp, p.rp, st))) return rc;
-      Ap = ap;
-    }
-    return launch_skinny(0, elt, p.tf, xb + p.mf * K, q, K, nullptr, r > 0 ? Ap : nullptr, ws + w.tl,
-                         M - p.mf, K, N, (int)r, p.rp, scales, static_cast<const uint16_t*>(B), N,
-                         static_cast<const uint16_t*>(bias), lora_scale,
-                         static_cast<uint16_t*>(y) + p.mf * N, nullptr, r, (int)r, st);
+    // the tokens past the whole rounds: the same weight rnd(q s) and the same h
+    return launch_skinny_tail(0, elt, p.tf, xb + p.mf * K, q, K, scales, r > 0 ? h + p.mf * p.rp : nullptr,
+                              M - p.mf, K, N, (int)r, p.rp, static_cast<const uint16_t*>(B), N,
+                              static_cast<const uint16_t*>(bias), lora_scale,
+                              static_cast<uint16_t*>(y) + p.mf * N, st);
   }
   return launch_i8gemm(0, elt, g, st);
 }
@@ -1698,10 +1689,10 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
       if (p.tb > 0) g.M = p.mb;
       if (g.gx && gelu_rows) *gelu_rows = g.M;
       if ((rc = launch_bfgemm(1, elt, g, wt, st))) return rc;
-      if (p.tb > 0 &&  // the tokens past the whole rounds (their u is the projection's)
-          (rc = launch_skinny(1, elt, p.tb, dyb + p.mb * N, q, K, scales, r > 0 ? Bb : nullptr, ws + w.tl,
-                              M - p.mb, N, K, (int)r, p.rp, nullptr, Ar, p.rp, nullptr, lora_scale,
-                              static_cast<uint16_t*>(dx) + p.mb * K, nullptr, p.rp, p.rp, st)))
+      if (p.tb > 0 &&  // the tokens past the whole rounds: the same weight and the same u
+          (rc = launch_skinny_tail(1, elt, p.tb, dyb + p.mb * N, q, K, scales, r > 0 ? u + p.mb * p.rp : nullptr,
+                                   M - p.mb, N, K, (int)r, p.rp, Ar, p.rp, nullptr, lora_scale,
+                                   static_cast<uint16_t*>(dx) + p.mb * K, st)))
         return rc;
     }
   } else if (r > 0 || (dx && !f16)) {

@@ -57,7 +57,7 @@ constexpr uint32_t kSpinLimit = 1u << 12;  // wait rounds of s_sleep 8 (about 1 
 struct SkArgs {
   const uint16_t* act;  // [M][Kred] 16-bit: x (FWD) or dy (DX)
   const int8_t* q;      // codes [N][K], row stride ldq
-  const float* s;       // DX: scale of the reduction index n
+  const float* s;       // DX: scale of the reduction index n; FWD with rounded weights: of the output row
   const uint16_t* lw;   // adapter operand: FWD A [Kred][rp] (zeros past r), DX B [r][Kred]
   float* part;          // split partials in MFMA fragment order (output tiles, then adapter tiles)
   uint16_t* hl;         // [M][rp] l rounded to the element type (zeros past r)
@@ -78,6 +78,7 @@ struct SkArgs {
   int nta;     // adapter tiles (lblk * tb)
   int64_t lpart0;  // first partial fragment of the adapter tiles (after the output tiles')
   int otb;     // row-wave output tiles: token tiles (the output tile is ti / otb, ti % otb)
+  bool lgiven; // hl holds l already (no adapter blocks)
 };
 
 struct SkBlock {
@@ -816,7 +817,26 @@ constexpr int rw_fslots(int To, int NI, int MODE) {
   return (160 * 1024 - 16) / rw_fstep(To, NI, MODE) > 8 ? 8 : (160 * 1024 - 16) / rw_fstep(To, NI, MODE);
 }
 
-template <int To, int NI, int MODE, int ELT>
+// 8 codes times their scales, rounded: Float16(q) * Float16(s), or bf16(fl32(q * s))
+template <int ELT>
+__device__ __forceinline__ typename Elt<ELT>::v8 rw_scaled(uint32_t lo, uint32_t hi, const f32x4& s0,
+                                                           const f32x4& s1) {
+  using E = Elt<ELT>;
+  if constexpr (ELT == REELS_HIP_F16) {
+    const u32x4 s16 = {E::pack2(s0[0], s0[1]), E::pack2(s0[2], s0[3]), E::pack2(s1[0], s1[1]), E::pack2(s1[2], s1[3])};
+    return E::scale8(E::from_i8x8(lo, hi), s16);
+  } else {
+    const u32x4 o = {E::pack2_fast((float)(int8_t)(lo & 0xffu) * s0[0], (float)(int8_t)((lo >> 8) & 0xffu) * s0[1]),
+                     E::pack2_fast((float)(int8_t)((lo >> 16) & 0xffu) * s0[2], (float)((int32_t)lo >> 24) * s0[3]),
+                     E::pack2_fast((float)(int8_t)(hi & 0xffu) * s1[0], (float)(int8_t)((hi >> 8) & 0xffu) * s1[1]),
+                     E::pack2_fast((float)(int8_t)((hi >> 16) & 0xffu) * s1[2], (float)((int32_t)hi >> 24) * s1[3])};
+    return E::as8(o);
+  }
+}
+
+// RND (FWD): the codes are multiplied as the dequantized weight rnd(q s[o]), o the lane's row, in
+// place of the exact codes
+template <int To, int NI, int MODE, int ELT, bool RND>
 __device__ __forceinline__ void rw_acc_dma(const SkArgs& a, int64_t r0, int64_t tok0, int rot,
                                            uint8_t* smem, f32x4 (&acc)[NI][To]) {
   using E = Elt<ELT>;
@@ -859,6 +879,17 @@ __device__ __forceinline__ void rw_acc_dma(const SkArgs& a, int64_t r0, int64_t 
       const int idx = (NI * w + i) * 64 + lane, n = idx / (4 * NI);
       const int64_t col = r0 + 16 * ((idx % (4 * NI)) ^ rw_dswz<NI>(n));
       vw[i] = col < a.Ncols ? (uint32_t)(n * a.ldq + col) : OOB;
+    }
+  }
+  f32x4 srow[NI];  // RND: the scale of row 16 i + l16, four times
+  if constexpr (RND) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int64_t row = r0 + 16 * NI * wr + 16 * i + l16;
+      float v = row < a.Ncols ? a.s[row] : 0.0f;
+      // arrived before the first copy is issued: the waits of the steps count copies alone
+      asm volatile("s_waitcnt vmcnt(0)" : "+v"(v)::"memory");
+      srow[i] = f32x4{v, v, v, v};
     }
   }
   const uint32_t wstep = MODE == 0 ? 128u : (uint32_t)(128 * a.ldq);
@@ -917,7 +948,9 @@ __device__ __forceinline__ void rw_acc_dma(const SkArgs& a, int64_t r0, int64_t 
 #pragma unroll
       for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) af[i][e] = E::from_i8x8(cv[i][2 * e], cv[i][2 * e + 1]);
+        for (int e = 0; e < 2; ++e)
+          af[i][e] = RND ? rw_scaled<ELT>(cv[i][2 * e], cv[i][2 * e + 1], srow[i], srow[i])
+                         : E::from_i8x8(cv[i][2 * e], cv[i][2 * e + 1]);
     } else {
       // per 16-k tile i and half e the transposed read: providing lane p of a 16-lane group
       // addresses row n = 64 par + 32 e + 8 g + p / 2, unit NI wr + i, bytes 8 (p % 2) .. +7;
@@ -933,18 +966,7 @@ __device__ __forceinline__ void rw_acc_dma(const SkArgs& a, int64_t r0, int64_t 
           const int row = 64 * par + 32 * e + 8 * g + (l16 >> 1);
           const uint8_t* p = base + SLOT + row * (64 * NI) + (((NI * wr + i) ^ rw_dswz<NI>(row)) << 4) + 8 * (l16 & 1);
           const i32x2 v = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(i32x2, p));
-          if constexpr (ELT == REELS_HIP_F16) {  // Float16(q) * Float16(s[n])
-            const u32x4 s16 = {E::pack2(s0[0], s0[1]), E::pack2(s0[2], s0[3]),
-                               E::pack2(s1[0], s1[1]), E::pack2(s1[2], s1[3])};
-            af[i][e] = E::scale8(E::from_i8x8((uint32_t)v[0], (uint32_t)v[1]), s16);
-          } else {  // bf16(fl32(q * s[n]))
-            const uint32_t lo = (uint32_t)v[0], hi = (uint32_t)v[1];
-            const u32x4 o = {E::pack2_fast((float)(int8_t)(lo & 0xffu) * s0[0], (float)(int8_t)((lo >> 8) & 0xffu) * s0[1]),
-                             E::pack2_fast((float)(int8_t)((lo >> 16) & 0xffu) * s0[2], (float)((int32_t)lo >> 24) * s0[3]),
-                             E::pack2_fast((float)(int8_t)(hi & 0xffu) * s1[0], (float)(int8_t)((hi >> 8) & 0xffu) * s1[1]),
-                             E::pack2_fast((float)(int8_t)((hi >> 16) & 0xffu) * s1[2], (float)((int32_t)hi >> 24) * s1[3])};
-            af[i][e] = E::as8(o);
-          }
+          af[i][e] = rw_scaled<ELT>((uint32_t)v[0], (uint32_t)v[1], s0, s1);
         }
       }
     }
@@ -1031,8 +1053,9 @@ __device__ __forceinline__ void rw_lora(const SkArgs& a, int64_t ob, int64_t tok
 
 // One row-wave output tile: the wave's accumulators, the pair sum of waves w and w + 4 (each
 // keeps half the token tiles), l when the adapter blocks have published it (or computed here with
-// their code, splits and order when they have not), then out = rnd(scale sum + c l R + bias).
-template <int To, int NI, int Ta, int MODE, int ELT>
+// their code, splits and order when they have not), then out = rnd(scale sum + c l R + bias). With
+// a.lgiven (always with RND) l lies in a.hl before the launch.
+template <int To, int NI, int Ta, int MODE, int ELT, bool RND>
 __device__ __forceinline__ void rw_block(const SkArgs& a, int rb, int tbo, uint8_t* smem,
                                          int lds_bytes) {
   using E = Elt<ELT>;
@@ -1045,7 +1068,7 @@ __device__ __forceinline__ void rw_block(const SkArgs& a, int rb, int tbo, uint8
   const int64_t ob = r0 + 16 * NI * wr;          // the wave's first output row
   const int64_t tw0 = tok0 + (int64_t)par * (16 * TH);  // the wave's first token after the pair sum
   uint32_t* words = reinterpret_cast<uint32_t*>(smem + lds_bytes - 16);  // [0], [3] key, [2] l ready
-  const bool wants_l = a.nad > 0;
+  const bool wants_l = !RND && a.nad > 0;
   sk_stash_key(words);
 
   f32x4 sum[NI][TH];
@@ -1058,7 +1081,7 @@ __device__ __forceinline__ void rw_block(const SkArgs& a, int rb, int tbo, uint8
     // row block: 512 tokens on 5120 x 5120 40.4 against 35.1 us forward.)
     const int nsteps = (int)(a.Kred / 128);
     const int rot = (int)(((int64_t)(blockIdx.x & 7) * nsteps) / 8);
-    rw_acc_dma<To, NI, MODE, ELT>(a, r0, tok0, rot, smem, acc);
+    rw_acc_dma<To, NI, MODE, ELT, RND>(a, r0, tok0, rot, smem, acc);
     // waves 4-7 give their first half of the token tiles, waves 0-3 their second, through LDS;
     // each then adds (partner + own, wave w's value first: the same sum for both halves)
     f32x4* ex = reinterpret_cast<f32x4*>(smem);
@@ -1081,7 +1104,7 @@ __device__ __forceinline__ void rw_block(const SkArgs& a, int rb, int tbo, uint8
     __syncthreads();  // LDS free again
   }
 
-  if (wants_l) {
+  if constexpr (!RND) if (wants_l) {
     // the adapter tiles of this tile's tokens: they come first in the logical order and wait for
     // nothing but their splits, so their keys are normally there; after a bounded wait the block
     // computes l for its tokens itself, with the adapter blocks' code, splits and order (the same
@@ -1123,7 +1146,7 @@ __device__ __forceinline__ void rw_block(const SkArgs& a, int rb, int tbo, uint8
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int tt = 0; tt < TH; ++tt) lo[i][tt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  if (wants_l) rw_lora<NI, TH, MODE, ELT>(a, ob, tw0, smem + w * (1024 * NI), lo);
+  if (wants_l || (a.lgiven && a.rp > 0)) rw_lora<NI, TH, MODE, ELT>(a, ob, tw0, smem + w * (1024 * NI), lo);
 
   // out = rnd(scale * sum + c * lo + bias), rows o = ob + 16 i + 4 g + v, token 16 tt + l16
 #pragma unroll
@@ -1150,7 +1173,7 @@ __device__ __forceinline__ void rw_block(const SkArgs& a, int rb, int tbo, uint8
   }
 }
 
-template <int To, int NI, int Ta, int MODE, int ELT>
+template <int To, int NI, int Ta, int MODE, int ELT, bool RND>
 __global__ __launch_bounds__(64 * sk::NWV, 1) void skinny_rw_kernel(SkArgs a, int lds_bytes) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   // the logical order and XCD mapping of skinny_kernel: adapter blocks first, then the output
@@ -1159,7 +1182,7 @@ __global__ __launch_bounds__(64 * sk::NWV, 1) void skinny_rw_kernel(SkArgs a, in
   const int b = (int)blockIdx.x, xcd = b & 7, idx = b >> 3;
   const int per = a.blocks >> 3, rem = a.blocks & 7;
   const int tk = xcd * per + (xcd < rem ? xcd : rem) + idx;
-  if (tk < a.nad) {
+  if (!RND && tk < a.nad) {
     int rest = tk;
     SkBlock d;
     d.tb = rest % a.tb;
@@ -1171,7 +1194,7 @@ __global__ __launch_bounds__(64 * sk::NWV, 1) void skinny_rw_kernel(SkArgs a, in
     skinny_block<Ta, MODE, ELT, true>(a, d, smem);
   } else {
     const int ti = tk - a.nad;
-    rw_block<To, NI, Ta, MODE, ELT>(a, ti / a.otb, ti % a.otb, smem, lds_bytes);
+    rw_block<To, NI, Ta, MODE, ELT, RND>(a, ti / a.otb, ti % a.otb, smem, lds_bytes);
   }
 }
 
@@ -1303,14 +1326,17 @@ SkinnyPlan skinny_plan(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode)
 }
 
 // Estimated time (us) of row-wave launches over chunks of M tokens, each chunk (out) filling one
-// round: 8.5 and per 128-deep step 0.6 (forward) or 0.76 (dX), 1.15 times that with 96-token tiles
-static double chunk_time(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode, int64_t& chunk) {
+// round: 8.5 and per 128-deep step 0.6 with exact codes or 0.76 with scaled ones, 1.15 times that with
+// 96-token tiles. all_rw: the last, shorter chunk takes row-wave tiles too
+static double chunk_time(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode, bool scaled, bool all_rw,
+                         int64_t& chunk) {
   constexpr int64_t kMaxChunks = 6;
   for (int64_t n = 1; n <= kMaxChunks; ++n) {
     chunk = ceil_div(ceil_div(M, n), 16) * 16;
-    SkinnyPlan p;
+    SkinnyPlan p, last;
     if (!skinny_limits(chunk, Kred, Ncols, rp) || !rw_choose(chunk, Kred, Ncols, rp, mode, p)) continue;
-    const double step = (mode == 0 ? 0.6 : 0.76) * (p.To == 6 ? 1.15 : 1.0);
+    if (all_rw && M % chunk != 0 && !rw_choose(M % chunk, Kred, Ncols, rp, mode, last)) continue;
+    const double step = (scaled ? 0.76 : 0.6) * (p.To == 6 ? 1.15 : 1.0);
     return (double)ceil_div(M, chunk) * (8.5 + step * (double)(Kred / 128));
   }
   return 1e30;
@@ -1334,21 +1360,24 @@ int64_t skinny_chunk(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode) {
   if (ks > 1) gemm += (double)(2 * ks * M * Ncols * 4) / 6e6;
   if (ks == 1 || mode == 1) gemm += (double)(3 * Ncols * Kred) / 4e6;
   int64_t chunk = 0;
-  return chunk_time(M, Kred, Ncols, rp, mode, chunk) < 0.95 * gemm ? chunk : 0;
+  return chunk_time(M, Kred, Ncols, rp, mode, mode == 1, false, chunk) < 0.95 * gemm ? chunk : 0;
 }
 
 // Tokens that the GEMM leaves to row-wave launches after it: with 256 x 256 tiles a little past whole
 // rounds of the 256 CUs, the last round is nearly empty and takes as long as a full one (1.05 us per
 // 64-deep step and 4 for its epilogue, measured with 222 against 258 tiles and 240 against 320). The
-// GEMM then takes the tokens of the whole rounds only. Returns M for no tail. Forward / backward, bf16:
-// 11008 tokens on 8960 -> 1536 390.7 / 323.7 -> 274.6 / 300.3 us, on 1536 x 1536 90.9 / 108.9 -> 70.7 /
-// 91.2, 6144 on 3072 x 3072 147.2 / 168.1 -> 117.5 / 143.5, 9360 on 1536 -> 8960 forward 252 -> 230.5.
-int64_t skinny_tail(int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode, int64_t& chunk) {
+// GEMM then takes the tokens of the whole rounds only, and the others multiply the same rounded weight
+// and the same l (launch_skinny_tail). Returns M for no tail. Forward / backward, bf16:
+// 11008 tokens on 8960 -> 1536 390.7 / 323.7 -> 278.6 / 304.2 us, on 1536 x 1536 90.9 / 108.9 -> 69.3 /
+// 91.4, 6144 on 3072 x 3072 147.2 / 168.1 -> 120.9 / 143.1, 9360 on 1536 -> 8960 forward 252 -> 233.
+// The scaled conversion of the codes costs no more than the adapter blocks that exact codes with an l
+// of the launch's own needed (the last, 233.0 us, and 11001 on 1536 x 1536, r 24, 75.2 -> 71.3).
+int64_t skinny_tail(int64_t M, int64_t Kred, int64_t Ncols, int mode, int64_t& chunk) {
   const int64_t tn = ceil_div(Ncols, 256), tiles = ceil_div(M, 256) * tn, rounds = tiles / 256;
   const int64_t rows = rounds * 256 / tn * 256;
   if (rounds < 1 || tiles % 256 == 0 || rows <= 0 || rows >= M) return M;
   const double saved = 4.0 + 1.05 * (double)(Kred / 64);
-  return chunk_time(M - rows, Kred, Ncols, rp, mode, chunk) + 3.0 < 0.85 * saved ? rows : M;
+  return chunk_time(M - rows, Kred, Ncols, 0, mode, true, true, chunk) + 3.0 < 0.85 * saved ? rows : M;
 }
 
 // workspace of one launch: split partials, l [M][rp], then the keys; the offsets are the same in
@@ -1394,17 +1423,38 @@ static hipError_t launch_skinny_t(const SkArgs& a, hipStream_t st) {
   return hipSuccess;
 }
 
-template <int To, int NI, int Ta, int MODE, int ELT>
+template <int To, int NI, int Ta, int MODE, int ELT, bool RND>
 static hipError_t launch_rw_t(const SkArgs& a, int lds, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [] {
-    attr = hipFuncSetAttribute((const void*)skinny_rw_kernel<To, NI, Ta, MODE, ELT>,
+    attr = hipFuncSetAttribute((const void*)skinny_rw_kernel<To, NI, Ta, MODE, ELT, RND>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, kRwLdsMax);
   });
   if (attr != hipSuccess) return attr;
-  skinny_rw_kernel<To, NI, Ta, MODE, ELT><<<dim3((unsigned)a.blocks), 64 * sk::NWV, lds, st>>>(a, lds);
+  skinny_rw_kernel<To, NI, Ta, MODE, ELT, RND><<<dim3((unsigned)a.blocks), 64 * sk::NWV, lds, st>>>(a, lds);
   return hipSuccess;
+}
+
+template <bool RND>
+static hipError_t launch_rw(int mode, int elt, const SkinnyPlan& p, const SkArgs& a, hipStream_t st) {
+  TraceScope _ts(st, mode == 0 ? "skinny_rw_kernel<0>" : "skinny_rw_kernel<1>");
+  const int lds = rw_lds_bytes(p.NI, p.To, mode, a.Kred);
+  hipError_t attr = hipSuccess;
+  with_elt(elt, [&](auto el) {
+    constexpr int EL = decltype(el)::value;
+    auto go = [&](auto m) {
+      constexpr int MD = decltype(m)::value;
+      constexpr bool R = RND && MD == 0;  // dX scales its codes in every form
+      if (p.NI == 1 && p.To == 2) attr = launch_rw_t<2, 1, 2, MD, EL, R>(a, lds, st);
+      else if (p.NI == 1 && p.To == 4) attr = launch_rw_t<4, 1, 4, MD, EL, R>(a, lds, st);
+      else if (p.NI == 2 && p.To == 4) attr = launch_rw_t<4, 2, 4, MD, EL, R>(a, lds, st);
+      else attr = launch_rw_t<6, 2, 3, MD, EL, R>(a, lds, st);
+    };
+    if (mode == 0) go(std::integral_constant<int, 0>{});
+    else go(std::integral_constant<int, 1>{});
+  });
+  return attr;
 }
 
 // the nonce of a row-wave launch's keys: a process-wide count from a random start (so two
@@ -1424,7 +1474,7 @@ static int launch_skinny_once(int mode, int elt, const SkinnyPlan& p, const uint
                               const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,
                               uint16_t* lsave, int64_t ld_lsave, int lsave_cols, hipStream_t st,
                               bool adapter_only) {
-  SkArgs a;
+  SkArgs a{};
   a.act = act; a.q = q; a.s = s; a.lw = lw;
   a.M = M; a.Kred = Kred; a.Ncols = Ncols; a.ldq = ldq;
   a.r = r; a.rp = r > 0 ? rp : 0; a.S = p.S;
@@ -1457,20 +1507,7 @@ static int launch_skinny_once(int mode, int elt, const SkinnyPlan& p, const uint
 
   hipError_t attr = hipSuccess;
   if (p.rw) {
-    TraceScope _ts(st, mode == 0 ? "skinny_rw_kernel<0>" : "skinny_rw_kernel<1>");
-    const int lds = rw_lds_bytes(p.NI, p.To, mode, Kred);
-    with_elt(elt, [&](auto el) {
-      constexpr int EL = decltype(el)::value;
-      auto go = [&](auto m) {
-        constexpr int MD = decltype(m)::value;
-        if (p.NI == 1 && p.To == 2) attr = launch_rw_t<2, 1, 2, MD, EL>(a, lds, st);
-        else if (p.NI == 1 && p.To == 4) attr = launch_rw_t<4, 1, 4, MD, EL>(a, lds, st);
-        else if (p.NI == 2 && p.To == 4) attr = launch_rw_t<4, 2, 4, MD, EL>(a, lds, st);
-        else attr = launch_rw_t<6, 2, 3, MD, EL>(a, lds, st);
-      };
-      if (mode == 0) go(std::integral_constant<int, 0>{});
-      else go(std::integral_constant<int, 1>{});
-    });
+    attr = launch_rw<false>(mode, elt, p, a, st);
   } else {
     TraceScope _ts(st, mode == 0 ? "skinny_kernel<0>" : "skinny_kernel<1>");
     with_elt(elt, [&](auto el) {
@@ -1508,6 +1545,31 @@ int launch_skinny(int mode, int elt, int64_t chunk, const uint16_t* act, const i
                                     lsave ? lsave + m0 * ld_lsave : nullptr, ld_lsave, lsave_cols, st,
                                     adapter_only))
       return rc;
+  }
+  return REELS_HIP_OK;
+}
+
+int launch_skinny_tail(int mode, int elt, int64_t chunk, const uint16_t* act, const int8_t* q, int64_t ldq,
+                       const float* s, const uint16_t* l, int64_t M, int64_t Kred, int64_t Ncols, int r, int rp,
+                       const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,
+                       hipStream_t st) {
+  for (int64_t m0 = 0; m0 < M; m0 += chunk) {
+    const int64_t m = std::min(chunk, M - m0);
+    SkinnyPlan p;
+    if (!rw_choose(m, Kred, Ncols, 0, mode, p)) return fail(REELS_HIP_EINVAL, "skinny_tail: shape not supported");
+    SkArgs a{};
+    a.act = act + m0 * Kred; a.q = q; a.s = s; a.M = m; a.Kred = Kred; a.Ncols = Ncols; a.ldq = ldq;
+    a.r = r; a.rp = r > 0 ? rp : 0; a.S = 1;
+    a.nblk = (int)(Ncols / sk::NB); a.tb = p.tb;
+    a.R = R; a.ldr = ldr; a.bias = bias; a.c = c; a.out = out + m0 * Ncols;
+    a.hl = const_cast<uint16_t*>(r > 0 ? l + m0 * rp : nullptr);
+    a.lgiven = true;
+    a.ntm = p.orb * p.otb; a.otb = p.otb;
+    a.blocks = a.ntm;
+    const hipError_t attr = launch_rw<true>(mode, elt, p, a, st);
+    if (attr != hipSuccess)
+      return fail(REELS_HIP_EHIP, std::string("skinny_kernel: hipFuncSetAttribute: ") + hipGetErrorString(attr));
+    if (int rc = check_launch("skinny_rw_kernel")) return rc;
   }
   return REELS_HIP_OK;
 }

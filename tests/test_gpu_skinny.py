@@ -425,3 +425,39 @@ def test_gelu_past_the_whole_rounds(dev):
     torch.cuda.synchronize(dev)
     assert torch.equal(g[0], gelu_tanh_backward(z, p[0]))
     assert torch.equal(g[1], p[1]) and torch.equal(g[2], p[2])
+
+
+@pytest.mark.parametrize("elt", ["bf16", "f16"])
+@pytest.mark.parametrize("M,mf,K,N,r", [
+    (11001, 10752, 1536, 1536, 24),  # both directions
+    (4900, 4608, 1536, 3584, 16),    # the forward; dX on the GEMM alone
+])
+def test_tokens_past_the_whole_rounds_multiply_the_same_operands(dev, M, mf, K, N, r, elt):
+    """The tokens that follow the GEMM repeat its first ones, row by row. Both multiply the dequantized
+    weight rnd(q s) and the same h (u), so their sums differ in f32 order alone: by about 2^-20 of an
+    output, which moves 2 * 2^-20 over one unit in the last place of them (2e-3 in f16 with its 2^-10,
+    an eighth of that in bf16; twice that is allowed) over a rounding boundary, by one unit. With the
+    exact codes for the weight two in five differ. With codes of zero and unit rows in B, y is the
+    saved h bit for bit."""
+    import torch
+    from reels_amd import QuantizedMatrix, i8lora_backward, i8lora_forward
+    print(f"[skinny] past the whole rounds {elt} M={M} K={K} N={N} r={r}", flush=True)
+    _, d = _case(dev, M, K, N, r, 7300 + M, elt)
+    for n in ("x", "dy"):
+        d[n][mf:] = d[n][:M - mf]
+    y, h = i8lora_forward(d["x"], d["W"], d["A"], d["B"], None, 0.5, save_h=True)
+    dx = i8lora_backward(d["dy"], d["x"], d["W"], d["A"], d["B"], 0.5, h=h)[0]
+    assert torch.equal(h[mf:], h[:M - mf])
+    ulp = 2.0 ** (-7 if elt == "bf16" else -10)
+    for name, t in (("y", y), ("dx", dx)):
+        a, b = t[:M - mf].double(), t[mf:].double()
+        off = float((a != b).double().mean())
+        print(f"[skinny] {name}: {off:.2e} of the repeated rows' outputs differ", flush=True)
+        assert off <= 4e-3, name
+        assert bool(((a - b).abs() <= ulp * a.abs() + 2.0 ** -20 * t.double().std()).all()), name
+    zero = QuantizedMatrix(torch.zeros_like(d["W"].values), d["W"].scales, d["x"].dtype)
+    B = torch.zeros_like(d["B"])
+    B[torch.arange(r), torch.arange(r)] = 1.0
+    y, h = i8lora_forward(d["x"], zero, d["A"], B, None, 1.0, save_h=True)
+    torch.cuda.synchronize(dev)
+    assert torch.equal(y[:, :r], h) and not bool(y[:, r:].any())
