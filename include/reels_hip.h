@@ -160,11 +160,11 @@ int reels_hip_i8lora_fwd_noalloc(const void* x, const int8_t* q, const float* sc
  *   u  = bf16(dy * B^T)                                                      [M][r]
  *   dx = bf16(sum_n dy[m][n] W[n][k] + lora_scale * sum_j u[m][j] A[k][j])
  *   dA = lora_scale * x^T u   (f32 [K][r]);   dB = lora_scale * h^T dy   (f32 [r][N])
- * W = bf16(fl32(q * s)) (a transposed copy in the workspace, or, on the few-token path of
- * reels_hip_i8lora_fwd, built in registers from the codes); K or N that are no multiples of 64 are
- * zero-padded in the workspace. On the smallest such layers (up to 64 tokens, K and N up to 128),
- * at sizes those copies do not support and with unaligned operands at multiples of 64, the product
- * is taken as sum_n bf16(dy[m][n] s[n]) q[n][k]. h: the
+ * W = bf16(fl32(q * s)) when K and N are multiples of 64 (a transposed copy in the workspace, or,
+ * on the few-token path of reels_hip_i8lora_fwd, built in registers from the codes); when K or N
+ * is not a multiple of 64 (on zero-padded copies in the workspace, the smallest layers and sizes
+ * those copies do not support excepted), and with unaligned operands, the product is taken as
+ * sum_n bf16(dy[m][n] s[n]) q[n][k]. h: the
  * forward's h_save ([M][r]) or NULL to recompute it.
  * dx, dA, dB may each be NULL to skip that output. r = 0 gives dx = deq(W)^T dy alone
  * (_weight_transpose_mul). dA and dB are overwritten (not accumulated) and are bitwise

@@ -104,7 +104,7 @@ int64_t skinny_tail(int64_t M, int64_t Kred, int64_t Ncols, int mode, int64_t& c
 // workspace of launches over chunks of M tokens: the split partials and l [chunk][rp]
 size_t skinny_ws_bytes(int64_t chunk, int64_t M, int64_t Kred, int64_t Ncols, int rp, int mode);
 // One launch per chunk tokens (a multiple of 16 unless it is M):
-// out = rnd(colscale * act W + c l R + bias) with l = rnd(act L) (h or u), written to lsave
+// out = rnd(colscale * oact W + c l R + bias) (oact NULL: act) with l = rnd(act L) (h or u), written to lsave
 // ([M][ld_lsave], lsave_cols columns, zeros past r) when not NULL; R(o, j) = R[j][o] (mode 0,
 // row stride ldr) or R[o][j] (mode 1, rows of ldr >= rp elements, zeros past r). adapter_only: l
 // alone, from the same blocks and split order as a full launch (so a recomputed h equals the
@@ -115,7 +115,7 @@ int launch_skinny(int mode, int elt, int64_t chunk, const uint16_t* act, const i
                   int64_t Kred, int64_t Ncols, int r, int rp, const float* colscale,
                   const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,
                   uint16_t* lsave, int64_t ld_lsave, int lsave_cols, hipStream_t st,
-                  bool adapter_only = false);
+                  bool adapter_only = false, const uint16_t* oact = nullptr);
 // The GEMM's products for the tokens it leaves: out = rnd(act rnd(q s)^T + c l R + bias) with the
 // weight the GEMM multiplies (s of the output row in mode 0, of the reduction in mode 1) and the l it
 // reads ([M][rp], zeros past r; NULL with r = 0). No workspace.

@@ -683,18 +683,19 @@ __global__ void fill_f32_kernel(float* p, int64_t n, float v) {
   if (i < n) p[i] = v;
 }
 
-// dst[i][j] = j < cols ? src[i][j] : 0 for j < cols_dst (16-bit elements; rows of ld_src and
-// ld_dst): widens a [rows][r] LoRA operand to the padded [rows][rp] layout of the fast kernels,
-// or (cols = cols_dst = r) compacts a padded one back to [rows][r]
 // Up to kMaxCopies 2-d copies in one launch: rows of bsrc valid bytes at stride lds go to rows of
 // bdst bytes at stride ldd, zeros past the valid bytes and past rows_src. Any alignment (a 16-byte
 // access at any address is one instruction; only the piece across the end of a row goes byte by
-// byte). Four 16-byte pieces per thread, their loads issued together.
+// byte). Four 16-byte pieces per thread, their loads issued together. SCALED: a job with a scale writes
+// bf16(src * scale[column]) of its bf16 elements to sdst, laid out as dst, beside the copy (or, with dst
+// NULL, alone), and a job without a source writes 1.0f.
 struct CopyJob {
   const uint8_t* src;
   uint8_t* dst;
   int64_t lds, ldd, bsrc, bdst, rows_src;
   uint32_t cpr, total;  // 16-byte pieces per output row, in all
+  const float* scale;
+  uint8_t* sdst;
 };
 constexpr int kMaxCopies = 8, kCopyPieces = 4;
 struct CopyJobs {
@@ -703,36 +704,64 @@ struct CopyJobs {
   int n;
 };
 typedef u32x4 u32x4_any __attribute__((aligned(1)));
+template <bool SCALED>
 __global__ __launch_bounds__(256) void copy2d_kernel(CopyJobs js) {
   int k = 0;
   while (k + 1 < js.n && blockIdx.x >= js.end[k]) ++k;
   const CopyJob& a = js.j[k];
   const uint32_t b = blockIdx.x - (k > 0 ? js.end[k - 1] : 0u);
   u32x4 v[kCopyPieces];
+  f32x4 sc[SCALED ? kCopyPieces : 1][2];
+  // scales past the last column read zeros, as the columns do
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(a.scale), (short)0, SCALED && a.scale != nullptr ? (int)(a.bsrc * 2) : 0, 0x00020000);
 #pragma unroll
   for (int i = 0; i < kCopyPieces; ++i) {
     const uint32_t id = (b * kCopyPieces + i) * 256u + threadIdx.x;
     v[i] = u32x4{0u, 0u, 0u, 0u};
+    if constexpr (SCALED) {
+      const uint32_t so = (id % a.cpr) * 32u;
+      sc[i][0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, so, 0, 0));
+      sc[i][1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, so + 16u, 0, 0));
+    }
     if (id >= a.total) continue;
     const uint32_t row = id / a.cpr, off = (id - row * a.cpr) * 16u;
     if (row >= a.rows_src) continue;
+    if (SCALED && a.src == nullptr) {
+      v[i] = u32x4{0x3f800000u, 0x3f800000u, 0x3f800000u, 0x3f800000u};
+      continue;
+    }
     const uint8_t* p = a.src + row * a.lds + off;
     if (off + 16 <= a.bsrc) v[i] = *reinterpret_cast<const u32x4_any*>(p);
     else
       for (int e = 0; off + e < a.bsrc; ++e) v[i][e >> 2] |= (uint32_t)p[e] << (8 * (e & 3));
   }
+  auto store = [&](uint8_t* p, uint32_t off, const u32x4& x) {
+    if (off + 16 <= a.bdst) *reinterpret_cast<u32x4_any*>(p) = x;
+    else
+      for (int e = 0; off + e < a.bdst; ++e) p[e] = (uint8_t)(x[e >> 2] >> (8 * (e & 3)));
+  };
 #pragma unroll
   for (int i = 0; i < kCopyPieces; ++i) {
     const uint32_t id = (b * kCopyPieces + i) * 256u + threadIdx.x;
     if (id >= a.total) continue;
     const uint32_t row = id / a.cpr, off = (id - row * a.cpr) * 16u;
-    uint8_t* p = a.dst + row * a.ldd + off;
-    if (off + 16 <= a.bdst) *reinterpret_cast<u32x4_any*>(p) = v[i];
-    else
-      for (int e = 0; off + e < a.bdst; ++e) p[e] = (uint8_t)(v[i][e >> 2] >> (8 * (e & 3)));
+    if (!SCALED || a.dst != nullptr) store(a.dst + row * a.ldd + off, off, v[i]);
+    if (SCALED && a.scale != nullptr) {
+      using E = Elt<REELS_HIP_BF16>;
+      const f32x4 s0 = sc[i][0], s1 = sc[i][1];
+      const u32x4 o = {E::pack2(E::lo(v[i][0]) * s0[0], E::hi(v[i][0]) * s0[1]),
+                       E::pack2(E::lo(v[i][1]) * s0[2], E::hi(v[i][1]) * s0[3]),
+                       E::pack2(E::lo(v[i][2]) * s1[0], E::hi(v[i][2]) * s1[1]),
+                       E::pack2(E::lo(v[i][3]) * s1[2], E::hi(v[i][3]) * s1[3])};
+      store(a.sdst + row * a.ldd + off, off, o);
+    }
   }
 }
 
+// dst[i][j] = j < cols ? src[i][j] : 0 for j < cols_dst (16-bit elements; rows of ld_src and
+// ld_dst): widens a [rows][r] LoRA operand to the padded [rows][rp] layout of the fast kernels,
+// or (cols = cols_dst = r) compacts a padded one back to [rows][r]
 __global__ void pad_cols_kernel(const uint16_t* __restrict__ src, int64_t rows, int cols,
                                 int64_t ld_src, uint16_t* __restrict__ dst, int cols_dst,
                                 int64_t ld_dst) {
@@ -1035,13 +1064,13 @@ static int64_t pad_width(int64_t M, int64_t d) {
 
 // Widths that are no multiples of 64: the call runs on copies zero-padded to the next multiples
 // (Kp, Np) in the workspace, so it meets the same kernels as any other shape, and the outputs'
-// valid parts are copied out. The forward then multiplies the int8 codes (s on the f32 sum), as
-// the direct kernels do for these widths; dX multiplies the dequantized weight. The copies cost a
-// read and a write of each operand, four launches of 5-9 us in 65 us forward and backward for 777
-// tokens, 1000 -> 3000 (rank 8); the one-output-per-thread kernels took 11.0 ms there, and widths that are
-// multiples of 16 ran unsplit 256 x 256 tiles (1000 tokens, 528 -> 2064: 236 against 89 us). dX's
-// error against 64 bits stays: 2.341e-3 to 2.349e-3 with rnd(dy s) times the codes, 2.343e-3 to
-// 2.347e-3 with rnd(q s), over seven shapes.
+// valid parts are copied out. The products are those of the direct kernels at these widths: the
+// forward multiplies the int8 codes (s on the f32 sum), dX in bf16 rnd(dy s) and the codes (the copy
+// of dy for it scaled and rounded, scales of one for the inner call), in f16 the dequantized weight.
+// The copies cost a read and a write of each operand, in four launches of 5-9 us in 65 us forward and
+// backward for 777 tokens, 1000 -> 3000 (rank 8; the scaled copy of dy 1.5 us of it, 12 us of 342 for the
+// backward of 8192 tokens, 2064 -> 5136); the one-output-per-thread kernels took 11.0 ms there, and widths
+// that are multiples of 16 ran unsplit 256 x 256 tiles (1000 tokens, 528 -> 2064: 236 against 89 us).
 static bool pad_shape(int64_t M, int64_t K, int64_t N) {
   if (K % 64 == 0 && N % 64 == 0) return false;
   // tiny layers: the direct kernels' single launch is shorter than the copies' launches (one token,
@@ -1055,7 +1084,7 @@ static bool pad_shape(int64_t M, int64_t K, int64_t N) {
 
 struct PadLayout {
   int64_t Kp, Np, rp;  // padded widths, and the rank padded to a multiple of 16
-  size_t q, s, x, A, B, bias, y, h, dy, dx, dA, dB, db, inner, total;
+  size_t q, s, x, A, B, bias, y, h, dy, dys, dx, dA, dB, db, inner, total;
   Plan p;  // the plan of the padded call
 };
 
@@ -1078,6 +1107,7 @@ static PadLayout pad_layout(int64_t M, int64_t K, int64_t N, int64_t r, int whic
     w.y = take((size_t)M * w.Np * 2);
   } else {
     w.dy = take((size_t)M * w.Np * 2);
+    w.dys = take((size_t)M * w.Np * 2);
     w.dx = take((size_t)M * w.Kp * 2);
     w.dA = take((size_t)w.Kp * r * 4);
     w.dB = take((size_t)w.Np * r * 4);
@@ -1097,12 +1127,15 @@ static int grid1(int64_t n, int bs = 256) { return (int)ceil_div(n, bs); }
 struct Copies {
   CopyJobs js{};
   uint32_t blocks = 0;
+  bool scaled = false;
   void add(const void* src, int64_t rows, int64_t cols, int64_t lds, void* dst, int64_t rows_d,
-           int64_t cols_d, int64_t ldd, int esz) {
+           int64_t cols_d, int64_t ldd, int esz, const float* scale = nullptr, void* sdst = nullptr) {
     if (rows_d <= 0 || cols_d <= 0) return;
     CopyJob& j = js.j[js.n];
     j.src = static_cast<const uint8_t*>(src); j.dst = static_cast<uint8_t*>(dst);
     j.lds = lds * esz; j.ldd = ldd * esz; j.bsrc = cols * esz; j.bdst = cols_d * esz; j.rows_src = rows;
+    j.scale = scale; j.sdst = static_cast<uint8_t*>(sdst);
+    scaled |= scale != nullptr || src == nullptr;
     j.cpr = (uint32_t)ceil_div(j.bdst, 16);
     j.total = (uint32_t)(rows_d * j.cpr);
     blocks += (uint32_t)ceil_div(j.total, 256 * kCopyPieces);
@@ -1110,7 +1143,8 @@ struct Copies {
   }
   int launch(hipStream_t st) const {
     if (js.n == 0) return REELS_HIP_OK;
-    { TraceScope _ts(st, "copy2d_kernel"); copy2d_kernel<<<blocks, 256, 0, st>>>(js); }
+    { TraceScope _ts(st, "copy2d_kernel"); if (scaled) copy2d_kernel<true><<<blocks, 256, 0, st>>>(js);
+      else copy2d_kernel<false><<<blocks, 256, 0, st>>>(js); }
     return check_launch("copy2d_kernel");
   }
 };
@@ -1562,7 +1596,8 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
                            const int8_t* q, const float* scales, const void* A, const void* B,
                            int64_t M, int64_t K, int64_t N, int64_t r, float lora_scale, void* dx,
                            float* dA, float* dB, float* dbias, void* workspace, size_t ws_bytes,
-                           void* stream, const void* gx = nullptr, int64_t* gelu_rows = nullptr) {
+                           void* stream, const void* gx = nullptr, int64_t* gelu_rows = nullptr,
+                           const void* dys_given = nullptr) {
   clear_error();
   if (M < 0 || K <= 0 || N <= 0 || r < 0 || r > 4096)
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": " "need M >= 0, K > 0, N > 0, 0 <= r <= 4096");
@@ -1607,6 +1642,8 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
                                       "reels_hip_i8lora_workspace_bytes(..., REELS_HIP_WS_BWD)");
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   const uint16_t* dyb = static_cast<const uint16_t*>(dy);
+  // what dX multiplies with the weight (a padded call: dy times the scales; u and the gradients take dy)
+  const uint16_t* dyx = dys_given ? static_cast<const uint16_t*>(dys_given) : dyb;
   const uint16_t* xb = static_cast<const uint16_t*>(x);
   const uint16_t* Ab = static_cast<const uint16_t*>(A);
   const uint16_t* Bb = static_cast<const uint16_t*>(B);
@@ -1663,7 +1700,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
     if ((rc = launch_skinny(1, elt, p.cb, dyb, q, K, scales, r > 0 ? Bb : nullptr,
                             reinterpret_cast<float*>(ws + w.wd), M, N, K, (int)r, p.rp, nullptr,
                             Ar, p.rp, nullptr, lora_scale, static_cast<uint16_t*>(dx),
-                            r > 0 ? u : nullptr, p.rp, p.rp, st)))
+                            r > 0 ? u : nullptr, p.rp, p.rp, st, false, dyx)))
       return rc;
   } else if (p.cb > 0) {
     if (r > 0 && dA &&
@@ -1680,7 +1717,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
       uint16_t* wt = reinterpret_cast<uint16_t*>(ws + w.wd);
       if ((rc = launch_dequant_transpose(elt, q, K, scales, N, K, wt, st))) return rc;
       GemmArgs g{};
-      g.act = dyb; g.q = nullptr; g.colscale = nullptr; g.L = r > 0 ? u : nullptr; g.R = Ar;
+      g.act = dyx; g.q = nullptr; g.colscale = nullptr; g.L = r > 0 ? u : nullptr; g.R = Ar;
       g.bias = nullptr; g.out = static_cast<uint16_t*>(dx);
       g.M = M; g.Ncols = K; g.Kred = N; g.ldq = N; g.rp = r > 0 ? p.rp : 0; g.c = lora_scale;
       g.ksplit = p.ksb; g.part = reinterpret_cast<float*>(ws + w.kp);
@@ -1690,7 +1727,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
       if (g.gx && gelu_rows) *gelu_rows = g.M;
       if ((rc = launch_bfgemm(1, elt, g, wt, st))) return rc;
       if (p.tb > 0 &&  // the tokens past the whole rounds: the same weight and the same u
-          (rc = launch_skinny_tail(1, elt, p.tb, dyb + p.mb * N, q, K, scales, r > 0 ? u + p.mb * p.rp : nullptr,
+          (rc = launch_skinny_tail(1, elt, p.tb, dyx + p.mb * N, q, K, scales, r > 0 ? u + p.mb * p.rp : nullptr,
                                    M - p.mb, N, K, (int)r, p.rp, Ar, p.rp, nullptr, lora_scale,
                                    static_cast<uint16_t*>(dx) + p.mb * K, st)))
         return rc;
@@ -1802,11 +1839,16 @@ static int padded_bwd(int elt, const char* fn, const PadLayout& w, const void* d
   const int64_t Kp = w.Kp, Np = w.Np, rp = w.rp;
   Copies in, out;
   in.add(q, N, K, K, ws + w.q, Np, Kp, Kp, 1);
-  in.add(scales, 1, N, N, ws + w.s, 1, Np, Np, 4);
+  // bf16: the codes are multiplied by rnd(dy s), not rnd(q s) by dy
+  void* dys = dx && elt == REELS_HIP_BF16 ? ws + w.dys : nullptr;
+  if (dys) in.add(nullptr, 1, Np, Np, ws + w.s, 1, Np, Np, 4);
+  else in.add(scales, 1, N, N, ws + w.s, 1, Np, Np, 4);
   const void *dyp = dy, *xp = x, *hp = h, *Ap = A, *Bp = B;
   void* dxp = dx;
   float *dAp = dA, *dBp = dB, *dbp = dbias;
-  if (Np != N || !aligned16(dy)) { in.add(dy, M, N, N, ws + w.dy, M, Np, Np, 2); dyp = ws + w.dy; }
+  const bool copy_dy = Np != N || !aligned16(dy);
+  if (copy_dy) dyp = ws + w.dy;
+  if (copy_dy || dys) in.add(dy, M, N, N, copy_dy ? ws + w.dy : nullptr, M, Np, Np, 2, dys ? scales : nullptr, dys);
   // x is read for dA and to recompute h only
   const bool need_x = x && r > 0 && (dA || (dB && !h));
   if (need_x && (Kp != K || !aligned16(x))) { in.add(x, M, K, K, ws + w.x, M, Kp, Kp, 2); xp = ws + w.x; }
@@ -1834,7 +1876,8 @@ static int padded_bwd(int elt, const char* fn, const PadLayout& w, const void* d
   if (int rc = in.launch(st)) return rc;
   if (int rc = i8lora_bwd_impl(elt, fn, dyp, xp, hp, reinterpret_cast<const int8_t*>(ws + w.q),
                                reinterpret_cast<const float*>(ws + w.s), Ap, Bp, M, Kp, Np, rp,
-                               lora_scale, dxp, dAp, dBp, dbp, ws + w.inner, ws_bytes - w.inner, stream))
+                               lora_scale, dxp, dAp, dBp, dbp, ws + w.inner, ws_bytes - w.inner, stream,
+                               nullptr, nullptr, dys))
     return rc;
   return out.launch(st);
 }

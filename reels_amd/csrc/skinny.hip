@@ -55,7 +55,8 @@ constexpr uint32_t kSpinLimit = 1u << 12;  // wait rounds of s_sleep 8 (about 1 
 }  // namespace sk
 
 struct SkArgs {
-  const uint16_t* act;  // [M][Kred] 16-bit: x (FWD) or dy (DX)
+  const uint16_t* act;  // [M][Kred] 16-bit: x (FWD) or dy (DX), for l
+  const uint16_t* oact; // the same for out (act, or dy in another scaling)
   const int8_t* q;      // codes [N][K], row stride ldq
   const float* s;       // DX: scale of the reduction index n; FWD with rounded weights: of the output row
   const uint16_t* lw;   // adapter operand: FWD A [Kred][rp] (zeros past r), DX B [r][Kred]
@@ -173,7 +174,7 @@ __device__ __forceinline__ void skinny_acc(const SkArgs& a, int blk, int sp, int
   // Descriptors: reads past num_records return zeros (tokens past M, weight rows past the
   // matrix, adapter rows past the rank, chunks past the split).
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(a.act), (short)0, (int)(a.M * a.Kred * 2), 0x00020000);
+      const_cast<uint16_t*>(lora ? a.act : a.oact), (short)0, (int)(a.M * a.Kred * 2), 0x00020000);
   const int64_t wbytes = lora ? (MODE == 0 ? a.Kred * a.rp * 2 : (int64_t)a.r * a.Kred * 2)
                               : (MODE == 0 ? a.Ncols * a.ldq : a.Kred * a.ldq);
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
@@ -850,7 +851,7 @@ __device__ __forceinline__ void rw_acc_dma(const SkArgs& a, int64_t r0, int64_t 
   const int wr = w & 3, par = w >> 2;
   const int l16 = lane & 15, g = lane >> 4;
   const int nsteps = (int)(a.Kred / 128);
-  const i32x4 rx = buffer_rsrc(a.act, (uint32_t)(a.M * a.Kred * 2));
+  const i32x4 rx = buffer_rsrc(a.oact, (uint32_t)(a.M * a.Kred * 2));
   const i32x4 rq = buffer_rsrc(a.q, (uint32_t)((MODE == 0 ? a.Ncols : a.Kred) * a.ldq));
   // DX: wave 0's lanes 0-31 copy a step's 128 scales (lanes 32-63 read zeros past the descriptor)
   const i32x4 rs = buffer_rsrc(a.s, (uint32_t)(MODE == 1 ? a.Kred * 4 : 0));
@@ -1473,9 +1474,9 @@ static int launch_skinny_once(int mode, int elt, const SkinnyPlan& p, const uint
                               int64_t Kred, int64_t Ncols, int r, int rp, const float* colscale,
                               const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,
                               uint16_t* lsave, int64_t ld_lsave, int lsave_cols, hipStream_t st,
-                              bool adapter_only) {
+                              bool adapter_only, const uint16_t* oact) {
   SkArgs a{};
-  a.act = act; a.q = q; a.s = s; a.lw = lw;
+  a.act = act; a.oact = oact; a.q = q; a.s = s; a.lw = lw;
   a.M = M; a.Kred = Kred; a.Ncols = Ncols; a.ldq = ldq;
   a.r = r; a.rp = r > 0 ? rp : 0; a.S = p.S;
   a.nblk = (int)(Ncols / sk::NB);
@@ -1536,14 +1537,15 @@ int launch_skinny(int mode, int elt, int64_t chunk, const uint16_t* act, const i
                   int64_t Kred, int64_t Ncols, int r, int rp, const float* colscale,
                   const uint16_t* R, int64_t ldr, const uint16_t* bias, float c, uint16_t* out,
                   uint16_t* lsave, int64_t ld_lsave, int lsave_cols, hipStream_t st,
-                  bool adapter_only) {
+                  bool adapter_only, const uint16_t* oact) {
+  if (oact == nullptr) oact = act;
   for (int64_t m0 = 0; m0 < M; m0 += chunk) {
     const int64_t m = std::min(chunk, M - m0);
     const SkinnyPlan p = skinny_plan(m, Kred, Ncols, r > 0 ? rp : 0, mode);
     if (int rc = launch_skinny_once(mode, elt, p, act + m0 * Kred, q, ldq, s, lw, ws, m, Kred, Ncols, r, rp,
                                     colscale, R, ldr, bias, c, out ? out + m0 * Ncols : nullptr,
                                     lsave ? lsave + m0 * ld_lsave : nullptr, ld_lsave, lsave_cols, st,
-                                    adapter_only))
+                                    adapter_only, oact + m0 * Kred))
       return rc;
   }
   return REELS_HIP_OK;
@@ -1558,7 +1560,7 @@ int launch_skinny_tail(int mode, int elt, int64_t chunk, const uint16_t* act, co
     SkinnyPlan p;
     if (!rw_choose(m, Kred, Ncols, 0, mode, p)) return fail(REELS_HIP_EINVAL, "skinny_tail: shape not supported");
     SkArgs a{};
-    a.act = act + m0 * Kred; a.q = q; a.s = s; a.M = m; a.Kred = Kred; a.Ncols = Ncols; a.ldq = ldq;
+    a.act = a.oact = act + m0 * Kred; a.q = q; a.s = s; a.M = m; a.Kred = Kred; a.Ncols = Ncols; a.ldq = ldq;
     a.r = r; a.rp = r > 0 ? rp : 0; a.S = 1;
     a.nblk = (int)(Ncols / sk::NB); a.tb = p.tb;
     a.R = R; a.ldr = ldr; a.bias = bias; a.c = c; a.out = out + m0 * Ncols;

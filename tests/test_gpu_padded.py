@@ -119,3 +119,40 @@ def test_padded_noalloc_forward(dev, M, K, N, r):
     rows = np.unique(np.linspace(0, M - 1, 40).astype(int))
     yo, _ = oracle.lora_forward(cs["x"][rows], cs["q"], cs["s"], cs["A"], cs["B"], 1.0, cs["bias"])
     assert_parity(bf16_f32(y)[rows], yo, "noalloc y")
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("M,K,N,r", [
+    (777, 1000, 3000, 8),   # row-wave launches
+    (65, 300, 127, 0),      # the few-token path
+    (9000, 1000, 500, 16),  # the GEMM
+    (1500, 130, 1111, 4),   # its split reduction
+])
+def test_padded_dx_rounding_points(dev, M, K, N, r, f16):
+    """dX of widths that are no multiples of 64 multiplies bf16(dy s) and the exact codes (f16: dy and
+    f16(q f16(s))). With one nonzero per row of dy a sum has one term, so dx is that product rounded
+    once, bit for bit; dA takes u from dy itself."""
+    import torch
+    from reels_amd import QuantizedMatrix, i8lora_backward
+    print(f"[padded] rounding points M={M} K={K} N={N} r={r} f16={f16}", flush=True)
+    cs = _case(M, K, N, r, 1200 + M + K + N + r, f16)
+    x, A, B, dy = (_dev(cs[k], dev, f16) for k in ("x", "A", "B", "dy"))
+    hot = torch.arange(M, device=dev) * 7 % N
+    keep = torch.zeros((M, N), dtype=torch.bool, device=dev)
+    keep[torch.arange(M, device=dev), hot] = True
+    dy = torch.where(keep, dy, torch.zeros_like(dy))
+    q, s = to_dev(cs["q"], dev, "raw"), to_dev(cs["s"], dev, "raw")
+    A0 = torch.zeros_like(A) if r else None
+    dx = i8lora_backward(dy, x, QuantizedMatrix(q, s), A0, B, 1.0)[0]
+    d = dy[torch.arange(M, device=dev), hot].float()
+    if f16:
+        w = (q.half() * s.half()[:, None])[hot].double()
+        want = (d.double()[:, None] * w).to(torch.float32).half()
+    else:
+        ds = (d * s[hot]).bfloat16().float()
+        want = (ds[:, None] * q[hot].float()).bfloat16()
+    assert torch.equal(dx, want)
+    if r:
+        _, dA, _ = i8lora_backward(dy, x, QuantizedMatrix(q, s), A, B, 1.0)
+        u = (dy.double() @ B.double().t()).to(dy.dtype).double()
+        assert_parity(dA.cpu().numpy(), (x.double().t() @ u).cpu().numpy(), "dA")
