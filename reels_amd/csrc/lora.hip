@@ -1478,8 +1478,9 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
                            int64_t M, int64_t K, int64_t N, int64_t r, float lora_scale, void* y,
                            void* h_save, void* workspace, size_t ws_bytes, void* stream,
                            bool noalloc = false, void* gout = nullptr, int64_t* gelu_rows = nullptr,
-                           bool codes = false) {
+                           bool codes = false, int rank = -1) {
   clear_error();
+  const int rl = rank >= 0 ? rank : (int)r;  // a padded call's own rank: h is zero past it
   if (M < 0 || K <= 0 || N <= 0 || r < 0 || r > 4096)
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": " "need M >= 0, K > 0, N > 0, 0 <= r <= 4096");
   if (!(lora_scale == lora_scale))
@@ -1535,7 +1536,7 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
       Ap = ap;
     }
     return launch_skinny(0, elt, p.cf, xb, q, K, nullptr, r > 0 ? Ap : nullptr,
-                         reinterpret_cast<float*>(ws + w.pa), M, K, N, (int)r, p.rp, scales,
+                         reinterpret_cast<float*>(ws + w.pa), M, K, N, rl, p.rp, scales,
                          static_cast<const uint16_t*>(B), N, static_cast<const uint16_t*>(bias),
                          lora_scale, static_cast<uint16_t*>(y), static_cast<uint16_t*>(h_save), r,
                          (int)r, st);
@@ -1563,7 +1564,7 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
     const TpJob ja = tp_job(static_cast<const uint16_t*>(A), K, r, K, at);
     const TpJob jb = tp_job(static_cast<const uint16_t*>(B), r, N, p.rp, bt);
     if ((rc = launch_transpose_pad(ja, &jb, st))) return rc;
-    if ((rc = launch_rowproj(elt, xb, M, K, at, (int)r, p.rp, h, nullptr, nullptr, st,
+    if ((rc = launch_rowproj(elt, xb, M, K, at, rl, p.rp, h, nullptr, nullptr, st,
                              reinterpret_cast<float*>(ws + w.rq)))) return rc;
     if (p.padded && h_save &&
         (rc = launch_pad_cols(h, M, (int)r, p.rp, static_cast<uint16_t*>(h_save), (int)r, r, st)))
@@ -1585,7 +1586,7 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
     if ((rc = launch_bfgemm(0, elt, g, wd, st)) || p.tf == 0) return rc;
     // the tokens past the whole rounds: the same weight rnd(q s) and the same h
     return launch_skinny_tail(0, elt, p.tf, xb + p.mf * K, q, K, scales, r > 0 ? h + p.mf * p.rp : nullptr,
-                              M - p.mf, K, N, (int)r, p.rp, static_cast<const uint16_t*>(B), N,
+                              M - p.mf, K, N, rl, p.rp, static_cast<const uint16_t*>(B), N,
                               static_cast<const uint16_t*>(bias), lora_scale,
                               static_cast<uint16_t*>(y) + p.mf * N, st);
   }
@@ -1597,8 +1598,9 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
                            int64_t M, int64_t K, int64_t N, int64_t r, float lora_scale, void* dx,
                            float* dA, float* dB, float* dbias, void* workspace, size_t ws_bytes,
                            void* stream, const void* gx = nullptr, int64_t* gelu_rows = nullptr,
-                           const void* dys_given = nullptr) {
+                           const void* dys_given = nullptr, int rank = -1) {
   clear_error();
+  const int rl = rank >= 0 ? rank : (int)r;  // a padded call's own rank: h and u are zero past it
   if (M < 0 || K <= 0 || N <= 0 || r < 0 || r > 4096)
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": " "need M >= 0, K > 0, N > 0, 0 <= r <= 4096");
   if (!(lora_scale == lora_scale))
@@ -1698,19 +1700,19 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
     // few tokens: dx and u = rnd(dy B^T) from one launch over the int8 codes (u lands in the
     // workspace for the dA pass)
     if ((rc = launch_skinny(1, elt, p.cb, dyb, q, K, scales, r > 0 ? Bb : nullptr,
-                            reinterpret_cast<float*>(ws + w.wd), M, N, K, (int)r, p.rp, nullptr,
+                            reinterpret_cast<float*>(ws + w.wd), M, N, K, rl, p.rp, nullptr,
                             Ar, p.rp, nullptr, lora_scale, static_cast<uint16_t*>(dx),
                             r > 0 ? u : nullptr, p.rp, p.rp, st, false, dyx)))
       return rc;
   } else if (p.cb > 0) {
     if (r > 0 && dA &&
-        (rc = launch_rowproj(elt, dyb, M, N, Bb, (int)r, p.rp, u, nullptr, nullptr, st,
+        (rc = launch_rowproj(elt, dyb, M, N, Bb, rl, p.rp, u, nullptr, nullptr, st,
                              p.few ? nullptr : reinterpret_cast<float*>(ws + w.rq))))
       return rc;
   } else if (p.deq) {
     // 1. u = dy B^T; 2. dx = dy wt^T + c u A^T with wt[k][n] = bf16(q[n][k] s[n])
     if (r > 0 && (dx || dA)) {
-      if ((rc = launch_rowproj(elt, dyb, M, N, Bb, (int)r, p.rp, u, nullptr, nullptr, st,
+      if ((rc = launch_rowproj(elt, dyb, M, N, Bb, rl, p.rp, u, nullptr, nullptr, st,
                                reinterpret_cast<float*>(ws + w.rq)))) return rc;
     }
     if (dx) {
@@ -1728,7 +1730,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
       if ((rc = launch_bfgemm(1, elt, g, wt, st))) return rc;
       if (p.tb > 0 &&  // the tokens past the whole rounds: the same weight and the same u
           (rc = launch_skinny_tail(1, elt, p.tb, dyx + p.mb * N, q, K, scales, r > 0 ? u + p.mb * p.rp : nullptr,
-                                   M - p.mb, N, K, (int)r, p.rp, Ar, p.rp, nullptr, lora_scale,
+                                   M - p.mb, N, K, rl, p.rp, Ar, p.rp, nullptr, lora_scale,
                                    static_cast<uint16_t*>(dx) + p.mb * K, st)))
         return rc;
     }
@@ -1766,7 +1768,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
         Ap = ap;
       }
       if ((rc = launch_skinny(0, elt, p.cf, xb, q, K, nullptr, Ap, reinterpret_cast<float*>(ws + w.wd),
-                              M, K, N, (int)r, p.rp, nullptr, nullptr, N, nullptr, lora_scale, nullptr,
+                              M, K, N, rl, p.rp, nullptr, nullptr, N, nullptr, lora_scale, nullptr,
                               hw, p.rp, p.rp, st, true)))
         return rc;
       hh = hw;
@@ -1775,7 +1777,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
       uint16_t* at = reinterpret_cast<uint16_t*>(ws + w.at);
       uint16_t* hw = reinterpret_cast<uint16_t*>(ws + w.h);
       if ((rc = launch_transpose_pad(tp_job(Ab, K, r, K, at), nullptr, st))) return rc;
-      if ((rc = launch_rowproj(elt, xb, M, K, at, (int)r, p.rp, hw, nullptr, nullptr, st,
+      if ((rc = launch_rowproj(elt, xb, M, K, at, rl, p.rp, hw, nullptr, nullptr, st,
                                reinterpret_cast<float*>(ws + w.rq)))) return rc;
       hh = hw;
     }
@@ -1825,7 +1827,7 @@ static int padded_fwd(int elt, const char* fn, const PadLayout& w, const void* x
   if (int rc = i8lora_fwd_impl(elt, fn, xp, reinterpret_cast<const int8_t*>(ws + w.q),
                                reinterpret_cast<const float*>(ws + w.s), Ap, Bp, bp, M, Kp, Np, rp,
                                lora_scale, yp, hp, ws + w.inner, ws_bytes - w.inner, stream, false,
-                               nullptr, nullptr, true))
+                               nullptr, nullptr, true, (int)r))
     return rc;
   return out.launch(st);
 }
@@ -1877,7 +1879,7 @@ static int padded_bwd(int elt, const char* fn, const PadLayout& w, const void* d
   if (int rc = i8lora_bwd_impl(elt, fn, dyp, xp, hp, reinterpret_cast<const int8_t*>(ws + w.q),
                                reinterpret_cast<const float*>(ws + w.s), Ap, Bp, M, Kp, Np, rp,
                                lora_scale, dxp, dAp, dBp, dbp, ws + w.inner, ws_bytes - w.inner, stream,
-                               nullptr, nullptr, dys))
+                               nullptr, nullptr, dys, (int)r))
     return rc;
   return out.launch(st);
 }

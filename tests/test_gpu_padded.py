@@ -156,3 +156,34 @@ def test_padded_dx_rounding_points(dev, M, K, N, r, f16):
         _, dA, _ = i8lora_backward(dy, x, QuantizedMatrix(q, s), A, B, 1.0)
         u = (dy.double() @ B.double().t()).to(dy.dtype).double()
         assert_parity(dA.cpu().numpy(), (x.double().t() @ u).cpu().numpy(), "dA")
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("M,K,N,r", [
+    (777, 1000, 3000, 3),   # row-wave launches
+    (20, 300, 127, 1),      # the few-token path
+    (9000, 1000, 500, 5),   # the GEMM
+])
+def test_padded_infinite_rows(dev, M, K, N, r, f16):
+    """An infinite x (dy) with positive codes, scales and adapters gives infinite y and h (dx) in its
+    own row and changes no other row: the padding of the rank adds nothing, also to infinities."""
+    import torch
+    from reels_amd import QuantizedMatrix, i8lora_backward, i8lora_forward
+    print(f"[padded] infinite rows M={M} K={K} N={N} r={r} f16={f16}", flush=True)
+    cs = _case(M, K, N, r, 1500 + M, f16)
+    x, A, B, dy = (_dev(cs[k], dev, f16) for k in ("x", "A", "B", "dy"))
+    W = QuantizedMatrix(to_dev(cs["q"], dev, "raw").abs().clamp(min=1), to_dev(cs["s"], dev, "raw"))
+    A, B = A.abs() + 0.01, B.abs() + 0.01
+
+    def run(x, dy):
+        y, h = i8lora_forward(x, W, A, B, None, 1.0, save_h=True)
+        return y, h, i8lora_backward(dy, x, W, A, B, 1.0, h=h)[0]
+    ref = run(x, dy)
+    bad = M // 2
+    x[bad, K - 1] = float("inf")
+    dy[bad, N - 1] = float("inf")
+    got = run(x, dy)
+    rest = torch.arange(M, device=dev) != bad
+    for name, a, b in zip(("y", "h", "dx"), ref, got):
+        assert bool(torch.isposinf(b[bad]).all()), name
+        assert torch.equal(a[rest], b[rest]), name
