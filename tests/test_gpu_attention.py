@@ -439,3 +439,50 @@ def test_attention_backward_writing_dq_over_q(dev, dt):
     ref = oracle.attention_backward(q, k, v, dy, elt=dt)
     for t, r in zip((tq, dk, dv), ref):
         assert_parity(_vals(_bits(t), dt), r, f"dq over q {dt}", tol=1e-5 if dt == "f32" else GTOL)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+def test_attention_generic_key_at_minus_infinity(dev, dt):
+    """A key of -Inf scores -+Inf by the sign of q's element, whatever q's low bits: probability zero or
+    no number. The queries it does not reach have the results of the other keys alone."""
+    from reels_amd import memory_efficient_attention
+    print(f"[case] generic attention, key at -Inf, {dt}", flush=True)
+    q, k, v, _ = _inputs(1, 70, 150, 2, 48, 79, dt)
+    tq, tk, tv = (_dev(a, dev, dt) for a in (q, k, v))
+    tk[0, 9, 0, 3] = -float("inf")
+    res = memory_efficient_attention(tq, tk, tv)
+    out, lse = res.output.float().cpu().numpy(), res.cache.logsumexp.cpu().numpy()
+    low = _vals(q, dt)[0, :, 0, 3] > 0
+    keep = np.arange(150) != 9
+    ro, rl = oracle.attention_forward(np.ascontiguousarray(q[:, :, :1]), np.ascontiguousarray(k[:, keep, :1]),
+                                      np.ascontiguousarray(v[:, keep, :1]), elt=dt)
+    assert np.isnan(out[0, ~low, 0]).all()
+    assert_parity(out[0, low, 0], ro[0, low, 0], f"key at -Inf {dt}", tol=1e-5 if dt == "f32" else 1e-2)
+    assert np.max(np.abs(lse[0, 0, low] - rl[0, 0, low])) <= 1e-5
+
+
+@pytest.mark.parametrize("Sq", [64])  # whole tiles of queries
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+def test_attention_generic_backward_key_at_minus_infinity(dev, dt, Sq):
+    """The backward with a key of -Inf that no query sees with any probability (q's element is positive
+    in all): dV and dK are those of the other keys, zero for that key; dQ is NaN in that element alone
+    (its dS of zero times the infinity) and that of the other keys elsewhere."""
+    from reels_amd import memory_efficient_attention, memory_efficient_attention_backward
+    print(f"[case] generic attention backward, key at -Inf, {dt} Sq={Sq}", flush=True)
+    q, k, v, dy = _inputs(1, Sq, 150, 2, 48, 80, dt)
+    tq, tk, tv, tdy = (_dev(a.copy(), dev, dt) for a in (q, k, v, dy))
+    tq[:, :, 0, 3] = tq[:, :, 0, 3].abs() + 0.5
+    tk[0, 9, 0, 3] = -float("inf")
+    res = memory_efficient_attention(tq, tk, tv)
+    got = [_vals(_bits(t), dt) for t in memory_efficient_attention_backward(tq, tk, tv, tdy, res.cache)]
+    keep = np.arange(150) != 9
+    ref = oracle.attention_backward(_bits(tq), np.ascontiguousarray(k[:, keep]),
+                                    np.ascontiguousarray(v[:, keep]), dy, elt=dt)
+    dq, dk, dv = (a[:, :, 0] for a in got)  # (key 9 is an ordinary one in head 1)
+    tol = 1e-5 if dt == "f32" else GTOL
+    assert np.isnan(dq[..., 3]).all()
+    rest = np.arange(48) != 3
+    assert_parity(dq[..., rest], ref[0][:, :, 0][..., rest], f"dq {dt}", tol=tol)
+    for a, r, name in ((dk, ref[1][:, :, 0], "dk"), (dv, ref[2][:, :, 0], "dv")):
+        assert not a[:, 9].any(), name
+        assert_parity(a[:, keep], r, f"{name} {dt}", tol=tol)
