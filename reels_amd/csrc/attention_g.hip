@@ -418,7 +418,9 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_fwd_kernel(AttgArgs a, int v
     // exp(-Inf - -Inf) = NaN there would only reach queries that see no key at all
     if (FIRST && __builtin_amdgcn_ballot_w64(bmax > m)) {
       const float nmax = fmaxf(m, wave_max16(bmax));
-      const float noff = nmax * a.ch;  // the exponents' offset: about the new maximum's exponent
+      // the exponents' offset: about the new maximum's exponent. It stays finite while a query has seen
+      // scores of -Inf alone, whose probabilities then come out as zero
+      const float noff = nmax == -INFINITY ? 0.0f : nmax * a.ch;
       const float ps = nmax == -INFINITY || m == -INFINITY ? (nmax == -INFINITY ? 1.0f : 0.0f) : exp2_f(off - noff);
       m = nmax;
       off = noff;

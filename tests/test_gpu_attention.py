@@ -486,3 +486,24 @@ def test_attention_generic_backward_key_at_minus_infinity(dev, dt, Sq):
     for a, r, name in ((dk, ref[1][:, :, 0], "dk"), (dv, ref[2][:, :, 0], "dv")):
         assert not a[:, 9].any(), name
         assert_parity(a[:, keep], r, f"{name} {dt}", tol=tol)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+def test_attention_generic_first_tile_at_minus_infinity(dev, dt):
+    """Queries whose first whole tile of keys scores -Inf (64 keys of -Inf, q's element positive) beside
+    queries of the same wave that meet a maximum there (element negative: +Inf, no number): the former
+    have the results of the keys that follow, whoever shares their wave."""
+    from reels_amd import memory_efficient_attention
+    print(f"[case] generic attention, first tile at -Inf, {dt}", flush=True)
+    q, k, v, _ = _inputs(1, 70, 150, 2, 48, 81, dt)
+    tq, tk, tv = (_dev(a.copy(), dev, dt) for a in (q, k, v))
+    tk[0, :64, 0, 3] = -float("inf")
+    tq[0, 0::2, 0, 3] = tq[0, 0::2, 0, 3].abs() + 0.5
+    tq[0, 1::2, 0, 3] = -tq[0, 1::2, 0, 3].abs() - 0.5
+    res = memory_efficient_attention(tq, tk, tv)
+    out, lse = _vals(_bits(res.output), dt)[0, :, 0], res.cache.logsumexp.cpu().numpy()[0, 0]
+    ro, rl = oracle.attention_forward(_bits(tq), np.ascontiguousarray(k[:, 64:]),
+                                      np.ascontiguousarray(v[:, 64:]), elt=dt)
+    assert np.isnan(out[1::2]).all()
+    assert_parity(out[0::2], ro[0, 0::2, 0], f"first tile at -Inf {dt}", tol=1e-5 if dt == "f32" else 1e-2)
+    assert np.max(np.abs(lse[0::2] - rl[0, 0, 0::2])) <= 1e-5
