@@ -461,7 +461,7 @@ def test_attention_generic_key_at_minus_infinity(dev, dt):
     assert np.max(np.abs(lse[0, 0, low] - rl[0, 0, low])) <= 1e-5
 
 
-@pytest.mark.parametrize("Sq", [64])  # whole tiles of queries
+@pytest.mark.parametrize("Sq", [64, 70])  # whole tiles of queries, and a partial one
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
 def test_attention_generic_backward_key_at_minus_infinity(dev, dt, Sq):
     """The backward with a key of -Inf that no query sees with any probability (q's element is positive
