@@ -139,6 +139,16 @@ __device__ __forceinline__ void split8_in(const float* x, u32x4 (&o)[NI]) {
   else parts(std::false_type{});
 }
 
+// dS: infinite where dY or V is (finite it stays below half of the range). As for input elements an Inf is
+// then all in the last part, so that it meets first parts only.
+__device__ __forceinline__ void split8_ds(const float* x, u32x4 (&o)[3]) {
+  float top = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(x[e]));
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(top == INFINITY) != 0, 0)) split8_in<3>(x, o);
+  else split8(x, o);
+}
+
 // 8 consecutive elements of a row: raw from memory, then as bf16 parts. Buffer loads, so rows and
 // elements past the end read zeros without a branch. VEC (rows 16-byte aligned, decided on the
 // host): 16-byte loads, of which D % 4 (f32) or D % 8 elements are never split; else one by one.
@@ -247,6 +257,41 @@ template <int ELT, int R, int DP, int NT> struct GTile {
     const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, q + 16 * PITCH));
     const u32x2 l = __builtin_bit_cast(u32x2, lo), h = __builtin_bit_cast(u32x2, hi);
     return u32x4{l[0], l[1], h[0], h[1]};
+  }
+};
+
+// The products of 32 rows of a tile, read transposed, with the parts b of P or dS, over the NDT 16-wide
+// blocks of the head dim in groups: run calls add(block, i + j, tile part i, b[j]) for the pairs of parts
+// i + j <= 2, smallest first; first loads the first group's fragments ahead of it.
+template <typename T, int NI, int NDT> struct GProducts {
+  static constexpr int G = NI == 1 ? 4 : 2;
+  u32x4 head[G][NI];
+  static __device__ __forceinline__ void load(const uint8_t* tile, int row, int l16, int d0, u32x4 (&f)[G][NI]) {
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+#pragma unroll
+      for (int q = 0; q < NI; ++q)
+        if (d0 + i < NDT) f[i][q] = T::frag_tr(tile, q, row, 16 * (d0 + i), l16);
+  }
+  __device__ __forceinline__ void first(const uint8_t* tile, int row, int l16) { load(tile, row, l16, 0, head); }
+  template <typename Add>
+  __device__ __forceinline__ void run(const uint8_t* tile, int row, int l16, const u32x4 (&b)[3], Add&& add) {
+    auto group = [&](int d0, const u32x4 (&f)[G][NI]) {
+#pragma unroll
+      for (int s = 2; s >= 0; --s)
+#pragma unroll
+        for (int q = 0; q < NI; ++q)
+#pragma unroll
+          for (int i = 0; i < G; ++i)
+            if (s - q >= 0 && d0 + i < NDT) add(d0 + i, s, f[i][q], b[s - q]);
+    };
+    group(0, head);
+#pragma unroll
+    for (int d0 = G; d0 < NDT; d0 += G) {
+      u32x4 f[G][NI];
+      load(tile, row, l16, d0, f);
+      group(d0, f);
+    }
   }
 };
 
@@ -563,9 +608,13 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dkdv_kernel(AttgArgs a, int 
   u32x4 kf[NKB][NI], vf[NKB][NI];
   attg_frags<ELT, DP>(rk, kj, g, D, vec, kf);
   attg_frags<ELT, DP>(rv, kj, g, D, vec, vf);
-  f32x4 dka[NDT], dva[NDT];
+  // 16-bit dY: an infinite element is (in) a first part, and times a low part of P (zero or negative) no
+  // number or of the other sign. dV's pairs of parts past the first have sums of their own, which count
+  // where the first pair's is finite. (The first part of P is zero only where P is.)
+  constexpr bool LOW = NI < 3;
+  f32x4 dka[NDT], dva[NDT], dvl[LOW ? NDT : 1];
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) dka[dt] = dva[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int dt = 0; dt < NDT; ++dt) dka[dt] = dva[dt] = dvl[LOW ? dt : 0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   // causal: queries before the workgroup's first key see none of its keys
   int64_t qstart = a.causal ? kb0 / QT * QT : 0, qend = Sq;
   if constexpr (SPLIT) {  // this workgroup's range of tiles
@@ -633,35 +682,29 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dkdv_kernel(AttgArgs a, int 
           ds[e] = in ? ds[e] : 0.0f;
         }
       }
+      // dV^T += dY^T P and dK^T += Q^T dS. dK's first fragments are on their way before the branch of
+      // split8_ds, which the compiler moves no load across
+      GProducts<T, NI, NDT> pr;
       u32x4 pb[3], db[3];
       split8(p, pb);
-      split8(ds, db);
-      constexpr int G = NI == 1 ? 4 : 2;
-#pragma unroll
-      for (int d0 = 0; d0 < NDT; d0 += G)
-#pragma unroll
-        for (int which = 0; which < 2; ++which) {
-          u32x4 tf[G][NI];
-#pragma unroll
-          for (int i = 0; i < G; ++i)
-#pragma unroll
-            for (int q = 0; q < NI; ++q)
-              if (d0 + i < NDT) tf[i][q] = T::frag_tr(which ? sq : sdy, q, qb + 4 * g, 16 * (d0 + i), l16);
-#pragma unroll
-          for (int s = 2; s >= 0; --s)
-#pragma unroll
-            for (int q = 0; q < NI; ++q)
-#pragma unroll
-              for (int i = 0; i < G; ++i)
-                if (s - q >= 0 && d0 + i < NDT) {
-                  if (which) dka[d0 + i] = mfma_bf(tf[i][q], db[s - q], dka[d0 + i]);
-                  else dva[d0 + i] = mfma_bf(tf[i][q], pb[s - q], dva[d0 + i]);
-                }
-        }
+      pr.first(sdy, qb + 4 * g, l16);
+      pr.run(sdy, qb + 4 * g, l16, pb, [&](int dt, int s, u32x4 t, u32x4 b) {
+        if (LOW && s > 0) dvl[LOW ? dt : 0] = mfma_bf(t, b, dvl[LOW ? dt : 0]);
+        else dva[dt] = mfma_bf(t, b, dva[dt]);
+      });
+      pr.first(sq, qb + 4 * g, l16);
+      split8_ds(ds, db);
+      pr.run(sq, qb + 4 * g, l16, db, [&](int dt, int, u32x4 t, u32x4 b) { dka[dt] = mfma_bf(t, b, dka[dt]); });
     }
   };
   attg_stream<T>(rq, rdy, qstart, qend, QT, D, vec, smem, w < NW / 2, step, extra);
   if (kj >= Sk) return;
+  if constexpr (LOW) {
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) dva[dt][v] = __builtin_isfinite(dva[dt][v]) ? dva[dt][v] + dvl[dt][v] : dva[dt][v];
+  }
   const int64_t ob = ((b * Sk + kj) * H + h) * D;
   if constexpr (SPLIT) {
     const int64_t plane = (int64_t)(gridDim.z / a.qsplits) * Sk * H * D;
@@ -763,25 +806,11 @@ __global__ __launch_bounds__(NW * 64, 2) void attng_dq_kernel(AttgArgs a, int ve
           ds[4 * u + v] = FULL || attg_visible<VM>(a, qi, kk, (mk[kb2 / 16 + u] >> (8 * v)) & 0xffu) ? x : 0.0f;
         }
       }
+      GProducts<T, NI, NDT> pr;
       u32x4 db[3];
-      split8(ds, db);
-      constexpr int G = NI == 1 ? 4 : 2;
-#pragma unroll
-      for (int d0 = 0; d0 < NDT; d0 += G) {
-        u32x4 tf[G][NI];
-#pragma unroll
-        for (int i = 0; i < G; ++i)
-#pragma unroll
-          for (int q = 0; q < NI; ++q)
-            if (d0 + i < NDT) tf[i][q] = T::frag_tr(sk, q, kb2 + 4 * g, 16 * (d0 + i), l16);
-#pragma unroll
-        for (int s = 2; s >= 0; --s)
-#pragma unroll
-          for (int q = 0; q < NI; ++q)
-#pragma unroll
-            for (int i = 0; i < G; ++i)
-              if (s - q >= 0 && d0 + i < NDT) dqa[d0 + i] = mfma_bf(tf[i][q], db[s - q], dqa[d0 + i]);
-      }
+      pr.first(sk, kb2 + 4 * g, l16);
+      split8_ds(ds, db);
+      pr.run(sk, kb2 + 4 * g, l16, db, [&](int dt, int, u32x4 t, u32x4 b) { dqa[dt] = mfma_bf(t, b, dqa[dt]); });
     }
   };
   attg_stream<T>(rk, rv, 0, kend, KT, D, vec, smem, w < NW / 2,

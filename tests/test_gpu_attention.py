@@ -507,3 +507,45 @@ def test_attention_generic_first_tile_at_minus_infinity(dev, dt):
     assert np.isnan(out[1::2]).all()
     assert_parity(out[0::2], ro[0, 0::2, 0], f"first tile at -Inf {dt}", tol=1e-5 if dt == "f32" else 1e-2)
     assert np.max(np.abs(lse[0::2] - rl[0, 0, 0::2])) <= 1e-5
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("Sq,Sk", [(70, 150), (600, 40)])  # the second with the queries split
+def test_attention_generic_backward_infinite_dy(dev, dt, Sq, Sk):
+    """One infinite element of dY: every gradient has the infinities, NaNs and finite values that the
+    formulas give in f64 (dV infinite in that element alone; dS of that query infinite or NaN by the
+    signs of V and of its output), and the finite ones their parity."""
+    from reels_amd import memory_efficient_attention, memory_efficient_attention_backward
+    D, qi, di = 48, 41, 7
+    print(f"[case] generic attention backward, infinite dY, {dt} {Sq}x{Sk}", flush=True)
+    q, k, v, dy = _inputs(1, Sq, Sk, 2, D, 83, dt)
+    tq, tk, tv, tdy = (_dev(a.copy(), dev, dt) for a in (q, k, v, dy))
+    tdy[0, qi, 1, di] = float("inf")
+    res = memory_efficient_attention(tq, tk, tv)
+    got = [_vals(_bits(t), dt).astype(np.float64) for t in
+           memory_efficient_attention_backward(tq, tk, tv, tdy, res.cache)]
+    f = lambda t: t.double().cpu().numpy()[0, :, 1]
+    Q, K, V, dY, O = (f(t) for t in (tq, tk, tv, tdy, res.output))
+    with np.errstate(invalid="ignore"):
+        sc = 1.0 / np.sqrt(D)
+        S = Q @ K.T * sc
+        P = np.exp(S - np.log(np.exp(S).sum(1, keepdims=True)))
+        dP, corr = np.zeros_like(P), (dY * O).sum(1, keepdims=True)
+        for d in range(D):  # (sums of products, term by term: no library's view of infinities)
+            dP += dY[:, d:d + 1] * V[:, d][None]
+        dS = P * (dP - corr)
+        ref = [np.zeros_like(Q), np.zeros_like(K), np.zeros_like(V)]
+        for j in range(Sk):
+            ref[0] += dS[:, j:j + 1] * K[j] * sc
+        for i in range(Sq):
+            ref[1] += dS[i][:, None] * Q[i] * sc
+            ref[2] += P[i][:, None] * dY[i]
+    assert np.isinf(ref[1]).any() and np.isposinf(ref[2][:, di]).all()
+    for name, a, r in zip(("dq", "dk", "dv"), got, ref):
+        a = a[0, :, 1]
+        fin = np.isfinite(r)
+        assert np.array_equal(np.isnan(a), np.isnan(r)), name
+        assert np.array_equal(a[~fin & ~np.isnan(r)], r[~fin & ~np.isnan(r)]), name
+        if fin.any():
+            assert_parity(a[fin], r[fin], f"{name} {dt}", tol=1e-5 if dt == "f32" else GTOL)
+        assert np.isfinite(got[0][0, :, 0]).all()
