@@ -7,10 +7,14 @@
 // the element type (the reference's own order: scores, softmax and P V in Float32), and only the
 // results are. The products run on bf16 MFMA with f32 sums: every f32 operand is taken apart into
 // three bf16 values that sum to it exactly (an f16 one into two, a bf16 one is itself), and a
-// product keeps the pairs of parts i, j with i + j <= 2; the pairs left out are below 2^-24 of the
-// product, with random sign. Six (f32) or three (P times a bf16 tensor) products at 16 times the
-// rate of fp32 MFMA, and the sums come out closer to 64 bits than a chain of v_mfma_f32_16x16x4_f32
-// (fewer roundings; small pairs are added before large ones or in accumulators of their own).
+// product keeps the pairs of parts i, j with i + j <= 2; the pairs left out are below 2^-25 of the
+// product, with random sign (parts are the nearest bf16 values: a second part is at most 2^-9, a third
+// 2^-18 of the element; with truncated first parts the pairs reached 2^-23). Six (f32) or three (P times
+// a bf16 tensor) products at 16 times the rate of fp32 MFMA, and from sums of two terms on they come out
+// closer to 64 bits than a chain of v_mfma_f32_16x16x4_f32 (fewer roundings; small pairs are added before
+// large ones or in accumulators of their own): dP of normal f32 data, rms error over the norms at head
+// dim 1, 2, 3: 2.60e-8, 1.84e-8, 1.54e-8 against 2.53e-8, 2.62e-8, 2.43e-8; at 128 (emulated) 3.2e-9
+// against 1.8e-8.
 // Deterministic: no atomics, fixed summation order.
 //
 // MFMA layouts (v_mfma_f32_16x16x32_bf16): lane l holds row l % 16 of A and of B with k = 8 (l / 16)
@@ -20,9 +24,9 @@
 // which are its own scores: no lane exchange. The transposed operand of that product is read from
 // the row-major LDS tile with ds_read_b64_tr_b16 in the same key order.
 //
-// Measured, forward / backward: 1560 tokens, 12 heads x 128, f32: 164 / 487 us (fp32 MFMA
-// with single-element LDS reads: 610 / 1556); 2 x 1024 tokens, 16 heads x 80, bf16: 56 /
-// 152 us (460 / 1143). The f32 kernels are bound by their MFMAs and LDS fragment reads (6 MFMAs
+// Measured, forward / backward: 1560 tokens, 12 heads x 128, f32: 148 / 425 us (fp32 MFMA
+// with single-element LDS reads: 610 / 1556); 2 x 1024 tokens, 16 heads x 80, bf16: 46 /
+// 115 us (460 / 1143). The f32 kernels are bound by their MFMAs and LDS fragment reads (6 MFMAs
 // per 3 fragments of 1 KiB), the 16-bit ones by the VALU work per score (exponential and split).
 #include <algorithm>
 #include <cmath>
@@ -101,10 +105,11 @@ __device__ __forceinline__ void split8(const float* x, u32x4 (&o)[3]) {
     o[2][d] = pk_bf16(ra - bf16_lo(m), rb - bf16_hi(m));
   }
 }
-// the same for input elements: the first part by truncation (no finite value overflows); NaN stays
-// NaN. Of three parts an Inf is all in the last, which is only multiplied by first parts (nonzero
-// unless the element is); of two it is in the first. That selection runs only where some lane of the
-// wave meets an Inf or NaN.
+// the same for input elements; NaN stays NaN. Of two parts (f16) the first is taken by truncation, so that
+// the second has the element's sign, and an Inf is in the first. Of three the first is the nearest bf16
+// value, or the truncated one where nearest would pass the end of the range, and an Inf is all in the
+// last, which is only multiplied by first parts (nonzero unless the element is). That selection runs
+// only where some lane of the wave meets an Inf, a NaN or such a value.
 template <int NI>
 __device__ __forceinline__ void split8_in(const float* x, u32x4 (&o)[NI]) {
   uint32_t top = 0u;  // largest magnitude pattern of the 8
@@ -122,11 +127,18 @@ __device__ __forceinline__ void split8_in(const float* x, u32x4 (&o)[NI]) {
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const float v = x[2 * d + e];
+        if (NI > 2 && !SP) continue;
         const bool inf = SP && __builtin_isinf(v);
         h[e] = NI > 2 && inf ? 0u : __float_as_uint(v) & 0xffff0000u;
         r[e] = NI > 2 || !inf ? v - __uint_as_float(h[e]) : 0.0f;
       }
-      o[0][d] = __builtin_amdgcn_perm(h[1], h[0], 0x07060302u);
+      if constexpr (NI > 2 && !SP) {
+        o[0][d] = pk_bf16(x[2 * d], x[2 * d + 1]);
+        r[0] = x[2 * d] - bf16_lo(o[0][d]);
+        r[1] = x[2 * d + 1] - bf16_hi(o[0][d]);
+      } else {
+        o[0][d] = __builtin_amdgcn_perm(h[1], h[0], 0x07060302u);
+      }
       if constexpr (NI == 2) o[1][d] = pk_bf16(r[0], r[1]);
       if constexpr (NI > 2) {
         const float m0 = SP && __builtin_isinf(r[0]) ? 0.0f : r[0], m1 = SP && __builtin_isinf(r[1]) ? 0.0f : r[1];
@@ -135,7 +147,7 @@ __device__ __forceinline__ void split8_in(const float* x, u32x4 (&o)[NI]) {
       }
     }
   };
-  if (__builtin_amdgcn_ballot_w64(top >= 0x7f800000u)) parts(std::true_type{});
+  if (__builtin_amdgcn_ballot_w64(top >= (NI > 2 ? 0x7f7f8000u : 0x7f800000u))) parts(std::true_type{});
   else parts(std::false_type{});
 }
 

@@ -549,3 +549,31 @@ def test_attention_generic_backward_infinite_dy(dev, dt, Sq, Sk):
         if fin.any():
             assert_parity(a[fin], r[fin], f"{name} {dt}", tol=1e-5 if dt == "f32" else GTOL)
         assert np.isfinite(got[0][0, :, 0]).all()
+
+
+@pytest.mark.parametrize("D", [1, 2, 3])
+def test_attention_generic_short_sums_keep_f32(dev, D):
+    """f32 products of one to three terms. With one key, q = 0 and k = (1, 0, ..) the probability is one
+    and dq = scale (dP - correction), dP = dY . v on the parts and the correction the f32 sum of the
+    rounded products, which is known: dP itself comes out. It is within 2^-24 (its rounding) + 2^-25
+    (the pairs of parts left out) of the norms' product, with several terms 2^-24 more (the rounding of
+    the first pairs' sum)."""
+    from reels_amd import memory_efficient_attention, memory_efficient_attention_backward
+    print(f"[case] generic attention, short sums D={D}", flush=True)
+    B, Sq, H = 1, 4096, 8
+    _, _, v, dy = _inputs(B, Sq, 1, H, D, 90 + D, "f32")
+    q, k = np.zeros_like(dy), np.zeros_like(v)
+    k[..., 0] = 1.0
+    tq, tk, tv, tdy = (_dev(a, dev, "f32") for a in (q, k, v, dy))
+    res = memory_efficient_attention(tq, tk, tv)
+    assert not res.cache.logsumexp.any()
+    dq = memory_efficient_attention_backward(tq, tk, tv, tdy, res.cache).q.cpu().numpy()[0, :, :, 0]
+    corr = (dy[0] * v[0]).astype(np.float32)  # [Sq][H][D] rounded products, summed as the lanes do
+    corr = corr[..., 0] if D == 1 else (corr[..., 0] + corr[..., 1] + (corr[..., 2] if D == 3 else 0)).astype(np.float32)
+    scale = np.float64(np.float32(1.0) / np.sqrt(np.float32(D)))
+    dp = dq.astype(np.float64) / scale + corr
+    exact = (dy[0].astype(np.float64) * v[0]).sum(-1)
+    norms = np.sqrt((dy[0].astype(np.float64) ** 2).sum(-1) * (v[0].astype(np.float64) ** 2).sum(-1))
+    e = np.abs(dp - exact) / norms
+    print(f"[parity] D={D}: rms {np.sqrt((e ** 2).mean()):.2e} max {e.max():.2e}", flush=True)
+    assert e.max() <= (1.5 if D == 1 else 2.5) * 2.0 ** -24
