@@ -561,18 +561,47 @@ constexpr int kRankChunk = 128;
 struct PlanF32 {
   bool fast;
   int64_t Kp, Np;        // reduction lengths padded to the GEMM's step of 64
-  int64_t chf, chb;      // tokens per chunk (forward over K, dX over N): planes below 2^31 bytes
-  int ksf, ksb;          // reduction splits of the two GEMMs
+  int64_t chf, chb;      // tokens per chunk (forward over K, dX over N)
   int psf, psb;          // column splits of the projections over K and N
   int64_t tpsa, tpsb;    // tokens per split of dA (columns K) and dB (columns N)
   int spa, spb;
 };
 
-// tokens per chunk: the GEMM's copies address the planes with 32-bit offsets; chunks of equal size
-static int64_t plane_chunk(int64_t M, int64_t Kp) {
-  const int64_t most = ((((int64_t)1 << 31) - 1) / (6 * Kp)) / 256 * 256;
-  const int64_t n = ceil_div(M, most > 0 ? most : 1);
-  return n > 0 ? ceil_div(ceil_div(M, n), 256) * 256 : 256;
+// Tokens per chunk. The planes of one chunk take up to kPlaneBytes of the workspace (the GEMM's copies
+// would address up to 2 GiB), so that a call needs no more than that beside the 16-bit weight copy. Longer
+// calls run as chunks of as many 256-row tiles as give the least time: rounds of 256 x 256 tiles over the
+// CUs at 2.4 us per 64-deep step and 4 for the epilogue, split partials at 5 TB/s, 3 us per chunk.
+// Forward / backward and forward workspace, one chunk of up to 2 GiB against chunks: 32760 tokens on 5120 x
+// 5120 4036 / 4297 us, 1015 MiB -> 4127 / 4400, 303; 16384 on 3072 x 3072 781 / 859, 307 -> 835 / 940,
+// 162; 32760 on 8960 -> 1536 2476 / 2598, 1711 -> 2762 / 2640, 345; 9360 there 791 / 841 -> 795 / 842.
+constexpr int64_t kPlaneBytes = (int64_t)256 << 20;
+static int64_t plane_chunk(int64_t M, int64_t Kp, int64_t Ncols) {
+  const int64_t most = std::max<int64_t>(kPlaneBytes / (6 * Kp) / 256, 1), tm = ceil_div(M, 256);
+  if (tm <= most) return std::max<int64_t>(tm, 1) * 256;
+  const int64_t tn = ceil_div(Ncols, 256);
+  const double round = 2.4 * (double)(Kp / 64) + 4.0;
+  auto chunk_us = [&](int64_t rows) {
+    if (rows == 0) return 0.0;
+    const int64_t ks = planegemm_splits(rows * 256, Ncols, Kp);
+    return 3.0 + round * (double)ceil_div(rows * tn * ks, 256) / (double)ks +
+           (ks > 1 ? (double)(2 * ks * rows * 256 * Ncols * 4) / 5e6 : 0.0);
+  };
+  int64_t best = most;
+  double tbest = 1e300;
+  for (int64_t t = most; t > most / 4; --t) {
+    const double time = (double)(tm / t) * chunk_us(t) + chunk_us(tm % t);
+    if (time < tbest) { tbest = time; best = t; }
+  }
+  return best * 256;
+}
+// most bytes of split partials of a chunk: the last, shorter one has a split of its own
+static size_t plane_partials(int64_t M, int64_t chunk, int64_t Kp, int64_t Ncols) {
+  size_t most = 0;
+  for (int64_t m : {std::min(M, chunk), M % chunk}) {
+    const int64_t ks = m > 0 ? planegemm_splits(m, Ncols, Kp) : 1;
+    if (ks > 1) most = std::max(most, (size_t)(ks * m * ((Ncols + 3) / 4 * 16)));
+  }
+  return most;
 }
 // column splits of a projection: 32-row blocks, about 512 of them (two per CU)
 static int project_splits(int64_t M, int64_t Kp) {
@@ -597,10 +626,8 @@ static PlanF32 plan_f32(int64_t M, int64_t K, int64_t N, int64_t r, bool aligned
   p.fast = aligned && K > 0 && N > 0 && p.Kp <= (1 << 20) && p.Np <= (1 << 20) &&
            p.Kp * p.Np * 2 < ((int64_t)1 << 31);
   if (!p.fast) return p;
-  p.chf = plane_chunk(M, p.Kp);
-  p.chb = plane_chunk(M, p.Np);
-  p.ksf = planegemm_splits(std::min(M, p.chf), N, p.Kp);
-  p.ksb = planegemm_splits(std::min(M, p.chb), K, p.Np);
+  p.chf = plane_chunk(M, p.Kp, N);
+  p.chb = plane_chunk(M, p.Np, K);
   p.psf = project_splits(std::min(M, p.chf), p.Kp);
   p.psb = project_splits(std::min(M, p.chb), p.Np);
   colgrad_split(M, K, r, p.tpsa, p.spa);
@@ -624,8 +651,7 @@ static WsF32 ws_f32(int64_t M, int64_t K, int64_t N, int64_t r, int which, const
     w.wd = take((size_t)(fwd ? N * p.Kp : K * p.Np) * 2);
     w.mant = take((size_t)N * 4);
     w.planes = take((size_t)ch * 6 * (fwd ? p.Kp : p.Np));
-    const int ks = fwd ? p.ksf : p.ksb;
-    w.kp = take(ks > 1 ? (size_t)ks * ch * ((fwd ? N : K) + 3) / 4 * 16 : 0);
+    w.kp = take(fwd ? plane_partials(M, p.chf, p.Kp, N) : plane_partials(M, p.chb, p.Np, K));
     // split partials of the projections (the backward also recomputes h)
     const size_t rc = (size_t)std::min<int64_t>(r, kRankChunk);
     const size_t pf = p.psf > 1 ? (size_t)p.psf * std::min(M, p.chf) * rc * 4 : 0;
@@ -814,7 +840,7 @@ static int i8lora_fwd_f32_impl(const float* x, const int8_t* q, const float* sca
     g.act = planes; g.colscale = mant; g.fL = hc; g.fR = bt; g.fbias = bias; g.fout = y + m0 * N;
     g.M = mc; g.Ncols = N; g.Kred = p.Kp; g.fr = (int)r; g.c = c;
     g.fvout = N % 4 == 0;
-    g.ksplit = p.ksf; g.part = reinterpret_cast<float*>(ws + w.kp); g.ldp = (N + 3) / 4 * 4;
+    g.ksplit = planegemm_splits(mc, N, p.Kp); g.part = reinterpret_cast<float*>(ws + w.kp); g.ldp = (N + 3) / 4 * 4;
     if ((rc = launch_planegemm(0, g, wd, st))) return rc;
   }
   return REELS_HIP_OK;
@@ -906,7 +932,7 @@ static int i8lora_bwd_f32_impl(const char* fn, const float* dy, const float* x, 
       g.act = planes; g.fL = uc; g.fR = A; g.fout = dx + m0 * K;
       g.M = mc; g.Ncols = K; g.Kred = p.Np; g.fr = (int)r; g.c = c;
       g.fvout = K % 4 == 0;
-      g.ksplit = p.ksb; g.part = reinterpret_cast<float*>(ws + w.kp); g.ldp = (K + 3) / 4 * 4;
+      g.ksplit = planegemm_splits(mc, K, p.Np); g.part = reinterpret_cast<float*>(ws + w.kp); g.ldp = (K + 3) / 4 * 4;
       if ((rc = launch_planegemm(1, g, wt, st))) return rc;
     }
   }

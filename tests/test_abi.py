@@ -39,6 +39,19 @@ def test_header_constants_match_binding():
                                                          _lib.WS_FWD_NOALLOC)
 
 
+def test_f32_workspace_is_bounded():
+    """Beside the 16-bit weight copy and the rank panels the f32 calls hold at most 256 MiB of
+    activation planes (and 96 MiB of split partials), whatever the token count."""
+    L = _lib.lib()
+    for (M, K, N, r) in [(32760, 5120, 5120, 32), (32760, 8960, 1536, 32), (32760, 1536, 8960, 32),
+                         (200000, 5120, 13824, 64), (1000000, 256, 256, 16), (40200, 8960, 96, 8)]:
+        for which, w in ((0, K), (1, N)):
+            pad = (w + 63) // 64 * 64
+            small = 264 * (K + N + 64) * r + 12 * M * r + 264 * N  # adapters, h, u and the gradients' partials
+            b = L.reels_hip_i8lora_workspace_bytes_f32(M, K, N, r, which)
+            assert 0 < b <= 2 * (N if which == 0 else K) * pad + (352 << 20) + small, (M, K, N, r, which)
+
+
 def test_workspace_sizes():
     L = _lib.lib()
     for (M, K, N, r) in [(32760, 5120, 5120, 32), (1024, 1536, 1536, 16), (77, 5120, 5120, 32),

@@ -220,8 +220,8 @@ def test_f32_plane_gemm_edges(dev, M, K, N, r, bias):
 
 
 def test_f32_token_chunks(dev):
-    # 40200 tokens x 8960: the planes of x would exceed 2 GiB, so the forward runs as two chunks;
-    # rows on both sides of the boundary against f64 products, h in full
+    # 40200 tokens x 8960: the planes of x would exceed 2 GiB, so the forward runs as chunks; rows on
+    # both sides of multiples of 256 tokens against f64 products
     import torch
     from reels_amd import QuantizedMatrix, i8lora_forward
     M, K, N, r = 40200, 8960, 96, 8
@@ -271,3 +271,32 @@ def test_f32_special_values(dev):
     dy[1, 2], dy[2, 3] = np.inf, np.nan
     dx = i8lora_backward(todev(dy, dev), None, W, want_dA=False, want_dB=False)[0].cpu().numpy()
     assert np.isinf(dx[1]).all() and np.isnan(dx[2]).all() and np.isfinite(dx[[0, 3, 4]]).all()
+
+
+@pytest.mark.parametrize("M,K,N,r", [
+    (6000, 8960, 300, 8),    # the forward in chunks, the last a shorter one with a split of its own
+    (6000, 300, 8960, 24),   # dX in chunks
+])
+def test_f32_chunks_of_bounded_planes(dev, M, K, N, r):
+    """Calls whose planes would take more than 256 MiB run as chunks of their tokens: every output in
+    full against f64 products, h given and recomputed."""
+    import torch
+    from reels_amd import QuantizedMatrix, i8lora_backward, i8lora_forward
+    print(f"[f32] bounded planes {M}x{K}x{N}r{r}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    rn = lambda *sh: torch.randn(sh, generator=g, device=dev)
+    x, dy, A, B, bias = rn(M, K), rn(M, N), rn(K, r) * 0.01, rn(r, N) * 0.01, rn(N)
+    q = torch.randint(-127, 128, (N, K), generator=g, device=dev).to(torch.int8)
+    s = torch.rand((N,), generator=g, device=dev) * 1e-3
+    W = QuantizedMatrix(q, s, torch.float32)
+    y, h = i8lora_forward(x, W, A, B, bias, 0.5, save_h=True)
+    first = i8lora_backward(dy, x, W, A, B, 0.5, h=h)
+    again = i8lora_backward(dy, x, W, A, B, 0.5, h=None)
+    torch.cuda.synchronize(dev)
+    assert all(torch.equal(a, b) for a, b in zip(first, again))
+    Wd, xd, dyd, Ad, Bd = q.double() * s.double()[:, None], x.double(), dy.double(), A.double(), B.double()
+    hd, ud = xd @ Ad, dyd @ Bd.t()
+    ref = (xd @ Wd.t() + bias.double() + 0.5 * hd @ Bd, hd, dyd @ Wd + 0.5 * ud @ Ad.t(),
+           0.5 * xd.t() @ ud, 0.5 * hd.t() @ dyd)
+    for name, a, b in zip(("y", "h", "dx", "dA", "dB"), (y, h) + tuple(first), ref):
+        assert_parity(a.cpu().numpy(), b.cpu().numpy(), f"bounded planes {name}", tol=TOL)
