@@ -5,9 +5,9 @@ checked against the f64 oracle (elt="f32") on the same seeded float32 inputs.
 
 Tolerance: fp32 compute with f32 sums over at most 5120 terms keeps the error near 2^-24 times a
 small multiple of sqrt(K); the bar here is normwise and elementwise 1e-5 (tests/_util.assert_parity
-with tol=1e-5), a thousand times tighter than the bf16 bar. Covered: the fp32-MFMA GEMM (K, N
-multiples of 4, aligned), the fp32 projection and split-M gradient kernels, the generic kernels
-(K or N not a multiple of 4), and the mirror API with autograd."""
+with tol=1e-5), a thousand times tighter than the bf16 bar. Covered: the GEMM on bf16 planes (any
+widths, any 4-byte aligned operands, chunks of tokens), the fp32 projection and split-M gradient
+kernels, the generic kernels (a workspace off its alignment), and the mirror API with autograd."""
 import numpy as np
 import pytest
 
@@ -202,8 +202,9 @@ def test_f32_gelu_tanh(dev, n):
 ])
 def test_f32_plane_gemm_edges(dev, M, K, N, r, bias):
     """The products on bf16 planes at the edges of their tiles and steps: every output against the
-    oracle within the file's 1e-5 (the planes are exact, the sums f32), and the result of unaligned
-    (4-byte aligned) operands equal to that of aligned copies bit for bit."""
+    oracle within the file's 1e-5 (the planes are exact, the sums f32), and the result of an unaligned
+    (4-byte aligned) x equal to that of an aligned copy bit for bit (every operand:
+    test_f32_operands_off_their_alignment)."""
     import torch
     from reels_amd import QuantizedMatrix, i8lora_forward
     cs = make_case(M, K, N, r, float(r), seed=900 + M + K + N + r, bias=bias)
@@ -300,3 +301,79 @@ def test_f32_chunks_of_bounded_planes(dev, M, K, N, r):
            0.5 * xd.t() @ ud, 0.5 * hd.t() @ dyd)
     for name, a, b in zip(("y", "h", "dx", "dA", "dB"), (y, h) + tuple(first), ref):
         assert_parity(a.cpu().numpy(), b.cpu().numpy(), f"bounded planes {name}", tol=TOL)
+
+
+@pytest.mark.parametrize("M,K,N,r", [
+    (300, 320, 260, 4),    # the adapter tiles in LDS, rows of 16 bytes
+    (77, 130, 515, 24),    # split reductions, widths that are no multiples of 4
+    (2100, 256, 1000, 32),  # several token splits
+    (40, 200, 96, 40),     # ranks above the LDS tile
+])
+def test_f32_operands_off_their_alignment(dev, M, K, N, r):
+    """Every f32 operand and output one element (the codes one byte) past a 16-byte boundary: forward
+    with h and bias, backward with h given and recomputed and with the bias gradient, bit for bit as
+    with aligned ones."""
+    import ctypes
+    import torch
+    from reels_amd import _lib
+    L = _lib.lib()
+    print(f"[f32] unaligned {M}x{K}x{N}r{r}", flush=True)
+    cs = make_case(M, K, N, r, float(r), seed=1300 + M, bias=True)
+    dy = f32v(1301 + M, (M, N), 1.0)
+    st = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    nb = max(L.reels_hip_i8lora_workspace_bytes_f32(M, K, N, r, w) for w in (0, 1))
+    ws = torch.empty((nb,), dtype=torch.uint8, device=dev)
+    assert ws.data_ptr() % 256 == 0
+
+    def shifted(a, off):
+        flat = torch.empty((a.numel() + 16,), dtype=a.dtype, device=dev)[off:off + a.numel()]
+        return flat.copy_(a.reshape(-1)).view(a.shape)
+
+    def run(off):
+        x, A, B, bias, q, s, d = (shifted(todev(a, dev), off) for a in
+                                  (cs["x"], cs["A"], cs["B"], cs["bias"], cs["q"], cs["s"], dy))
+        y, h, dx, dA, dB, db = (shifted(torch.zeros(sh, device=dev), off) for sh in
+                                ((M, N), (M, r), (M, K), (K, r), (r, N), (N,)))
+        assert all((t.data_ptr() % 16 != 0) == (off > 0) for t in (x, A, B, bias, q, s, d, y, h, dx, dA, dB, db))
+        p = lambda t: ctypes.c_void_p(t.data_ptr())
+        _lib.check("fwd", L.reels_hip_i8lora_fwd_f32(
+            p(x), p(q), p(s), p(A), p(B), p(bias), M, K, N, r, 0.5, p(y), p(h), p(ws), nb, st))
+        out = [y, h]
+        for hp in (p(h), None):
+            _lib.check("bwd", L.reels_hip_i8lora_bwd_bias_f32(
+                p(d), p(x), hp, p(q), p(s), p(A), p(B), M, K, N, r, 0.5, p(dx), p(dA), p(dB), p(db), p(ws), nb, st))
+            out += [t.clone() for t in (dx, dA, dB, db)]
+        torch.cuda.synchronize(dev)
+        return out
+    names = ("y", "h") + 2 * ("dx", "dA", "dB", "dbias")
+    for name, a, b in zip(names, run(0), run(1)):
+        assert torch.equal(a, b), name
+
+
+def test_f32_generic_kernels(dev):
+    """A workspace off its 16-byte alignment: the one-output-per-thread kernels, against the oracle."""
+    import ctypes
+    import torch
+    from reels_amd import _lib
+    L = _lib.lib()
+    M, K, N, r = 33, 70, 50, 5
+    print("[f32] generic kernels", flush=True)
+    cs = make_case(M, K, N, r, float(r), seed=1400, bias=True)
+    x, A, B, bias, q, s, dy = (todev(cs[k], dev) for k in ("x", "A", "B", "bias", "q", "s", "dy"))
+    nb = max(L.reels_hip_i8lora_workspace_bytes_f32(M, K, N, r, w) for w in (0, 1))
+    ws = torch.empty((nb + 16,), dtype=torch.uint8, device=dev)[4:4 + nb]
+    y, h, dx, dA, dB, db = (torch.zeros(sh, device=dev) for sh in ((M, N), (M, r), (M, K), (K, r), (r, N), (N,)))
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    st = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    c = cs["c"]
+    _lib.check("fwd", L.reels_hip_i8lora_fwd_f32(
+        p(x), p(q), p(s), p(A), p(B), p(bias), M, K, N, r, c, p(y), p(h), p(ws), nb, st))
+    yo, ho = oracle.lora_forward(cs["x"], cs["q"], cs["s"], cs["A"], cs["B"], c, cs["bias"], elt="f32")
+    ref = oracle.lora_backward(cs["dy"], cs["x"], cs["q"], cs["s"], cs["A"], cs["B"], c, elt="f32")
+    for hp in (p(h), None):
+        _lib.check("bwd", L.reels_hip_i8lora_bwd_bias_f32(
+            p(dy), p(x), hp, p(q), p(s), p(A), p(B), M, K, N, r, c, p(dx), p(dA), p(dB), p(db), p(ws), nb, st))
+        torch.cuda.synchronize(dev)
+        for name, a, b in (("y", y, yo), ("h", h, ho), ("dx", dx, ref["dx"]), ("dA", dA, ref["dA"]),
+                           ("dB", dB, ref["dB"]), ("dbias", db, oracle.bias_gradient(cs["dy"], elt="f32"))):
+            assert_parity(a.cpu().numpy(), b, f"generic {name}", tol=TOL)
