@@ -1071,7 +1071,7 @@ static int64_t pad_width(int64_t M, int64_t d) {
 // backward for 777 tokens, 1000 -> 3000 (rank 8; the scaled copy of dy 1.5 us of it, 12 us of 342 for the
 // backward of 8192 tokens, 2064 -> 5136); the one-output-per-thread kernels took 11.0 ms there, and widths
 // that are multiples of 16 ran unsplit 256 x 256 tiles (1000 tokens, 528 -> 2064: 236 against 89 us).
-static bool pad_shape(int64_t M, int64_t K, int64_t N) {
+static bool pad_shape(int64_t M, int64_t K, int64_t N, int64_t r) {
   if (K % 64 == 0 && N % 64 == 0) return false;
   // tiny layers: the direct kernels' single launch is shorter than the copies' launches (one token,
   // 100 -> 100 forward 14 against 21 us; 64 tokens forward and backward 60 us either way; 256 tokens
@@ -1079,7 +1079,7 @@ static bool pad_shape(int64_t M, int64_t K, int64_t N) {
   if (M <= 64 && K <= 128 && N <= 128) return false;
   const int64_t Kp = pad_width(M, K), Np = pad_width(M, N), most = (int64_t)1 << 31;
   return Kp < ((int64_t)1 << 22) && Np < ((int64_t)1 << 22) && Kp * Np * 2 < most &&
-         M * std::max(Kp, Np) / 8 < most;  // the copies count their 16-byte pieces in 32 bits
+         M * std::max({Kp, Np, (r + 15) / 16 * 16}) / 8 < most;  // the copies count their 16-byte pieces in 32 bits
 }
 
 struct PadLayout {
@@ -1412,7 +1412,7 @@ extern "C" size_t reels_hip_i8lora_workspace_bytes(int64_t M, int64_t K, int64_t
     return 0;
   // sized for the fast layout when the shape allows it (pointer alignment cannot be known here;
   // the fast layout is never smaller than the generic one)
-  if (K > 0 && N > 0 && pad_shape(M, K, N)) {
+  if (K > 0 && N > 0 && pad_shape(M, K, N, r)) {
     const size_t t = pad_layout(M, K, N, r, which == REELS_HIP_WS_BWD ? which : REELS_HIP_WS_FWD).total;
     if (which != REELS_HIP_WS_FWD_NOALLOC || t <= kScratchBytes) return t;
   }
@@ -1488,7 +1488,7 @@ static int i8lora_fwd_impl(int elt, const char* fn, const void* x, const int8_t*
   if (M == 0) return REELS_HIP_OK;
   if (!x || !q || !scales || !y || (r > 0 && (!A || !B)))
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": " "NULL x, q, scales, y, or A/B with r > 0");
-  if (pad_shape(M, K, N)) {
+  if (pad_shape(M, K, N, r)) {
     const PadLayout w = pad_layout(M, K, N, r, REELS_HIP_WS_FWD);
     // without a workspace the padded copies have to fit the scratch; beyond it the direct kernels run
     if (!noalloc || w.total <= kScratchBytes) {
@@ -1627,7 +1627,7 @@ static int i8lora_bwd_impl(int elt, const char* fn, const void* dy, const void* 
     return fail(REELS_HIP_EINVAL, std::string(fn) + ": " "NULL dy, q, scales, A/B with r > 0, or x "
                                   "needed for dA / recomputing h");
   if (!dx && !dA && !dB && !dbias) return REELS_HIP_OK;
-  if (pad_shape(M, K, N)) {
+  if (pad_shape(M, K, N, r)) {
     const PadLayout w = pad_layout(M, K, N, r, REELS_HIP_WS_BWD);
     if (workspace == nullptr || ws_bytes < w.total)
       return fail(REELS_HIP_EWORKSPACE, std::string(fn) + ": " "workspace NULL or smaller than "

@@ -52,6 +52,15 @@ def test_f32_workspace_is_bounded():
             assert 0 < b <= 2 * (N if which == 0 else K) * pad + (352 << 20) + small, (M, K, N, r, which)
 
 
+def test_padded_copies_fit_their_piece_counts():
+    """The padded forms count the 16-byte pieces of a copy in 32 bits: a rank panel of 2^35 bytes and
+    more (16M tokens at rank 4096) leaves them, and the call holds one panel, not a padded second."""
+    L = _lib.lib()
+    M, r = 1 << 24, 4096
+    assert L.reels_hip_i8lora_workspace_bytes(M, 100, 100, r, _lib.WS_FWD) < 1.5 * M * r * 2
+    assert L.reels_hip_i8lora_workspace_bytes(M // 8, 100, 100, r, _lib.WS_FWD) > 1.5 * (M // 8) * r * 2
+
+
 def test_workspace_sizes():
     L = _lib.lib()
     for (M, K, N, r) in [(32760, 5120, 5120, 32), (1024, 1536, 1536, 16), (77, 5120, 5120, 32),
