@@ -921,22 +921,20 @@ def main():
         rs = recs[step * per_step:(step + 1) * per_step]
         fi = [ms for (n, ms) in rs if "gemm_kernel" in n and n.endswith("<0>")]
         bi = [ms for (n, ms) in rs if "gemm_kernel" in n and n.endswith("<1>")]
-        for (pr, ms) in zip(projs, fi):
-            gemm_ms["fwd"] += ms; gemm_n["fwd"] += 1
-            gemm_fl["fwd"] += gemm_flops("fwd", M, pr.K, pr.N, RANK)
-        for (pr, ms) in zip(reversed(projs), bi):
-            gemm_ms["dx"] += ms; gemm_n["dx"] += 1
-            gemm_fl["dx"] += gemm_flops("dx", M, pr.K, pr.N, RANK)
+        # (a projection's GEMM may run as several launches over token chunks: f32)
+        for d, ms in (("fwd", fi), ("dx", bi)):
+            gemm_ms[d] += sum(ms); gemm_n[d] += len(ms)
+            gemm_fl[d] += sum(gemm_flops(d, M, pr.K, pr.N, RANK) for pr in projs)
     tot_ms = gemm_ms["fwd"] + gemm_ms["dx"]
     achieved = (gemm_fl["fwd"] + gemm_fl["dx"]) / (tot_ms * 1e-3) / 1e12 if tot_ms > 0 else 0.0
     gemm_names = sorted({n for (n, _) in recs if "gemm_kernel" in n})
     vendor = vendor_gemm_tflops(dev, M, 5120, 5120, dtype=act)
-    deq = {"bf16": "bf16(q*s)", "f16": "f16(q*f16(s))",
-           "f32": "exact codes, f32 activations as three bf16 planes"}[args.dtype]
+    deq = {"bf16": "bf16 MFMA on the dequantized weight bf16(q*s)",
+           "f16": "f16 MFMA on the dequantized weight f16(q*f16(s))",
+           "f32": "bf16 MFMA on the exact codes, f32 activations as three bf16 planes"}[args.dtype]
     peak = PEAK_TFLOPS[args.dtype]
     roofline = {
-        "kernel": " + ".join(gemm_names) + f" (<0> fwd, <1> dX; {args.dtype} MFMA on the "
-                                           f"dequantized weight {deq})",
+        "kernel": " + ".join(gemm_names) + f" (<0> fwd, <1> dX; {deq})",
         "bound": "mfma", "achieved": round(achieved, 2), "peak": peak,
         "unit": "TFLOP/s", "frac": round(achieved / peak, 4),
         "traffic": GEMM_TRAFFIC_BYTES,
