@@ -98,17 +98,17 @@ size_t reels_hip_i8lora_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t
  * with W = bf16(fl32(q * s)) written into the workspace once per call when K and N are multiples
  * of 64 and there are many tokens (the reference's _materialize_weight, quantization.jl:54-64);
  * otherwise W = q * s exact with s[n] applied to the f32 sum: K or N not a multiple of 64 (on
- * zero-padded copies in the workspace), and the
- * few-token path (M <= 240, or M <= 1024 with N * K <= 2^22; K and N multiples of 64), which
- * reads the int8 codes without a weight copy. Up to a few thousand tokens that path also runs over
- * chunks of the tokens where it is faster than the GEMM. One call multiplies one weight: the tokens
- * past the GEMM's whole rounds of 256 x 256 output tiles run on other kernels, with the same W and h
- * (their sums are taken in another f32 order, so equal rows of x may differ in the last bit of y by
- * their position, here as between the tiles of the few-token path). With few 256 x 256 output tiles (a few hundred
- * tokens) the GEMM splits its reduction over several workgroups and sums their f32 partials in a
- * fixed order before the one rounding (the workspace holds them); the forward then multiplies the
- * int8 codes with s on the f32 sum, no weight copy. bias may be NULL. r = 0 (A, B NULL) gives the base-only
- * linear(::DenseLayer) of src/layers/linear.jl:38-46. h_save ([M][r] or NULL) receives h for the
+ * zero-padded copies in the workspace), and the few-token path (M <= 240, or M <= 1024 with
+ * N * K <= 2^22; K and N multiples of 64), which reads the int8 codes without a weight copy and, up
+ * to a few thousand tokens, also runs over chunks of the tokens where it is faster than the GEMM.
+ * With few 256 x 256 output tiles (a few hundred tokens) the GEMM splits its reduction over several
+ * workgroups and sums their f32 partials in a fixed order before the one rounding (the workspace
+ * holds them); the forward then multiplies the int8 codes with s on the f32 sum, no weight copy.
+ * One call multiplies one weight: the tokens past the GEMM's whole rounds of output tiles run on
+ * other kernels with the same W and h. Their sums are taken in another f32 order, so equal rows of x
+ * may differ in the last bit of y by their position, there as between the tiles of the few-token
+ * path. bias may be NULL. r = 0 (A, B NULL) gives the base-only linear(::DenseLayer) of
+ * src/layers/linear.jl:38-46. h_save ([M][r] or NULL) receives h for the
  * backward. workspace: device memory of reels_hip_i8lora_workspace_bytes(M, K, N, r,
  * REELS_HIP_WS_FWD).
  */

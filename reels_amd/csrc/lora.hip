@@ -1067,7 +1067,7 @@ static int64_t pad_width(int64_t M, int64_t d) {
 // valid parts are copied out. The products are those of the direct kernels at these widths: the
 // forward multiplies the int8 codes (s on the f32 sum), dX in bf16 rnd(dy s) and the codes (the copy
 // of dy for it scaled and rounded, scales of one for the inner call), in f16 the dequantized weight.
-// The copies cost a read and a write of each operand, in four launches of 5-9 us in 65 us forward and
+// The copies cost a read and a write of each operand, in four launches of 5-12 us in 67 us forward and
 // backward for 777 tokens, 1000 -> 3000 (rank 8; the scaled copy of dy 1.5 us of it, 12 us of 342 for the
 // backward of 8192 tokens, 2064 -> 5136); the one-output-per-thread kernels took 11.0 ms there, and widths
 // that are multiples of 16 ran unsplit 256 x 256 tiles (1000 tokens, 528 -> 2064: 236 against 89 us).

@@ -1,10 +1,8 @@
 """The few-token path's single launch (reels_amd/csrc/skinny.hip): output tiles wait for the
 adapter's rank projection l, published by the adapter blocks of the same launch, and a tile that
-stops waiting computes l itself with the adapter blocks' code and order. With split tiles the
-counters live in the call's own workspace, cleared by a one-block kernel just before the launch;
-row-wave launches (a few hundred tokens on a large weight) hand l and the adapter tiles' split
-partials over under a key of the launch (its dispatch in its queue and the host call's nonce)
-and clear nothing.
+stops waiting computes l itself with the adapter blocks' code and order. Blocks hand l and the split
+partials over under a key of the launch (its dispatch in its queue and the host call's nonce), in
+the call's own workspace, and clear nothing.
 
 These tests force the fallback from the host (REELS_HIP_SKINNY_SPIN=0: no wait at all, so
 split-0 adapter blocks also compute the other splits' partials) and require the same bits as
