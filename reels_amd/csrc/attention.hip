@@ -1,7 +1,7 @@
 // Exact scaled dot-product attention with an online softmax: memory_efficient_attention and its
 // backward (src/layers/attention.jl:106-221 CPU, 225-371 CUDA), for bf16 / f16 tensors with f32
 // arithmetic, head_dim 64 or 128 (f32 tensors and the other head dims up to 128 go to the
-// generic kernels of attention_g.hip).
+// generic kernels of attention_g_impl.h).
 //
 // Layouts (row-major; the reference's (head_dim, heads, tokens, batch) arrays): q, out, dq
 // [B][Sq][H][D]; k, v, dk, dv [B][Sk][H][D]; lse [B][H][Sq] f32; mask [Sq][Sk] uint8 (nonzero =
@@ -965,7 +965,7 @@ __global__ __launch_bounds__(256) void attn_zero_kernel(uint16_t* p, int64_t n) 
 // ---------------------------------------------------------------------------------------------
 // host side
 // bf16 / f16 with head dim 64 or 128 take the tuned kernels above; f32 and the other head dims
-// up to 128 the generic kernels of attention_g.hip
+// up to 128 the generic kernels of attention_g_impl.h
 static bool attn_tuned(int dtype, int64_t D) {
   return (dtype == REELS_HIP_BF16 || dtype == REELS_HIP_F16) && (D == 64 || D == 128);
 }

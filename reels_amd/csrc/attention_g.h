@@ -1,4 +1,4 @@
-// Attention for element types and head dims outside the tuned kernels (attention_g.hip):
+// Attention for element types and head dims outside the tuned kernels (attention_g_impl.h):
 // arguments and launchers, called by the entry points of attention.hip.
 #pragma once
 #include "common.h"
@@ -48,5 +48,8 @@ inline int64_t dq_scratch_bytes(const Args& a, int64_t B, int64_t D, int esz) {
 // REELS_HIP_F32, _BF16 or _F16 and 1 <= D <= 128; the caller has checked the arguments
 int attn_generic_fwd(const AttgArgs& a, int dtype, int64_t B, hipStream_t st);
 int attn_generic_bwd(const AttgArgs& a, int dtype, int64_t B, hipStream_t st);
+// the same of one element type, instantiated in attention_g_<type>.hip
+template <int ELT> int attng_fwd(const AttgArgs& a, int64_t B, hipStream_t st);
+template <int ELT> int attng_bwd(const AttgArgs& a, int64_t B, hipStream_t st);
 
 }  // namespace reels

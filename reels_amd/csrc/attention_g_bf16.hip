@@ -1,0 +1,7 @@
+// The generic attention kernels for bf16 tensors (attention_g_impl.h).
+#include "attention_g_impl.h"
+
+namespace reels {
+template int attng_fwd<REELS_HIP_BF16>(const AttgArgs&, int64_t, hipStream_t);
+template int attng_bwd<REELS_HIP_BF16>(const AttgArgs&, int64_t, hipStream_t);
+}  // namespace reels
