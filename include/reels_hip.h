@@ -316,7 +316,8 @@ int reels_hip_gelu_tanh_bwd_f32(const float* x, const float* dy, float* dx, int6
  * and sums run in f32 with scale 1/sqrt(Float32(D)) (attention.jl:129). bf16 / f16 with D = 64
  * or 128 take the tuned kernels, which round P to dtype for the P V product; f32 and other head
  * dims take kernels that keep every bit of P (the reference's order), their f32 operands as sums of
- * three bf16 values on the matrix cores, at a lower rate.
+ * three bf16 values on the matrix cores, at a lower rate (at D = 1 and 2 scores have to stay below
+ * 2.3e38).
  * A query with no visible key gets NaN output and NaN lse (-Inf when Sk = 0), as the reference;
  * it contributes nothing to dq, dk, dv (in the reference its NaN correction reaches every dk of
  * the head). The reference's query_block / key_block do not change the result and have no

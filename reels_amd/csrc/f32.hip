@@ -5,7 +5,7 @@
 //
 // The weight product runs on bf16 MFMA without giving up a bit of its operands: an int8 code is
 // exact in bf16, and an f32 activation is the exact sum of three bf16 values (8 significant bits
-// each). With s = mant 2^e (mant in [0.5, 1)), the weight operand is q 2^e (exact in bf16) and
+// each). With s = mant 2^e, the weight operand is q 2^e (exact in bf16) and
 // mant multiplies the f32 sum (forward, one output column) or the activation before it is taken
 // apart (dX, fl32(dy mant): one rounding, where fl32(q s) rounded the weight before). See the
 // bf16-plane form of bfgemm_kernel (i8gemm.hip) for the order of the sums and their error. The
@@ -23,11 +23,15 @@
 namespace reels {
 
 // ---------------------------------------------------------------------------------------------
-// s = mant 2^e, mant in [0.5, 1) (0 for s = 0). e stays in [-126, 120], where q 2^e is exact in
-// bf16 for every code; outside it mant takes the rest (s below 2^-126: mant below 0.5).
+// s = mant 2^e, mant in [0.5, 1) where it multiplies the activation (dX), in [1, 2) where it multiplies
+// the sum (forward), so that neither passes the end of the range before the product with s does (0 for
+// s = 0). e stays in [-126, 120], where q 2^e is exact in bf16 for every code; outside it mant takes the
+// rest (s below 2^-126: mant below that).
+template <bool FORWARD>
 __device__ __forceinline__ float scale_mant(float s, int& e) {
   int x = 0;
   (void)frexpf(s, &x);
+  if (FORWARD) --x;
   e = x < -126 ? -126 : (x > 120 ? 120 : x);
   if (!(fabsf(s) < INFINITY)) e = 0;
   return ldexpf(s, -e);
@@ -118,7 +122,7 @@ __global__ __launch_bounds__(256) void f32_operands_kernel(OperandArgs a) {
       if (i >= total) break;
       const int64_t n = i / groups, c = i - n * groups;
       int e;
-      const float m = scale_mant(a.s[n], e), p2 = pow2f(e);
+      const float m = scale_mant<true>(a.s[n], e), p2 = pow2f(e);
       if (c == 0) a.mant[n] = m;
       u32x4 o[2];
 #pragma unroll
@@ -141,7 +145,7 @@ __global__ __launch_bounds__(256) void f32_operands_kernel(OperandArgs a) {
     float p2 = 0.0f;
     if (n0 + nl < a.N) {
       int e;
-      const float m = scale_mant(a.s[n0 + nl], e);
+      const float m = scale_mant<false>(a.s[n0 + nl], e);
       p2 = pow2f(e);
       if (kb == 0 && kl == 0) a.mant[n0 + nl] = m;
     }

@@ -377,3 +377,26 @@ def test_f32_generic_kernels(dev):
         for name, a, b in (("y", y, yo), ("h", h, ho), ("dx", dx, ref["dx"]), ("dA", dA, ref["dA"]),
                            ("dB", dB, ref["dB"]), ("dbias", db, oracle.bias_gradient(cs["dy"], elt="f32"))):
             assert_parity(a.cpu().numpy(), b, f"generic {name}", tol=TOL)
+
+
+def test_f32_results_near_the_end_of_the_range(dev):
+    """y and dx of up to 3.2e38 from single terms, scales on both sides of a power of two: the scale's
+    parts overflow on neither side of the products."""
+    import torch
+    from reels_amd import QuantizedMatrix, i8lora_backward, i8lora_forward
+    print("[f32] near the end of the range", flush=True)
+    K, N = 70, 9
+    q = np.full((N, K), 127, np.int8)
+    s = (np.float32(2.0 ** -7) * np.float32([1.0, 1.01, 1.3, 1.6, 1.99, 0.51, 0.75, 0.99, 1.0001])).astype(np.float32)
+    W = QuantizedMatrix(todev(q, dev), todev(s, dev), torch.float32)
+    x = np.zeros((N, K), np.float32)  # row n for scale n
+    x[:, 5] = np.minimum(3.2e38 / (s.astype(np.float64) * 127), 3.3e38)
+    dy = np.zeros((N, N), np.float32)
+    dy[np.arange(N), np.arange(N)] = x[:, 5]
+    y = i8lora_forward(todev(x, dev), W)[0].cpu().numpy()
+    dx = i8lora_backward(todev(dy, dev), None, W, want_dA=False, want_dB=False)[0].cpu().numpy()
+    want = x[:, 5].astype(np.float64) * 127 * s
+    assert want.max() > 3e38
+    d = np.arange(N)
+    assert (np.abs(y[d, d] - want) <= 4 * 2.0 ** -24 * want).all()
+    assert (np.abs(dx - want[:, None]) <= 4 * 2.0 ** -24 * want[:, None]).all()
